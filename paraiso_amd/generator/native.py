@@ -48,6 +48,11 @@ class Setup:
     # a later phase evaluates in registers from mostly the same expansion, and let a launch
     # take the whole CU's LDS (for launches whose registers allow one workgroup per CU)
     join: bool = False
+    # evaluate what both sides of a Select compute alike once, after it (ir.merge_selects).
+    # Off where a rounding must not move: the multiply-adds a fast FP32 build contracts depend
+    # on the expressions around them, and a gradient through limiter switches amplifies the
+    # last bit of the forward run
+    merge_selects: bool = True
     # per OM kernel, a launch form overriding the above: ((kernel name, {"tile": ...,
     # "threads": ..., "persist": ..., "march": ..., "mat_gain": ..., "join": ...}), ...)
     kernel_forms: Tuple[Tuple[str, dict], ...] = ()

@@ -128,7 +128,8 @@ VARIANTS = {
                                                      tile=(32, 8)), True),
     # FP32 bulk arithmetic with the hardware reciprocal and square root in the adjoint too
     "hydro_adj_f32_fast": (_hydro_adj(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2,
-                                                          tile=(32, 8)), False),
+                                                          tile=(32, 8), merge_selects=False),
+                           False),
     # the fixed-dt step in FP32 (fast arithmetic) at the headline's launch form
     "hydro_fixed_f32": (_hydro(CType.Float, dt_mode="fixed"),
                         Setup((64, 64), Language.HIP, boundary=CYC2, tile=(64, 32), threads=1024,
@@ -141,7 +142,8 @@ VARIANTS = {
                                                       tile=(32, 8)), True),
     # the adjoint per stage (see _hydro_adj_staged), FP32 fast and FP64 correctly rounded
     "hydro_adj2_f32_fast": (_hydro_adj_staged(CType.Float),
-                            Setup((64, 64), Language.HIP, boundary=CYC2, tile=(32, 8)), False),
+                            Setup((64, 64), Language.HIP, boundary=CYC2, tile=(32, 8),
+                                  merge_selects=False), False),
     "hydro_adj2_f64": (_hydro_adj_staged(CType.Double),
                        Setup((64, 64), Language.HIP, boundary=CYC2, tile=(32, 8)), True),
     # the same with the adjoint kernels' shared expansions joined into earlier phases
