@@ -19,7 +19,7 @@
 // Workgroups a persistent launch starts: as many as the device holds at once (per_cu per
 // CU, from the launch's LDS and work-items), a multiple of 8 so that workgroup b, which the
 // dispatcher places on XCD b % 8, keeps to that XCD's band of tiles; at most ntiles.
-static inline unsigned om_resident_workgroups(unsigned ntiles, int per_cu) {
+static inline int om_cus() {
   static int cus = 0;
   if (cus <= 0) {
     int d = 0;
@@ -28,7 +28,11 @@ static inline unsigned om_resident_workgroups(unsigned ntiles, int per_cu) {
         cus <= 0)
       cus = 256;
   }
-  unsigned n = ((unsigned)cus * (unsigned)(per_cu > 0 ? per_cu : 1)) & ~7u;
+  return cus;
+}
+
+static inline unsigned om_resident_workgroups(unsigned ntiles, int per_cu) {
+  unsigned n = ((unsigned)om_cus() * (unsigned)(per_cu > 0 ? per_cu : 1)) & ~7u;
   if (n == 0) n = 8;
   return n < ntiles ? n : ntiles;
 }
@@ -89,6 +93,74 @@ __device__ __forceinline__ T om_block_reduce(T v, Op op, T* scratch /* >= NT / 6
 #pragma unroll
   for (int w = 1; w < NT / 64; ++w) r = op(r, scratch[w]);
   return r;   // every thread gets the block result
+}
+
+// ---- register streaming (a wave64 owns a strip of the grid, a lane a column of cells)
+
+// The value of the lane D places to the right (left for D < 0): wave-wide DPP moves, one
+// VALU instruction per place and 32 bits.  Lanes moved in from outside the wave hold 0 and
+// lie in the overlap of neighbouring strips, where nothing is stored.
+template <int D> __device__ __forceinline__ int om_lane32(int v) {
+  if constexpr (D > 0)
+    return om_lane32<D - 1>(__builtin_amdgcn_update_dpp(0, v, 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
+  else if constexpr (D < 0)
+    return om_lane32<D + 1>(__builtin_amdgcn_update_dpp(0, v, 0x138 /* wave_shr:1 */, 0xf, 0xf, true));
+  else
+    return v;
+}
+template <int D> __device__ __forceinline__ int om_lane(int v) { return om_lane32<D>(v); }
+template <int D> __device__ __forceinline__ bool om_lane(bool v) { return om_lane32<D>((int)v) != 0; }
+template <int D> __device__ __forceinline__ float om_lane(float v) {
+  return __builtin_bit_cast(float, om_lane32<D>(__builtin_bit_cast(int, v)));
+}
+template <int D> __device__ __forceinline__ double om_lane(double v) {
+  struct P { int lo, hi; };
+  const P p = __builtin_bit_cast(P, v);
+  return __builtin_bit_cast(double, P{om_lane32<D>(p.lo), om_lane32<D>(p.hi)});
+}
+
+// Element x of the row at a scalar address: the address stays in scalar registers and the
+// lane adds a 32-bit byte offset (a row has fewer than 2^31 cells of at most 8 bytes; rows
+// of 2^29 cells or more, whose byte offset does not fit, do not take this form).
+template <class T> __device__ __forceinline__ T om_at(const T* row, int x) {
+  return *(const T*)((const char*)row + (unsigned)x * (unsigned)sizeof(T));
+}
+template <class T> __device__ __forceinline__ void om_put(T* row, int x, T v) {
+  *(T*)((char*)row + (unsigned)x * (unsigned)sizeof(T)) = v;
+}
+
+template <class T, class Op> __device__ __forceinline__ T om_wave_reduce(T v, Op op) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = op(v, __shfl_xor(v, off, 64));
+  return v;
+}
+
+// Steps along the streaming axis (n long) that one wave takes, for `groups` waves side by
+// side: the axis is cut into as many chunks as make the shortest launch, where a chunk costs
+// its own steps and a run-up worth `runup` steps, and a SIMD takes as long for a step of its
+// waves as for `fill` of them where it holds fewer (issue slots or memory latency that too few
+// waves leave unused: 1.2 for the Hydro step, where one wave takes 1.36 us a row and two 2.27;
+// 4 where memory bounds).  At most `cap` waves, at least `least` steps.
+static inline int om_lane_chunk(int n, unsigned groups, double runup, double fill, unsigned cap,
+                                int least, unsigned simds) {
+  int best = n;
+  double cost = 1e300;
+  if (groups == 0) groups = 1;
+  for (unsigned k = 1; k <= 8; ++k) {
+    unsigned chunks = k * simds / groups;
+    if (chunks > cap / groups) chunks = cap / groups;
+    if (chunks < 1) chunks = 1;
+    int h = (int)((n + chunks - 1) / chunks);
+    if (h < least) h = least < n ? least : n;
+    const unsigned waves = groups * (unsigned)((n + h - 1) / h);
+    const unsigned per = (waves + simds - 1) / simds;
+    const double c = ((double)h + runup) * (per > fill ? per : fill);
+    if (c < 0.999 * cost) {
+      cost = c;
+      best = h;
+    }
+  }
+  return best;
 }
 
 // Reduce `count` partials in a fixed order.  Thread t keeps eight accumulators: lane

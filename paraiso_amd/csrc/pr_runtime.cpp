@@ -887,7 +887,8 @@ int pr_batch_create(const pr_machine_desc* d, int n_grids, const int* sizes, pr_
   }
   for (int g = 0; g < n_grids; ++g) {
     pr_machine* m = nullptr;
-    int rc = pr_create(d, sizes + 3 * g, &m);
+    // batched launches address a row with 32-bit byte offsets
+    int rc = sizes[3 * g] < (1 << 29) ? pr_create(d, sizes + 3 * g, &m) : PR_E_INVALID;
     if (rc == PR_OK) rc = pr_set_stream(m, b->stream);
     if (rc) {
       b->err = "grid " + std::to_string(g) + ": " + (m ? m->err : std::string("pr_create"));

@@ -173,8 +173,10 @@ def build_machine(setup: Setup, om: OM, variant: str, precise: bool = False,
     if precise:
         flags += ["-ffp-contract=off"]
     else:
-        # FP32 division and square root use v_rcp_f32 / v_sqrt_f32 in the generated source
-        flags += ["-ffp-contract=fast"]
+        # FP32 division and square root use v_rcp_f32 / v_sqrt_f32 in the generated source;
+        # register streaming writes its multiply-adds out and turns contraction off
+        flags += ["-ffp-contract=%s" % ("fast-honor-pragmas" if "fp contract(off)" in src
+                                        else "fast")]
     d = os.path.join(GEN_DIR, variant)
     os.makedirs(d, exist_ok=True)
     hip_path = os.path.join(d, variant + ".hip")

@@ -36,6 +36,7 @@ from ...om.arith import Op, ReduceOp
 from ...om.dyn import CType, Realm, fraction_to_float32
 from ...om.literal import c_literal
 from .ir import LKernel
+from .lane import LaneEmitter, fused_products, plan_lane
 from .schedule import OUT, ArrayLaunch, KernelSchedule, ring_depth
 
 NT = 256
@@ -233,7 +234,9 @@ class MachineEmitter:
         self.schedules = schedules
         self.tile = tuple(tile) + (1,) * (3 - len(tile))
         self._base = {"tile": self.tile, "threads": self.nt, "persist": self.persist,
-                      "march": self.march}
+                      "march": self.march, "lane": None}
+        self.lane = None
+        self._lane_memo: Dict[Tuple[int, int], list] = {}
         self.forms = forms or [None] * len(schedules)
         self.ns = len(statics)
         self.n_user = len(statics)
@@ -263,6 +266,7 @@ class MachineEmitter:
         self.nt = int(f["threads"])
         self.march = int(f["march"])
         self.persist = bool(f["persist"]) and not self.march
+        self.lane = f["lane"]
 
     def fn_name(self, ki: int, launch: int) -> str:
         """Kernel symbol: machine, OM kernel and launch, so that profiles name them."""
@@ -305,6 +309,9 @@ class MachineEmitter:
         self._launch_reach = 0
         has_work = bool(la.targets)
         L = la.index
+        lanes = self._lane_plans(ki, k, la) if has_work else []
+        lane = lanes[0][1] if lanes else None
+        block = lane is None or not self.lane.get("always")     # the tile form exists too
         # ---- argument struct
         loads = sorted(set(self.sidx(ki, nodes[v].payload) for v in la.lc if nodes[v].op == "load"
                            and nodes[v].realm is Realm.Array))
@@ -320,6 +327,10 @@ class MachineEmitter:
                    "int wide;  /* some axis shorter than tile plus reach: om_wrap takes the "
                    "remainder */",
                    "unsigned nwg;   /* reduction partials written (workgroups that reduce) */"]
+        if lane:
+            fields += ["unsigned ln, lx, ly, mx, my;  /* register streaming: waves, strips along "
+                       "x and y, reciprocals */", "int lc;  /* steps a wave streams */",
+                       "int lv;  /* which of the launch's streaming forms */"]
         struct = "struct Args_%s {\n  %s\n};\n" % (fn, "\n  ".join(fields))
 
         decls: List[str] = []
@@ -344,6 +355,7 @@ class MachineEmitter:
             elif lvl <= L:
                 w("  const %s u%d = *(const %s*)(a.scal + %d);" % (
                     n.ctype.c_name, n.id, n.ctype.c_name, self.slot_off(ki, n.id)))
+        uniforms = list(body)
         # LDS views
         for v, b in sorted(la.lds.items()):
             w("  %s* __restrict__ s%d = (%s*)(smem + %d);" % (
@@ -411,20 +423,24 @@ class MachineEmitter:
         fin_decls = ["  __shared__ %s om_scr_%s[%d];" % (at.c_name, at.c_name, self.nt // 64)
                      for at in sorted(acc_types, key=lambda c: c.value)]
         ks = [struct]
+        if lane:
+            for form, plan, name in lanes:
+                ks.extend(self._lane_kernel(ki, k, la, form, plan, fn, name, uniforms))
         core = "\n".join(coords + pre + work + epilogue("tile"))
-        ks.append("extern \"C\" __global__ void __launch_bounds__(%d) %s(Args_%s a) {" % (self.nt, fn, fn))
-        ks.extend(decls)
-        if persist:
-            ks.extend(pre)
-            ks.extend(loop)
-            ks.extend(epilogue("blockIdx.x"))
-        else:
-            ks.append("  unsigned tile = blockIdx.x;")
-            ks.append("  if ((a.ntiles & 7u) == 0u) tile = (tile & 7u) * (a.ntiles >> 3) + (tile >> 3);")
-            ks.append(core)
-        ks.append("}")
+        if block:
+            ks.append("extern \"C\" __global__ void __launch_bounds__(%d) %s(Args_%s a) {" % (self.nt, fn, fn))
+            ks.extend(decls)
+            if persist:
+                ks.extend(pre)
+                ks.extend(loop)
+                ks.extend(epilogue("blockIdx.x"))
+            else:
+                ks.append("  unsigned tile = blockIdx.x;")
+                ks.append("  if ((a.ntiles & 7u) == 0u) tile = (tile & 7u) * (a.ntiles >> 3) + (tile >> 3);")
+                ks.append(core)
+            ks.append("}")
         # batched form: the tiles of many grids in one launch (grid table in device memory)
-        if self.batched:
+        if self.batched and block:
             ks.append("extern \"C\" __global__ void __launch_bounds__(%d) %s_batched(const Args_%s* __restrict__ grids, "
                       "const int* __restrict__ tile_grid, const unsigned* __restrict__ tile_base, unsigned total) {"
                       % (self.nt, fn, fn))
@@ -461,25 +477,44 @@ class MachineEmitter:
             h.append("  a.st%d = (%s*)c->%s[%d];" % (s, self.statics[s].dyn.ctype.c_name, src, s))
         h.append("  a.scal = c->scal; a.part = c->part; a.counter = c->counter;")
         h.append("  a.n0 = c->n[0]; a.n1 = c->n[1]; a.n2 = c->n[2];")
-        h.append("  a.t0 = c->tiles[0]; a.t1 = c->tiles[1]; a.t2 = c->tiles[2]; a.ntiles = c->ntiles;")
-        h.append("  a.m0 = om_udiv_magic((unsigned)c->tiles[0]); a.m1 = om_udiv_magic((unsigned)c->tiles[1]);")
+        if self._own_tiles(lane):
+            for ax in range(3):
+                h.append("  a.t%d = (c->n[%d] + %d) / %d;" % (ax, ax, self.tile[ax] - 1, self.tile[ax]))
+            h.append("  a.ntiles = (unsigned)a.t0 * (unsigned)a.t1 * (unsigned)a.t2;")
+        else:
+            h.append("  a.t0 = c->tiles[0]; a.t1 = c->tiles[1]; a.t2 = c->tiles[2]; a.ntiles = c->ntiles;")
+        h.append("  a.m0 = om_udiv_magic((unsigned)a.t0); a.m1 = om_udiv_magic((unsigned)a.t1);")
         reach = self._max_reach(sch, la)
         h.append("  a.wide = (%s) ? 1 : 0;" % " || ".join(
             "c->n[%d] < %d" % (ax, self.tile[ax] + reach) for ax in range(self.ndim)))
         if persist:
-            h.append("  a.nwg = om_resident_workgroups(c->ntiles, %d);" % self._per_cu(la))
+            h.append("  a.nwg = om_resident_workgroups(a.ntiles, %d);" % self._per_cu(la))
         else:
-            h.append("  a.nwg = c->ntiles;")
+            h.append("  a.nwg = a.ntiles;")
+        if lane:
+            h.extend(self._lane_fill(la, lanes))
         h.append("}")
         h.append("static void pack_%s(const pr_launch_ctx* c, void* out) {" % fn)
-        h.append("  Args_%s a; fill_%s(c, a); a.nwg = c->ntiles; memcpy(out, &a, sizeof a);" % (fn, fn))
+        # (a batch's waves follow the runtime's table of tiles: a fixed number of steps each)
+        fixed = "" if block else " a.lc = %d; a.ln = c->ntiles;" % self.lane["steps"]
+        h.append("  Args_%s a; fill_%s(c, a); a.nwg = c->ntiles;%s memcpy(out, &a, sizeof a);"
+                 % (fn, fn, fixed))
         h.append("}")
         h.append("static int launch_batched_%s(const pr_batch_ctx* bc) {" % fn)
         if not self.batched:
             h.append("  (void)bc; return -1;")
         elif has_work:
-            h.append("  hipLaunchKernelGGL(%s_batched, dim3(bc->total_tiles), dim3(%d), 0, (hipStream_t)bc->stream, "
-                     "(const Args_%s*)bc->args, bc->tile_grid, bc->tile_base, bc->total_tiles);" % (fn, self.nt, fn))
+            wg = self.lane["waves"] if lane else 1
+            if block:
+                h.append("  hipLaunchKernelGGL(%s_batched, dim3(bc->total_tiles), dim3(%d), 0, (hipStream_t)bc->stream, "
+                         "(const Args_%s*)bc->args, bc->tile_grid, bc->tile_base, bc->total_tiles);" % (fn, self.nt, fn))
+            else:
+                # below two waves per SIMD a tile is split over a workgroup
+                h.append("  const int split = bc->total_tiles < 8u * (unsigned)om_cus();")
+                h.append("  hipLaunchKernelGGL(%s_batched, dim3(split ? bc->total_tiles : "
+                         "(bc->total_tiles + %du) / %du), dim3(%d), 0, (hipStream_t)bc->stream, "
+                         "(const Args_%s*)bc->args, bc->tile_grid, bc->tile_base, bc->total_tiles, split);"
+                         % (fn, wg - 1, wg, 64 * wg, fn))
         if needs_tail and self.batched:
             h.append("  hipLaunchKernelGGL(%s_fin_batched, dim3(bc->n_grids), dim3(%d), 0, (hipStream_t)bc->stream, "
                      "(const Args_%s*)bc->args);" % (fn, self.nt, fn))
@@ -488,15 +523,228 @@ class MachineEmitter:
         h.append("}")
         h.append("static int launch_%s(const pr_launch_ctx* c) {" % fn)
         h.append("  Args_%s a; fill_%s(c, a);" % (fn, fn))
-        if has_work:
+        if lane:
+            wg = self.lane["waves"]
+            h.append("  if (a.ln) {")
+            h.append("  a.nwg = (a.ln + %du) / %du;" % (wg - 1, wg))
+            for i, (_, _, name) in enumerate(lanes):
+                h.append("  %sif (a.lv == %d) hipLaunchKernelGGL(%s, dim3(a.nwg), dim3(%d), 0, "
+                         "(hipStream_t)c->stream, a);" % ("else " if i else "", i, name, 64 * wg))
+            h.append("  }" + (" else" if block else ""))
+        if has_work and block:
             h.append("  hipLaunchKernelGGL(%s, dim3(%s), dim3(%d), 0, (hipStream_t)c->stream, a);"
-                     % (fn, "a.nwg" if persist else "c->ntiles", self.nt))
+                     % (fn, "a.nwg" if persist else "a.ntiles", self.nt))
         if needs_tail:
             h.append("  hipLaunchKernelGGL(%s_fin, dim3(1), dim3(%d), 0, (hipStream_t)c->stream, a);"
                      % (fn, self.nt))
         h.append("  return hipPeekAtLastError() == hipSuccess ? 0 : -1;")
         h.append("}")
         return kernel_src, "\n".join(h) + "\n"
+
+    # ------------------------------------------------------------ register streaming
+    def _lane_plans(self, ki, k, la):
+        """[(form, plan, kernel name)] of the launch's register-streaming forms, the first for
+        large grids, a second (``small``) with other rows per lane for those ``below`` a number
+        of cells; empty where its form asks for none or it reads no array."""
+        if not self.lane or any(self.open_axes[:self.ndim]):
+            return []
+        key = (ki, la.index)
+        if key not in self._lane_memo:
+            out = []
+            for name in ("lane", "small"):
+                f = dict(self.lane)
+                if name == "small":
+                    if "small" not in f:
+                        break
+                    f.update(f["small"])
+                p = plan_lane(k, la.targets, f.get("rows", 1), f.get("prefetch", 1))
+                if p is not None:
+                    out.append((f, p, "%s_%s" % (self.fn_name(ki, la.index), name)))
+            self._lane_memo[key] = out
+        return self._lane_memo[key]
+
+    def lane_tile(self, form, plan) -> List[int]:
+        """Cells a wave takes at least: strip width, rows and steps."""
+        steps = form["steps"]
+        return ([plan.width, steps, 1] if self.ndim == 2 else [plan.width, plan.rows, steps])
+
+    def _lane_kernel(self, ki, k, la, f, plan, fn, name, uniforms) -> List[str]:
+        nodes = k.nodes
+        out: List[str] = []
+        pre = list(uniforms)
+        for v in plan.uniform:
+            n = nodes[v]
+            tn = n.ctype.c_name
+            if n.op == "imm":
+                e = c_literal(n.payload, n.ctype)
+            elif n.op == "size":
+                e = "(%s)%s" % (tn, self._local_size(n.payload))
+            elif n.op == "bcast":
+                e = "u%d" % n.args[0]
+            elif n.op == "shift":
+                e = "n%d" % n.args[0]
+            else:
+                op, cast_to = n.payload
+                e = device_arith(op, ["n%d" % x for x in n.args], cast_to,
+                                 [nodes[x].ctype for x in n.args], n.ctype, self.fast_fp32,
+                                 [k.exact.get(x) for x in n.args], self._comp)
+            pre.append("  const %s n%d = %s;" % (tn, v, e))
+        reduces = []
+        for r in la.reduces:
+            arg = nodes[r].args[0]
+            at = acc_type(nodes[r].payload, nodes[arg].ctype)
+            pre.append("  %s acc%d = %s;" % (at.c_name, r, acc_init(nodes[r].payload, at)))
+            reduces.append(("acc%d" % r, acc_op(nodes[r].payload, at), at.c_name,
+                            acc_init(nodes[r].payload, at), arg))
+        stores = [("a.st%d" % self.sidx(ki, s), nodes[v].ctype.c_name, v) for s, v in la.stores]
+
+        def consts(v):
+            return [k.exact.get(x) for x in nodes[v.node].args]
+
+        def split(v):
+            """(x, y) of a fusable product: multiplication or division by a value."""
+            if v.op != "arith" or v.ctype is not CType.Float or not self.fast_fp32:
+                return None
+            c = consts(v)
+            if v.payload[0] is Op.Mul:
+                return "mul" if c[0] is None and c[1] is None else None
+            return "div" if v.payload[0] is Op.Div and c[0] is None and c[1] is None else None
+
+        def arith(v, args):
+            op, cast_to = v.payload
+            pair = next((x for x in args if isinstance(x, tuple)), None)
+            if pair is not None:
+                i = args.index(pair)
+                x, y = pair[1]
+                if pair[0].payload[0] is Op.Div:
+                    y = "__builtin_amdgcn_rcpf(%s)" % y
+                other = args[1 - i]
+                if op is Op.Sub and i == 1:
+                    return "__builtin_fmaf(-%s, %s, %s)" % (x, y, other)
+                return "__builtin_fmaf(%s, %s, %s%s)" % (x, y, "-" if op is Op.Sub else "", other)
+            types = [nodes[x].ctype for x in nodes[v.node].args]
+            return device_arith(op, args, cast_to, types, v.ctype, self.fast_fp32, consts(v),
+                                self._comp)
+        em = LaneEmitter(plan, k, lambda s: "a.ld%d" % self.sidx(ki, s), arith, stores, reduces,
+                         fused_products(plan, lambda v: split(v) is not None))
+        last = self.ndim - 1
+        where = ["  const int lane = threadIdx.x & 63;"]
+        if self.ndim == 2:
+            where += ["  const unsigned chunk = om_udiv(tile, a.lx, a.mx);",
+                      "  const int X0 = (int)(tile - chunk * a.lx) * %d, S0 = (int)chunk * a.lc;"
+                      % plan.width]
+        else:
+            where += ["  const unsigned q_ = om_udiv(tile, a.lx, a.mx), chunk = om_udiv(q_, a.ly, a.my);",
+                      "  const int X0 = (int)(tile - q_ * a.lx) * %d, Y0 = (int)(q_ - chunk * a.ly) * %d, "
+                      "S0 = (int)chunk * a.lc;" % (plan.width, plan.rows)]
+        core = ["#pragma clang fp contract(off)"] if self.fast_fp32 else []
+        core += ["    const int H = a.n%d - S0 < steps ? a.n%d - S0 : steps;" % (last, last)]
+        core += em.body(f.get("unroll", 1))
+        wg = f["waves"]
+
+        def epilogue(index, wave):
+            """Partials: one per workgroup, or (batches: a workgroup's waves may belong to
+            different grids) one per wave."""
+            e = []
+            for j, r in enumerate(la.reduces):
+                at = acc_type(nodes[r].payload, nodes[nodes[r].args[0]].ctype)
+                op = acc_op(nodes[r].payload, at)
+                red = ("om_wave_reduce(acc%d, %s)" % (r, op) if wave else
+                       "om_block_reduce<%d>(acc%d, %s, om_scr_%s)" % (64 * wg, r, op, at.c_name))
+                e.append("  { const %s wr = %s;" % (at.c_name, red))
+                e.append("    if (%s == 0) ((%s*)a.part)[%d * a.ntiles + %s] = wr; }" % (
+                    "(threadIdx.x & 63)" if wave else "threadIdx.x", at.c_name, j, index))
+            return e
+        scr = ["  __shared__ %s om_scr_%s[%d];" % (c.c_name, c.c_name, wg) for c in sorted(
+            set(acc_type(nodes[r].payload, nodes[nodes[r].args[0]].ctype) for r in la.reduces),
+            key=lambda c: c.value)]
+        bounds = "__launch_bounds__(%d, %d)" % (64 * f["waves"], f["occupancy"])
+        wave = ["  unsigned b_ = blockIdx.x;",
+                "  if ((gridDim.x & 7u) == 0u) b_ = (b_ & 7u) * (gridDim.x >> 3) + (b_ >> 3);",
+                "  const unsigned wv = b_ * %du + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);"
+                % wg]
+        out.append("extern \"C\" __global__ void %s %s(Args_%s a) {" % (bounds, name, fn))
+        out += scr + wave + ["  const unsigned tile = wv;"] + where
+        out += ["  const int steps = a.lc;"] + pre
+        out += ["  if (wv < a.ln) {"] + core + ["  }"] + epilogue("b_", False) + ["}"]
+        if self.batched and f.get("always"):
+            # a tile of the batch is a wave's; `split`: a workgroup's, each wave taking its
+            # share of the steps, where the batch has too few tiles to fill the chip
+            out.append("extern \"C\" __global__ void %s %s_batched(const Args_%s* __restrict__ grids, "
+                       "const int* __restrict__ tile_grid, const unsigned* __restrict__ tile_base, "
+                       "unsigned total, int split) {" % (bounds, fn, fn))
+            out += scr + wave[:-1]
+            out += ["  const unsigned w_ = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);",
+                    "  const unsigned wv = split ? b_ : b_ * %du + w_;" % wg,
+                    "  if (wv >= total) return;", "  const int g = tile_grid[wv];",
+                    "  const Args_%s a = grids[g];" % fn,
+                    "  const unsigned tile = wv - tile_base[g];",
+                    "  const int steps = split ? a.lc / %d : a.lc;" % wg]
+            out += [ln.replace("S0 = (int)chunk * a.lc;",
+                               "S0 = (int)chunk * a.lc + (split ? (int)w_ * steps : 0);")
+                    for ln in where] + pre
+            out += ["  if (S0 < a.n%d) {" % last] + core + ["  }"]
+            if la.reduces:
+                out += (["  if (split) {"] + epilogue("tile", False) + ["  } else {"]
+                        + epilogue("tile", True) + ["  }"])
+            out += ["}"]
+        return out
+
+    def _own_tiles(self, lane) -> bool:
+        """The runtime's tiles are the waves' (lane_tile) and the tile form counts its own: a
+        single-grid launch with both forms, whose partials the waves outnumber otherwise."""
+        return lane is not None and not self.batched and not self.lane.get("always")
+
+    def _lane_fill(self, la, lanes) -> List[str]:
+        """Host side: the form for this grid, its strips and its steps per wave."""
+        last = self.ndim - 1
+        h = ["  const long long cells = (long long)a.n0 * a.n1 * a.n2; (void)cells;", "  a.lv = 0;"]
+        if len(lanes) > 1:
+            h.append("  if (cells < %dLL) a.lv = 1;" % lanes[1][0]["below"])
+        for i, (f, plan, _) in enumerate(lanes):
+            wg = f["waves"]
+            # (grids below the smallest skip the search for the steps per wave: their launches
+            # are short and the host issues them)
+            few = "cells < %dLL" % f["min_cells"] if f.get("min_cells") else ""
+            h.append("  if (%s) a.ln = 0;" % few if few else "")
+            h.append("  %sif (a.lv == %d) {" % ("else " if few else "", i))
+            h += ["  a.lx = (unsigned)((a.n0 + %d) / %d); a.ly = %s;" % (
+                     plan.width - 1, plan.width,
+                     "(unsigned)((a.n1 + %d) / %d)" % (plan.rows - 1, plan.rows)
+                     if self.ndim == 3 else "1u"),
+                  "  a.mx = om_udiv_magic(a.lx); a.my = om_udiv_magic(a.ly);"]
+            cap = "c->ntiles * %du" % wg if la.reduces else "0x7fffffffu"
+            h.append("  a.lc = om_lane_chunk(a.n%d, a.lx * a.ly, %.2f, %g, %s, %d, "
+                     "(unsigned)om_cus() * 4u);"
+                     % (last, plan.runup, f.get("fill", 1.2), cap, f["steps"]))
+            h.append("  a.ln = a.lx * a.ly * (unsigned)((a.n%d + a.lc - 1) / a.lc);" % last)
+            wide = ["a.n0 < %d" % (64 + 2 * plan.reach), "a.n%d < %d" % (last, 2 * plan.reach)]
+            if self.ndim == 3:
+                wide.append("a.n1 < %d" % (plan.rows + 2 * plan.reach))
+            wide = "(%s) ? 1 : 0" % " || ".join(wide)
+            if f.get("always"):
+                h += ["  a.wide = %s;" % wide, "  }"]
+                continue
+            # grids the form is not for take the tile form: a row's bytes must fit the 32-bit
+            # lane offsets, a workgroup's partials the space for them
+            not_for = ["a.n0 >= (1 << 29)"]
+            if la.reduces:
+                not_for.append("(a.ln + %du) / %du > c->ntiles" % (wg - 1, wg))
+            if self.march and f.get("ratio"):
+                # a streaming tile form keeps memory busier where its workgroups (one per CU)
+                # fill the chip: `ratio` is its time per cell next to this form's, measured full
+                vol = 1
+                for t in self.tile:
+                    vol *= t
+                h.append("  const unsigned rounds = (a.ntiles + (unsigned)om_cus() - 1u) / (unsigned)om_cus();")
+                not_for.append("(double)rounds * om_cus() * %d.0 * %g < (double)cells"
+                               % (vol, f["ratio"]))
+            h.append("  if (%s) a.ln = 0;" % " || ".join(not_for))
+            h.append("  if (a.ln) a.wide = %s;" % wide)
+            if self._own_tiles(plan):
+                h.append("  if (a.ln) a.ntiles = c->ntiles;   // the stride of the partials")
+            h.append("  }")
+        return h
 
     def _max_reach(self, sch, la) -> int:
         """A bound on how far outside its tile a launch's coordinates go on any axis: the
@@ -1130,6 +1378,12 @@ class MachineEmitter:
                 out.append(ksrc)
                 launchers.append(hsrc)
                 tile = list(self.tile) if la.targets else [0, 0, 0]
+                lanes = (self._lane_plans(ki, la.kernel_override or sch.kernel, la)
+                         if la.targets else [])
+                always = bool(lanes) and bool(self.lane.get("always"))
+                if lanes and (always or self._own_tiles(lanes[0][1])):
+                    waves = [self.lane_tile(f, p) for f, p, _ in lanes]
+                    tile = [min(x) for x in zip(*(waves if always else waves + [tile]))]
                 if self.batched:
                     fn = self.fn_name(ki, la.index)
                     ldesc.append("{launch_%s, {%d, %d, %d}, %d, pack_%s, sizeof(Args_%s), "

@@ -436,6 +436,7 @@ def merge_selects(k: LKernel) -> LKernel:
         nodes[out].hint_manifest |= n.hint_manifest
         new[s1] = out
     replace(new)
+    changed = bool(new)
     # ---- groups of selects with one condition
     done = set()
     while True:
@@ -501,6 +502,9 @@ def merge_selects(k: LKernel) -> LKernel:
                 nodes[m].hint_manifest |= nodes[s].hint_manifest
                 new[s] = m
         replace(new)
+        changed |= bool(new)
+    if not changed:
+        return k
     order = _topological(nodes, _reach(nodes, [v for _, v in stores]))
     at = {v: i for i, v in enumerate(order)}
     out = [LNode(at[v], nodes[v].op, tuple(at[a] for a in nodes[v].args), nodes[v].realm,

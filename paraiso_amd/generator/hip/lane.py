@@ -24,6 +24,7 @@ from __future__ import annotations
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Set, Tuple
 
+from ...om.arith import Op
 from ...om.dyn import CType, Realm
 from .ir import LKernel
 
@@ -62,6 +63,13 @@ class LanePlan:
     @property
     def width(self) -> int:
         return self.lanes[1] - self.lanes[0] + 1
+
+    @property
+    def runup(self) -> float:
+        """What the steps before the first store cost, in steps."""
+        size = lambda v: len(v.rows) if v.op == "arith" else 0
+        return (sum(size(v) * max(0, -v.first) for v in self.values)
+                / max(1, sum(size(v) for v in self.values)))
 
 
 def plan_lane(k: LKernel, targets: List[int], rows: int = 1, prefetch: int = 1
@@ -253,3 +261,185 @@ def plan_lane(k: LKernel, targets: List[int], rows: int = 1, prefetch: int = 1
 def registers(p: LanePlan) -> int:
     """32-bit registers the values kept from step to step take, per lane."""
     return sum(v.depth * len(v.rows) * max(1, v.ctype.size // 4) for v in p.values)
+
+
+def _n(x: int) -> str:
+    return "m%d" % -x if x < 0 else "%d" % x
+
+
+def fused_products(p: LanePlan, product) -> Dict[int, int]:
+    """The multiply-adds of a fast FP32 build: addition or subtraction -> the argument that is
+    a product it takes in.  Fixed here rather than left to the compiler, which would choose
+    anew in every copy of a step (the run-up, the unrolled loop): a cell's bits must not
+    depend on which copy computed it, that is on how the grid was cut into chunks.  A product
+    is taken in by all its readers or by none.  ``product(value)``: it may be fused."""
+    by_id = {v.id: v for v in p.values}
+    users: Dict[int, List[LaneValue]] = {v.id: [] for v in p.values}
+    for v in p.values:
+        for b, o in v.args:
+            if o is not None:
+                users[b].append(v)
+    targets = set(b for b, _ in p.targets.values())
+    out: Dict[int, int] = {}
+    for v in p.values:
+        if not product(v) or v.id in targets or v.depth or not users[v.id]:
+            continue
+        spots = []
+        for u in users[v.id]:
+            i = [j for j, (b, o) in enumerate(u.args) if b == v.id and o is not None]
+            if (u.op != "arith" or u.payload[0] not in (Op.Add, Op.Sub) or u.id in out
+                    or u.ctype is not CType.Float or len(i) != 1 or any(u.args[i[0]][1])
+                    or u.lead != v.lead or u.place != v.place):
+                break
+            spots.append((u.id, i[0]))
+        else:
+            out.update(spots)
+    return out
+
+
+class LaneEmitter:
+    """The device code of one launch in register-streaming form (see the module's docstring).
+
+    ``load_ptr(static)`` is a static's pointer; ``arith(value, args)`` the C expression of an
+    operation; ``stores`` and ``reduces`` list (C pointer, C type, target) and (accumulator,
+    operator, C type, initial value, target)."""
+
+    def __init__(self, plan: LanePlan, k: LKernel, load_ptr, arith, stores, reduces, fused=None):
+        """``fused``: as ``fused_products`` gives it; ``arith`` then gets, in the place of that
+        argument, the pair of names it multiplies."""
+        self.p, self.k = plan, k
+        self.fused = fused or {}
+        self.inside = set(self._arg(u, i) for u, i in self.fused.items())
+        self.by_id = {v.id: v for v in plan.values}
+        self.load_ptr, self.arith = load_ptr, arith
+        self.stores, self.reduces = stores, reduces
+        self.ma = plan.ndim - 1
+        self.lines: List[str] = []
+
+    def _arg(self, u: int, i: int) -> int:
+        return next(v for v in self.p.values if v.id == u).args[i][0]
+
+    # ------------------------------------------------------------ names
+    def name(self, v: LaneValue, row: int, delay: int) -> str:
+        r = "_r%s" % _n(row) if self.p.ndim == 3 else ""
+        return "v%d%s" % (v.id, r) if delay == 0 else "h%d%s_%d" % (v.id, r, delay)
+
+    def read(self, b: int, off, place: int, lead: int, row: int, moved: Dict, w) -> str:
+        """Value ``b`` at ``off`` from a reader placed at (place, lead), as a C name; lane moves
+        are emitted once per step."""
+        v = self.by_id[b]
+        delay = v.lead - lead - off[self.ma]
+        dx = place + off[0] - v.place
+        r = row + (off[1] if self.p.ndim == 3 else 0)
+        nm = self.name(v, r, delay)
+        if dx == 0:
+            return nm
+        key = (b, r, delay, dx)
+        if key not in moved:
+            moved[key] = "x%s_%s" % (nm, _n(dx))
+            w("const %s %s = om_lane<%d>(%s);" % (v.ctype.c_name, moved[key], dx, nm))
+        return moved[key]
+
+    # ------------------------------------------------------------ parts
+    def setup(self) -> List[str]:
+        """Per-wave coordinates: the lane's column, the rows' offsets and the kept registers."""
+        p, out = self.p, []
+        w = out.append
+        lo, hi = p.lanes
+        w("const int x = X0 + lane - %d;" % lo)
+        w("const bool ok = lane >= %d && lane <= %d && x < a.n0;" % (lo, hi))
+        for place in sorted(set(v.place for v in p.values if v.op == "load" or
+                                (v.op == "index" and v.payload == 0))):
+            w("const int x_%s = om_wrap(x + (%d), a.n0, a.wide);" % (_n(place), place))
+        if p.ndim == 3:
+            for r in sorted(set(r for v in p.values for r in v.rows)):
+                w("const int y_%s = om_wrap(Y0 + (%d), a.n1, a.wide);" % (_n(r), r))
+        for v in p.values:
+            for r in v.rows:
+                if v.depth:
+                    w("%s %s;" % (v.ctype.c_name, ", ".join(
+                        "%s = (%s)0" % (self.name(v, r, d), v.ctype.c_name)
+                        for d in range(1, v.depth + 1))))
+        return out
+
+    def step(self, s: str, at: Optional[int]) -> List[str]:
+        """One step; ``at`` is its number in the run-up before the first store, or None."""
+        p, out = self.p, []
+        w = out.append
+        on = lambda v: at is None or v.first <= at
+        last = "a.n%d" % self.ma
+        for lead in sorted(set(v.lead for v in p.values if on(v) and
+                               (v.op == "load" or (v.op == "index" and v.payload == self.ma)))):
+            w("const int m_%s = om_wrap(S0 + (%s) + (%d), %s, a.wide);" % (_n(lead), s, lead, last))
+        moved: Dict = {}
+        for v in p.values:
+            if not on(v) or v.id in self.inside:
+                continue
+            tn = v.ctype.c_name
+            for r in v.rows:
+                nm = self.name(v, r, 0)
+                if v.op == "load":
+                    row = ("(size_t)m_%s * a.n0" % _n(v.lead) if p.ndim == 2 else
+                           "((size_t)m_%s * a.n1 + y_%s) * a.n0" % (_n(v.lead), _n(r)))
+                    w("const %s %s = om_at(%s + %s, x_%s);" % (tn, nm, self.load_ptr(v.payload), row,
+                                                              _n(v.place)))
+                elif v.op == "index":
+                    src = ("x_%s" % _n(v.place) if v.payload == 0 else
+                           "m_%s" % _n(v.lead) if v.payload == self.ma else "y_%s" % _n(r))
+                    w("const %s %s = (%s)%s;" % (tn, nm, tn, src))
+                else:
+                    def names(u):
+                        return [b if o is None else self.read(b, o, u.place, u.lead, r, moved, w)
+                                for b, o in u.args]
+                    i = self.fused.get(v.id)
+                    args = [b if o is None else None if j == i else
+                            self.read(b, o, v.place, v.lead, r, moved, w)
+                            for j, (b, o) in enumerate(v.args)]
+                    if i is not None:
+                        args[i] = (self.by_id[v.args[i][0]], names(self.by_id[v.args[i][0]]))
+                    w("const %s %s = %s;" % (tn, nm, self.arith(v, args)))
+        if at is None:
+            rows = range(p.rows) if p.ndim == 3 else [0]
+            for r in rows:
+                pre = []
+                def target(t):
+                    if t in p.uniform_targets:
+                        return "n%d" % t
+                    b, o = p.targets[t]
+                    return self.read(b, o, 0, 0, r, moved, pre.append)
+                vals = [target(t) for _, _, t in self.stores]
+                reds = [target(t) for _, _, _, _, t in self.reduces]
+                out.extend(pre)
+                if p.ndim == 3:
+                    w("if (Y0 + %d < a.n1) {" % r)
+                if self.stores:
+                    w("if (ok) {")
+                    row = ("(size_t)(S0 + (%s)) * a.n0" % s if p.ndim == 2 else
+                           "((size_t)(S0 + (%s)) * a.n1 + (Y0 + %d)) * a.n0" % (s, r))
+                    for (ptr, tn, _), val in zip(self.stores, vals):
+                        w("  om_put(%s + %s, x, (%s)%s);" % (ptr, row, tn, val))
+                    w("}")
+                for (acc, op, tn, init, _), val in zip(self.reduces, reds):
+                    w("%s = %s(%s, ok ? (%s)%s : (%s)%s);" % (acc, op, acc, tn, val, tn, init))
+                if p.ndim == 3:
+                    w("}")
+        for v in p.values:
+            if on(v):
+                for r in v.rows:
+                    for d in range(v.depth, 0, -1):
+                        w("%s = %s;" % (self.name(v, r, d), self.name(v, r, d - 1)))
+        return out
+
+    def body(self, unroll: int) -> List[str]:
+        """The steps of a wave: the run-up, each step with only the values that something reads
+        later, then the loop."""
+        out = ["    " + ln for ln in self.setup()]
+        for s in range(self.p.first, 0):
+            out.append("    {  // run-up, step %d" % s)
+            out += ["      " + ln for ln in self.step("%d" % s, s)]
+            out.append("    }")
+        out.append("#pragma unroll %d" % max(1, unroll))
+        out.append("    for (int s = 0; s < H; ++s) {")
+        out += ["      " + ln for ln in self.step("s", None)]
+        out.append("    }")
+        return out

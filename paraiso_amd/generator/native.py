@@ -53,6 +53,13 @@ class Setup:
     # on the expressions around them, and a gradient through limiter switches amplifies the
     # last bit of the forward run
     merge_selects: bool = True
+    # register streaming (hip/lane.py): {"rows": y rows per lane (3-D), "waves": waves per
+    # workgroup, "occupancy": waves per SIMD the registers are held to, "fill": waves per SIMD
+    # below which a launch gains from more (om_lane_chunk), "steps": least steps per wave,
+    # "unroll", "prefetch": steps the loads are issued ahead, "min_cells": smallest grid that
+    # takes the form, "always": every grid does and no tile form is built, "ratio": see
+    # MachineEmitter._lane_fill, "small": what differs on grids of fewer than "below" cells}
+    lane: Optional[dict] = None
     # per OM kernel, a launch form overriding the above: ((kernel name, {"tile": ...,
     # "threads": ..., "persist": ..., "march": ..., "mat_gain": ..., "join": ...}), ...)
     kernel_forms: Tuple[Tuple[str, dict], ...] = ()
@@ -77,7 +84,8 @@ class Setup:
     def form_of(self, kernel: str) -> dict:
         """The launch form of one OM kernel: the machine's, with the kernel's overrides."""
         f = {"tile": self.tile, "threads": self.threads, "persist": self.persist,
-             "march": self.march, "mat_gain": self.mat_gain, "join": self.join}
+             "march": self.march, "mat_gain": self.mat_gain, "join": self.join,
+             "lane": self.lane}
         for name, over in self.kernel_forms:
             if name == kernel:
                 f.update(over)

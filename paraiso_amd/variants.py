@@ -109,11 +109,31 @@ def _optable(real):
     return mk
 
 
+# Register streaming (generator/hip/lane.py).  Hydro: a wave streams along y; below min_cells
+# the strips are too short for their run-up and the tile form is faster (FP32: 22.6 us a step
+# at 700^2 in tiles, 24.0 streaming; 33.4 and 28.3 at 1021x767; 112 and 91 at 2048^2.  FP64:
+# 31.9 and 33.7 at 512^2, 55.9 and 51.2 at 700^2, 344 and 250 at 2048^2).
+LANE_HYDRO_F32 = {"waves": 4, "occupancy": 2, "steps": 4, "min_cells": 600_000}
+LANE_HYDRO_F64 = {"waves": 4, "occupancy": 2, "steps": 4, "min_cells": 400_000}
+# Batches: a tile is 32 steps of one wave (24 and 40: within 1%), 0.92 -> 0.64 ms a step for
+# 256 uneven grids.
+LANE_HYDRO_BATCH = {"waves": 4, "occupancy": 2, "steps": 32, "always": True}
+# LinearWave 3-D: a lane holds rows of y, fewer on small grids (64^3: 11.6 us a step with 8, 8.9
+# with 4; 128^3 15.3 and 13.9; 300^3 128 and 128, two steps 123 and 141).  FP32 keeps its
+# streaming tiles where they fill the chip: at 512^3 they move 4.7 TB/s and the waves' unaligned
+# rows 3.6 (``ratio``), but a 201x150x97 box is 40 tiles (172 us a step) and 1,500 waves (18 us),
+# 192^3 148 and 27 us.  FP64: 51 us in tiles and 32 streaming at 160^3, 327 and 220 at 300^3,
+# three rows a lane at 100x150x80 15.6 us, four 17.1.
+LANE_WAVE_F32 = {"rows": 8, "waves": 4, "occupancy": 3, "steps": 4, "fill": 3, "ratio": 0.75,
+                 "small": {"rows": 4, "occupancy": 4, "fill": 4, "below": 2_500_000}}
+LANE_WAVE_F64 = {"rows": 4, "waves": 4, "occupancy": 2, "steps": 4, "fill": 3,
+                 "small": {"rows": 3, "occupancy": 3, "below": 2_000_000}}
+
 # name -> (OM factory, setup, precise)
 VARIANTS = {
     "life_i32": (_life, Setup((64, 64), Language.HIP, boundary=CYC2), True),
-    "hydro_f32": (_hydro(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2, batched=True),
-                  False),
+    "hydro_f32": (_hydro(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2, batched=True,
+                                             lane=LANE_HYDRO_F32), False),
     # the headline machine's launch form (tile, work-items, resident tile loop), correctly
     # rounded: checked bit for bit against the oracle
     "hydro_f32_precise": (_hydro(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2,
@@ -121,9 +141,12 @@ VARIANTS = {
                           True),
     # the same machine, tuned for batches of small uneven grids
     "hydro_f32_batch": (_hydro(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2,
-                                                   batched=True), False),
-    "hydro_f64": (_hydro(CType.Double), Setup((64, 64), Language.HIP, boundary=CYC2, batched=True),
-                  True),
+                                                   batched=True, lane=LANE_HYDRO_BATCH), False),
+    "hydro_f64": (_hydro(CType.Double), Setup((64, 64), Language.HIP, boundary=CYC2, batched=True,
+                                              lane=LANE_HYDRO_F64), True),
+    # register streaming at every size, correctly rounded: checked bit for bit
+    "hydro_f64_lane": (_hydro(CType.Double), Setup((64, 64), Language.HIP, boundary=CYC2,
+                                                   batched=True, lane=LANE_HYDRO_BATCH), True),
     "hydro_adj_f32": (_hydro_adj(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2,
                                                      tile=(32, 8)), True),
     # FP32 bulk arithmetic with the hardware reciprocal and square root in the adjoint too
@@ -133,11 +156,11 @@ VARIANTS = {
     # the fixed-dt step in FP32 (fast arithmetic) at the headline's launch form
     "hydro_fixed_f32": (_hydro(CType.Float, dt_mode="fixed"),
                         Setup((64, 64), Language.HIP, boundary=CYC2, tile=(64, 32), threads=1024,
-                              persist=True), False),
+                              persist=True, lane=LANE_HYDRO_F32), False),
     # the plain FP64 fixed-dt step at its fastest launch form (the comparison for the adjoint)
     "hydro_fixed_f64": (_hydro(CType.Double, dt_mode="fixed"),
                         Setup((64, 64), Language.HIP, boundary=CYC2, tile=(32, 32), threads=1024,
-                              persist=True), True),
+                              persist=True, lane=LANE_HYDRO_F64), True),
     "hydro_adj_f64": (_hydro_adj(CType.Double), Setup((64, 64), Language.HIP, boundary=CYC2,
                                                       tile=(32, 8)), True),
     # the adjoint per stage (see _hydro_adj_staged), FP32 fast and FP64 correctly rounded
@@ -154,8 +177,10 @@ VARIANTS = {
                                   kernel_forms=(("proceed_stage1_adjoint", {"join": True}),
                                                 ("proceed_stage2_adjoint", {"join": True}))),
                             True),
-    "wave3d_f32": (_wave_adj(3, CType.Float), Setup((64, 64, 64), Language.HIP, boundary=CYC3), False),
-    "wave3d_f64": (_wave_adj(3, CType.Double), Setup((64, 64, 64), Language.HIP, boundary=CYC3), True),
+    "wave3d_f32": (_wave_adj(3, CType.Float), Setup((64, 64, 64), Language.HIP, boundary=CYC3,
+                                                    lane=LANE_WAVE_F32), False),
+    "wave3d_f64": (_wave_adj(3, CType.Double), Setup((64, 64, 64), Language.HIP, boundary=CYC3,
+                                                     lane=LANE_WAVE_F64), True),
     # streaming along the last axis (rings of planes in LDS), checked bit for bit
     "life_i32_march": (_life, Setup((64, 64), Language.HIP, boundary=CYC2, tile=(64, 32),
                                     march=4), True),
