@@ -45,6 +45,19 @@ enum pr_ctype { PR_BOOL = 0, PR_INT = 1, PR_FLOAT = 2, PR_DOUBLE = 3 };
 
 typedef struct pr_machine pr_machine;
 
+/* Where a launch stands in a run of calls of one kernel (pr_run, pr_run_graph).  Only what
+ * the last call leaves behind can be seen, so
+ *   - a kernel with a form that makes several calls in one launch (Setup.fused) asks for it:
+ *     its launcher returns 1, with the kernel in `use` and its number of calls in `done`,
+ *   - a kernel none of whose launches reads a scalar it stores leaves its reductions and
+ *     scalar stores to the last call of the run, which repeats the scalar stores that count
+ *     calls (`pending` of them before its own). */
+typedef struct pr_run_state {
+  int left;                /* calls still to make, this one included */
+  int use, done;           /* set by a launcher that returns 1 */
+  int pending;             /* launches whose finish is still to come */
+} pr_run_state;
+
 /* What a generated launch callback receives (one kernel launch of one OM kernel). */
 typedef struct pr_launch_ctx {
   const void* const* cur;  /* per static: current device buffer (arrays) or NULL */
@@ -58,6 +71,7 @@ typedef struct pr_launch_ctx {
   int tiles[3];            /* tiles per axis */
   unsigned ntiles;         /* product of tiles[] */
   void* stream;            /* hipStream_t */
+  struct pr_run_state* run; /* null: one call, finished before the launcher returns */
 } pr_launch_ctx;
 
 typedef int (*pr_launch_fn)(const pr_launch_ctx* ctx);

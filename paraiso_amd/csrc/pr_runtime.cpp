@@ -39,6 +39,13 @@ struct GraphKey {
   }
 };
 
+// A run of calls captured as a graph, and the statics whose buffers it leaves swapped (its
+// launches, which may each make several calls, decide that: not the number of calls).
+struct RunGraph {
+  hipGraphExec_t exec = nullptr;
+  std::vector<int> flips;
+};
+
 struct pr_machine {
   const pr_machine_desc* d = nullptr;
   int n[3] = {1, 1, 1};              // array extents (local size plus margins)
@@ -56,7 +63,7 @@ struct pr_machine {
   std::vector<std::vector<size_t>> counter_idx; // [kernel][launch]
   hipStream_t stream = nullptr;
   bool own_stream = false;
-  std::map<GraphKey, hipGraphExec_t> graphs;
+  std::map<GraphKey, RunGraph> graphs;
   std::vector<std::vector<void*>> snaps;        // snapshot buffers
   std::vector<char*> snap_scal;
   std::vector<int> snap_sel;                    // statics a snapshot holds
@@ -101,12 +108,22 @@ std::vector<char> parity_key(const pr_machine* m) {
 // One call of kernel k.  A static with a non-null entry in cur_ov is read from that buffer
 // instead of the machine's own, and a store of it goes to next_ov[s]; such statics keep
 // their ping-pong parity (the adjoint driver's tape lives outside the machine's buffers).
-int launch_kernel_ov(pr_machine* m, int k, const void* const* cur_ov, void* const* next_ov) {
+// ``run``: the call's place in a run of calls of this kernel, or null; with it, a positive
+// result asks for another kernel (pr_run_state).
+int launch_kernel_ov(pr_machine* m, int k, const void* const* cur_ov, void* const* next_ov,
+                     pr_run_state* run = nullptr) {
   const pr_kernel_desc& kd = m->d->kernels[k];
   const int ns = m->d->n_static;
-  std::vector<const void*> cur(ns, nullptr);
-  std::vector<void*> next(ns, nullptr);
+  constexpr int FEW = 64;
+  const void* few_cur[FEW];
+  void* few_next[FEW];
+  std::vector<const void*> many_cur(ns > FEW ? ns : 0);
+  std::vector<void*> many_next(ns > FEW ? ns : 0);
+  const void** cur = ns > FEW ? many_cur.data() : few_cur;
+  void** next = ns > FEW ? many_next.data() : few_next;
   for (int s = 0; s < ns; ++s) {
+    cur[s] = nullptr;
+    next[s] = nullptr;
     if (m->d->statics[s].realm != PR_ARRAY) continue;
     if (cur_ov && cur_ov[s]) {
       cur[s] = cur_ov[s];
@@ -118,8 +135,8 @@ int launch_kernel_ov(pr_machine* m, int k, const void* const* cur_ov, void* cons
   }
   for (int l = 0; l < kd.n_launch; ++l) {
     pr_launch_ctx ctx;
-    ctx.cur = cur.data();
-    ctx.next = next.data();
+    ctx.cur = cur;
+    ctx.next = next;
     ctx.scal = m->scal;
     ctx.part = m->part + m->part_off[k][l];
     ctx.counter = reinterpret_cast<unsigned*>(m->scal + 8 * m->counter_idx[k][l]);
@@ -129,11 +146,13 @@ int launch_kernel_ov(pr_machine* m, int k, const void* const* cur_ov, void* cons
     }
     ctx.ntiles = m->ntiles[k][l];
     ctx.stream = m->stream;
+    ctx.run = run;
     hipEvent_t* ev = m->timing ? m->timing + 2 * ((size_t)m->timing_call * m->timing_stride + l)
                                : nullptr;
     if (ev) (void)hipEventRecord(ev[0], m->stream);
     int rc = kd.launches[l].fn(&ctx);
     if (ev) (void)hipEventRecord(ev[1], m->stream);
+    if (rc > 0) return rc;
     if (rc != 0) {
       hipError_t e = hipGetLastError();
       return fail(m, PR_E_HIP, std::string("launch ") + kd.name + "[" + std::to_string(l) +
@@ -148,6 +167,24 @@ int launch_kernel_ov(pr_machine* m, int k, const void* const* cur_ov, void* cons
 }
 
 int launch_kernel_once(pr_machine* m, int k) { return launch_kernel_ov(m, k, nullptr, nullptr); }
+
+// `count` calls of kernel k, of which only the last one's results can be seen.
+int launch_kernel_run(pr_machine* m, int k, int count) {
+  pr_run_state own = {}, other = {};
+  for (int c = 0; c < count;) {
+    own.left = count - c;
+    int rc = launch_kernel_ov(m, k, nullptr, nullptr, &own);
+    if (rc > 0) {   // a kernel that makes own.done calls at once
+      other.left = own.left / own.done;
+      rc = launch_kernel_ov(m, own.use, nullptr, nullptr, &other);
+      c += own.done;
+    } else {
+      ++c;
+    }
+    if (rc) return rc < 0 ? rc : fail(m, PR_E_UNSUPPORTED, "launch: fused kernel of a fused kernel");
+  }
+  return PR_OK;
+}
 
 }  // namespace
 
@@ -250,7 +287,7 @@ int pr_create(const pr_machine_desc* d, const int* local_size, pr_machine** out)
 int pr_destroy(pr_machine* m) {
   if (!m) return PR_E_INVALID;
   if (m->stream) hipStreamSynchronize(m->stream);
-  for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
+  for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second.exec);
   for (int b = 0; b < 2; ++b)
     for (void* p : m->buf[b])
       if (p) (void)hipFree(p);
@@ -272,7 +309,7 @@ int pr_set_stream(pr_machine* m, void* stream) {
   if (m->own_stream) hipStreamDestroy(m->stream);
   m->stream = static_cast<hipStream_t>(stream);
   m->own_stream = false;
-  for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
+  for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second.exec);
   m->graphs.clear();
   return PR_OK;
 }
@@ -287,11 +324,7 @@ const char* pr_last_error(const pr_machine* m) { return m ? m->err.c_str() : "nu
 
 int pr_run(pr_machine* m, int k, int count) {
   if (!m || k < 0 || k >= m->d->n_kernel || count < 0) return PR_E_INVALID;
-  for (int c = 0; c < count; ++c) {
-    int rc = launch_kernel_once(m, k);
-    if (rc) return rc;
-  }
-  return PR_OK;
+  return launch_kernel_run(m, k, count);
 }
 
 int pr_run_timed(pr_machine* m, int k, int count, double* launch_ms) {
@@ -330,22 +363,22 @@ int pr_run_graph(pr_machine* m, int k, int count) {
     std::vector<int> saved = m->cur;
     hipGraph_t g;
     PR_HIP(m, hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-    int rc = PR_OK;
-    for (int c = 0; c < count && rc == PR_OK; ++c) rc = launch_kernel_once(m, k);
+    int rc = launch_kernel_run(m, k, count);
     hipError_t e = hipStreamEndCapture(m->stream, &g);
+    const std::vector<int> after = m->cur;
     m->cur = saved;
     if (rc) return rc;
     if (e != hipSuccess) return hip_fail(m, e, "hipStreamEndCapture");
-    hipGraphExec_t ex;
-    e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
+    RunGraph rg;
+    e = hipGraphInstantiate(&rg.exec, g, nullptr, nullptr, 0);
     hipGraphDestroy(g);
     if (e != hipSuccess) return hip_fail(m, e, "hipGraphInstantiate");
-    it = m->graphs.emplace(key, ex).first;
+    rg.flips.resize(after.size());
+    for (size_t s = 0; s < after.size(); ++s) rg.flips[s] = after[s] ^ saved[s];
+    it = m->graphs.emplace(key, rg).first;
   }
-  PR_HIP(m, hipGraphLaunch(it->second, m->stream));
-  const pr_kernel_desc& kd = m->d->kernels[k];
-  if (count % 2)
-    for (int i = 0; i < kd.n_stored; ++i) m->cur[kd.stored[i]] ^= 1;
+  PR_HIP(m, hipGraphLaunch(it->second.exec, m->stream));
+  for (size_t s = 0; s < m->cur.size(); ++s) m->cur[s] ^= it->second.flips[s];
   return PR_OK;
 }
 
@@ -814,6 +847,7 @@ void grid_ctx(pr_machine* m, int k, int l, std::vector<const void*>& cur, std::v
   }
   ctx.ntiles = m->ntiles[k][l];
   ctx.stream = m->stream;
+  ctx.run = nullptr;
 }
 
 // Device block of packed arguments for (k, l) at the grids' current parity; built on first use
@@ -1203,6 +1237,7 @@ extern "C" int pr_run_noalloc(const pr_machine_desc* d, const int* local_size, i
       }
       ctx.ntiles = ntiles[l];
       ctx.stream = st;
+      ctx.run = nullptr;
       if (kd.launches[l].fn(&ctx) != 0)
         return noalloc_fail(err, err_len, PR_E_HIP, "launch %s[%d]: %s", kd.name, l,
                             hipGetErrorString(hipGetLastError()));

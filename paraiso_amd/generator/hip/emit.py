@@ -199,8 +199,8 @@ class MachineEmitter:
                  tile: Tuple[int, ...], fast_fp32: bool = False, batched: bool = False,
                  threads: int = NT, open_axes: Tuple[bool, ...] = (), margins=None,
                  regions=None, march: int = 0, prefetch: bool = True, persist: bool = False,
-                 forms: Optional[List[dict]] = None):
-        """``forms``: per kernel, the launch form overriding the machine's (keys ``tile``,
+                 forms: Optional[List[dict]] = None, fused=()):
+        """``fused``: (kernel, kernel making n calls of it, n) names (Setup.fused).  ``forms``: per kernel, the launch form overriding the machine's (keys ``tile``,
         ``threads``, ``persist``, ``march``), or None."""
         self.name = name
         self.nt = threads
@@ -236,6 +236,14 @@ class MachineEmitter:
         self._base = {"tile": self.tile, "threads": self.nt, "persist": self.persist,
                       "march": self.march, "lane": None}
         self.lane = None
+        names = [sch.kernel.name for sch in schedules]
+        self.fused: Dict[int, List[Tuple[int, int]]] = {}       # kernel -> [(n, kernel)]
+        for a, b, n in fused:
+            ka, kb = names.index(a), names.index(b)
+            if set(s for s, _ in schedules[ka].kernel.stores) != set(
+                    s for s, _ in schedules[kb].kernel.stores) or n < 2:
+                raise ValueError("%s does not stand for %d calls of %s" % (b, n, a))
+            self.fused.setdefault(ka, []).append((n, kb))
         self._lane_memo: Dict[Tuple[int, int], list] = {}
         self.forms = forms or [None] * len(schedules)
         self.ns = len(statics)
@@ -327,6 +335,7 @@ class MachineEmitter:
                    "int wide;  /* some axis shorter than tile plus reach: om_wrap takes the "
                    "remainder */",
                    "unsigned nwg;   /* reduction partials written (workgroups that reduce) */"]
+        fields.append("int repeat;   /* calls the finish kernel stands for */")
         if lane:
             fields += ["unsigned ln, lx, ly, mx, my;  /* register streaming: waves, strips along "
                        "x and y, reciprocals */", "int lc;  /* steps a wave streams */",
@@ -380,6 +389,8 @@ class MachineEmitter:
         # kernel's scalar stores (a launch with none of these has no finish kernel)
         needs_tail = bool(la.reduces) or bool(la.tail_scalars) or (la.commit and bool(sch.scalar_stores))
 
+        defer = needs_tail and self._defers(sch)
+
         def epilogue(index):
             e = []
             for j, r in enumerate(la.reduces):
@@ -393,15 +404,19 @@ class MachineEmitter:
         fin = []
         if needs_tail:
             f = fin.append
-            for n in nodes:
-                if n.realm is not Realm.Scalar:
-                    continue
-                lvl = sch.level[n.id]
-                if lvl == 0:
-                    f("  const %s u%d = %s;" % (n.ctype.c_name, n.id, self.scalar_expr(k, n.id)))
-                elif lvl <= L:
-                    f("  const %s u%d = *(const %s*)(a.scal + %d);" % (
-                        n.ctype.c_name, n.id, n.ctype.c_name, self.slot_off(ki, n.id)))
+
+            def scalars(ind):
+                for n in nodes:
+                    if n.realm is not Realm.Scalar:
+                        continue
+                    lvl = sch.level[n.id]
+                    if lvl == 0:
+                        f(ind + "const %s u%d = %s;" % (n.ctype.c_name, n.id, self.scalar_expr(k, n.id)))
+                    elif lvl <= L:
+                        f(ind + "const %s u%d = *(const %s*)(a.scal + %d);" % (
+                            n.ctype.c_name, n.id, n.ctype.c_name, self.slot_off(ki, n.id)))
+            if not defer:
+                scalars("  ")
             for j, r in enumerate(la.reduces):
                 a_ct = nodes[nodes[r].args[0]].ctype
                 at = acc_type(nodes[r].payload, a_ct)
@@ -411,6 +426,10 @@ class MachineEmitter:
                                               acc_init(nodes[r].payload, at),
                                               acc_op(nodes[r].payload, at), at.c_name))
             f("  if (threadIdx.x == 0) {")
+            if defer:
+                # the scalar stores of every call this finish stands for
+                f("  for (int it = 0; it < a.repeat; ++it) {")
+                scalars("    ")
             for v in la.tail_scalars:
                 n = nodes[v]
                 expr = "(%s)(fr%d)" % (n.ctype.c_name, v) if n.op == "reduce" else self.scalar_expr(k, v)
@@ -419,6 +438,8 @@ class MachineEmitter:
             if la.commit:
                 for s_, v in sch.scalar_stores:
                     f("    *(%s*)(a.scal + %d) = u%d;" % (nodes[v].ctype.c_name, 8 * s_, v))
+            if defer:
+                f("  }")
             f("  }")
         fin_decls = ["  __shared__ %s om_scr_%s[%d];" % (at.c_name, at.c_name, self.nt // 64)
                      for at in sorted(acc_types, key=lambda c: c.value)]
@@ -484,6 +505,7 @@ class MachineEmitter:
         else:
             h.append("  a.t0 = c->tiles[0]; a.t1 = c->tiles[1]; a.t2 = c->tiles[2]; a.ntiles = c->ntiles;")
         h.append("  a.m0 = om_udiv_magic((unsigned)a.t0); a.m1 = om_udiv_magic((unsigned)a.t1);")
+        h.append("  a.repeat = 1;")
         reach = self._max_reach(sch, la)
         h.append("  a.wide = (%s) ? 1 : 0;" % " || ".join(
             "c->n[%d] < %d" % (ax, self.tile[ax] + reach) for ax in range(self.ndim)))
@@ -522,6 +544,10 @@ class MachineEmitter:
             h.append("  return hipPeekAtLastError() == hipSuccess ? 0 : -1;")
         h.append("}")
         h.append("static int launch_%s(const pr_launch_ctx* c) {" % fn)
+        if L == 0:
+            for n_, kb in sorted(self.fused.get(ki, ()), reverse=True):
+                h.append("  if (c->run && c->run->left >= %d) { c->run->use = %d; c->run->done = %d; "
+                         "return 1; }" % (n_, kb, n_))
         h.append("  Args_%s a; fill_%s(c, a);" % (fn, fn))
         if lane:
             wg = self.lane["waves"]
@@ -534,12 +560,47 @@ class MachineEmitter:
         if has_work and block:
             h.append("  hipLaunchKernelGGL(%s, dim3(%s), dim3(%d), 0, (hipStream_t)c->stream, a);"
                      % (fn, "a.nwg" if persist else "a.ntiles", self.nt))
+        if defer:
+            # (a shorter rest of the run goes to this kernel's own fused forms or to itself)
+            h.append("  if (c->run) {")
+            h.append("    if (c->run->left > 1) { ++c->run->pending; "
+                     "return hipPeekAtLastError() == hipSuccess ? 0 : -1; }")
+            h.append("    a.repeat = c->run->pending + 1; c->run->pending = 0;")
+            h.append("  }")
         if needs_tail:
             h.append("  hipLaunchKernelGGL(%s_fin, dim3(1), dim3(%d), 0, (hipStream_t)c->stream, a);"
                      % (fn, self.nt))
         h.append("  return hipPeekAtLastError() == hipSuccess ? 0 : -1;")
         h.append("}")
         return kernel_src, "\n".join(h) + "\n"
+
+    def _defers(self, sch) -> bool:
+        """The kernel's finish may be left to the last call of a run (pr_run_state): no launch
+        reads a scalar the kernel stores, and no stored scalar counts something of every call
+        but what it can count from scalars alone (a reduction's result is then only the last
+        call's)."""
+        if len(sch.launches) != 1 or not sch.scalar_stores:
+            return False
+        nodes = sch.kernel.nodes
+        own = set(s for s, _ in sch.scalar_stores)
+
+        def reads(roots):
+            seen, stack = set(), list(roots)
+            while stack:
+                x = stack.pop()
+                if x not in seen:
+                    seen.add(x)
+                    stack.extend(nodes[x].args)
+            return [nodes[x] for x in seen]
+        carried = lambda ns: any(n.op == "load" and n.realm is Realm.Scalar and n.payload in own
+                                 for n in ns)
+        if carried(reads(sch.launches[0].targets)):
+            return False
+        for _, v in sch.scalar_stores:
+            ns = reads([v])
+            if carried(ns) and any(n.op == "reduce" for n in ns):
+                return False
+        return True
 
     # ------------------------------------------------------------ register streaming
     def _lane_plans(self, ki, k, la):

@@ -60,6 +60,9 @@ class Setup:
     # takes the form, "always": every grid does and no tile form is built, "ratio": see
     # MachineEmitter._lane_fill, "small": what differs on grids of fewer than "below" cells}
     lane: Optional[dict] = None
+    # ((kernel, kernel that makes n calls of it at once, n), ...), such as those transform.unroll
+    # adds: a run of at least n calls uses them, the largest n first
+    fused: Tuple[Tuple[str, str, int], ...] = ()
     # per OM kernel, a launch form overriding the above: ((kernel name, {"tile": ...,
     # "threads": ..., "persist": ..., "march": ..., "mat_gain": ..., "join": ...}), ...)
     kernel_forms: Tuple[Tuple[str, dict], ...] = ()

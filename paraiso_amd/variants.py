@@ -129,9 +129,13 @@ LANE_WAVE_F32 = {"rows": 8, "waves": 4, "occupancy": 3, "steps": 4, "fill": 3, "
 LANE_WAVE_F64 = {"rows": 4, "waves": 4, "occupancy": 2, "steps": 4, "fill": 3,
                  "small": {"rows": 3, "occupancy": 3, "below": 2_000_000}}
 
+# Runs of calls take the kernels that make several at once (transform.unroll).
+FUSED_LIFE = (("proceed", "proceed_x4", 4), ("proceed", "proceed_x8", 8))
+FUSED_WAVE = (("proceed", "proceed_x2", 2), ("proceed_adjoint", "proceed_adjoint_x2", 2))
+
 # name -> (OM factory, setup, precise)
 VARIANTS = {
-    "life_i32": (_life, Setup((64, 64), Language.HIP, boundary=CYC2), True),
+    "life_i32": (_life, Setup((64, 64), Language.HIP, boundary=CYC2, fused=FUSED_LIFE), True),
     "hydro_f32": (_hydro(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2, batched=True,
                                              lane=LANE_HYDRO_F32), False),
     # the headline machine's launch form (tile, work-items, resident tile loop), correctly
@@ -178,12 +182,12 @@ VARIANTS = {
                                                 ("proceed_stage2_adjoint", {"join": True}))),
                             True),
     "wave3d_f32": (_wave_adj(3, CType.Float), Setup((64, 64, 64), Language.HIP, boundary=CYC3,
-                                                    lane=LANE_WAVE_F32), False),
+                                                    lane=LANE_WAVE_F32, fused=FUSED_WAVE), False),
     "wave3d_f64": (_wave_adj(3, CType.Double), Setup((64, 64, 64), Language.HIP, boundary=CYC3,
-                                                     lane=LANE_WAVE_F64), True),
+                                                     lane=LANE_WAVE_F64, fused=FUSED_WAVE), True),
     # streaming along the last axis (rings of planes in LDS), checked bit for bit
     "life_i32_march": (_life, Setup((64, 64), Language.HIP, boundary=CYC2, tile=(64, 32),
-                                    march=4), True),
+                                    march=4, fused=FUSED_LIFE), True),
     "hydro_f64_march": (_hydro(CType.Double), Setup((64, 64), Language.HIP, boundary=CYC2,
                                                     tile=(64, 32), march=4), True),
     # a tile whose load and annotated-value tiles alone overflow LDS: the scheduler reads the
