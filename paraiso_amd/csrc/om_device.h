@@ -129,6 +129,14 @@ template <class T> __device__ __forceinline__ void om_put(T* row, int x, T v) {
   *(T*)((char*)row + (unsigned)x * (unsigned)sizeof(T)) = v;
 }
 
+// Lane r's two words become the 64-bit mask: row r of a square of bits (r is a constant after
+// unrolling; the masks are scalar).
+__device__ int om_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+__device__ __forceinline__ void om_turn(int r, unsigned long long mask, unsigned& w0, unsigned& w1) {
+  w0 = (unsigned)om_writelane((int)(unsigned)mask, r, (int)w0);
+  w1 = (unsigned)om_writelane((int)(unsigned)(mask >> 32), r, (int)w1);
+}
+
 template <class T, class Op> __device__ __forceinline__ T om_wave_reduce(T v, Op op) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = op(v, __shfl_xor(v, off, 64));

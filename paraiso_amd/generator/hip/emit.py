@@ -36,6 +36,7 @@ from ...om.arith import Op, ReduceOp
 from ...om.dyn import CType, Realm, fraction_to_float32
 from ...om.literal import c_literal
 from .ir import LKernel
+from .bits import BitEmitter, plan_bits
 from .lane import LaneEmitter, fused_products, plan_lane
 from .schedule import OUT, ArrayLaunch, KernelSchedule, ring_depth
 
@@ -619,6 +620,10 @@ class MachineEmitter:
                         break
                     f.update(f["small"])
                 p = plan_lane(k, la.targets, f.get("rows", 1), f.get("prefetch", 1))
+                if p is not None and f.get("bits"):
+                    nodes = k.nodes
+                    p = plan_bits(k, p, [v for _, v in la.stores],
+                                  [(nodes[r].payload, nodes[r].args[0]) for r in la.reduces])
                 if p is not None:
                     out.append((f, p, "%s_%s" % (self.fn_name(ki, la.index), name)))
             self._lane_memo[key] = out
@@ -626,10 +631,15 @@ class MachineEmitter:
 
     def lane_tile(self, form, plan) -> List[int]:
         """Cells a wave takes at least: strip width, rows and steps."""
+        if form.get("bits"):
+            return [plan.width, plan.height, 1]
         steps = form["steps"]
         return ([plan.width, steps, 1] if self.ndim == 2 else [plan.width, plan.rows, steps])
 
     def _lane_kernel(self, ki, k, la, f, plan, fn, name, uniforms) -> List[str]:
+        bits = plan if f.get("bits") else None
+        plan = bits.lane if bits else plan
+        width = bits.width if bits else plan.width
         nodes = k.nodes
         out: List[str] = []
         pre = list(uniforms)
@@ -693,14 +703,16 @@ class MachineEmitter:
         if self.ndim == 2:
             where += ["  const unsigned chunk = om_udiv(tile, a.lx, a.mx);",
                       "  const int X0 = (int)(tile - chunk * a.lx) * %d, S0 = (int)chunk * a.lc;"
-                      % plan.width]
+                      % width]
         else:
             where += ["  const unsigned q_ = om_udiv(tile, a.lx, a.mx), chunk = om_udiv(q_, a.ly, a.my);",
                       "  const int X0 = (int)(tile - q_ * a.lx) * %d, Y0 = (int)(q_ - chunk * a.ly) * %d, "
                       "S0 = (int)chunk * a.lc;" % (plan.width, plan.rows)]
         core = ["#pragma clang fp contract(off)"] if self.fast_fp32 else []
         core += ["    const int H = a.n%d - S0 < steps ? a.n%d - S0 : steps;" % (last, last)]
-        core += em.body(f.get("unroll", 1))
+        core += em.body(f.get("unroll", 1), width, peel=not bits)
+        if bits:
+            core = self._bit_square(bits, la, em, stores, reduces, core)
         wg = f["waves"]
 
         def epilogue(index, wave):
@@ -751,6 +763,21 @@ class MachineEmitter:
             out += ["}"]
         return out
 
+    def _bit_square(self, bits, la, em, stores, reduces, stream) -> List[str]:
+        """The wave's square in bit planes, or, where a cell holds neither 0 nor 1, by the
+        lines ``stream``."""
+        sq = BitEmitter(bits, em.load_ptr)
+        lo, hi = bits.cols
+        out = ["    bool done = false;", "    {",
+               "    const int x = X0 + lane - %d;" % lo,
+               "    const bool ok = lane >= %d && lane <= %d && x < a.n0;" % (lo, hi)]
+        out += ["    " + ln for ln in sq.pack()]
+        out += ["    if (!__any((bad & ~1) != 0)) {", "      done = true;",
+                "      const unsigned long long in = __ballot(ok);",
+                "      const unsigned m0 = (unsigned)in, m1 = (unsigned)(in >> 32); (void)m0; (void)m1;"]
+        out += ["      " + ln for ln in sq.body(stores, [(acc, t) for acc, _, _, _, t in reduces])]
+        return out + ["    }", "    }", "    if (!done) {"] + stream + ["    }"]
+
     def _own_tiles(self, lane) -> bool:
         """The runtime's tiles are the waves' (lane_tile) and the tile form counts its own: a
         single-grid launch with both forms, whose partials the waves outnumber otherwise."""
@@ -763,6 +790,9 @@ class MachineEmitter:
         if len(lanes) > 1:
             h.append("  if (cells < %dLL) a.lv = 1;" % lanes[1][0]["below"])
         for i, (f, plan, _) in enumerate(lanes):
+            bits = plan if f.get("bits") else None
+            plan = bits.lane if bits else plan
+            width = bits.width if bits else plan.width
             wg = f["waves"]
             # (grids below the smallest skip the search for the steps per wave: their launches
             # are short and the host issues them)
@@ -770,16 +800,20 @@ class MachineEmitter:
             h.append("  if (%s) a.ln = 0;" % few if few else "")
             h.append("  %sif (a.lv == %d) {" % ("else " if few else "", i))
             h += ["  a.lx = (unsigned)((a.n0 + %d) / %d); a.ly = %s;" % (
-                     plan.width - 1, plan.width,
+                     width - 1, width,
                      "(unsigned)((a.n1 + %d) / %d)" % (plan.rows - 1, plan.rows)
                      if self.ndim == 3 else "1u"),
                   "  a.mx = om_udiv_magic(a.lx); a.my = om_udiv_magic(a.ly);"]
             cap = "c->ntiles * %du" % wg if la.reduces else "0x7fffffffu"
-            h.append("  a.lc = om_lane_chunk(a.n%d, a.lx * a.ly, %.2f, %g, %s, %d, "
-                     "(unsigned)om_cus() * 4u);"
-                     % (last, plan.runup, f.get("fill", 1.2), cap, f["steps"]))
+            if bits:
+                h.append("  a.lc = %d;" % bits.height)
+            else:
+                h.append("  a.lc = om_lane_chunk(a.n%d, a.lx * a.ly, %.2f, %g, %s, %d, "
+                         "(unsigned)om_cus() * 4u);"
+                         % (last, plan.runup, f.get("fill", 1.2), cap, f["steps"]))
             h.append("  a.ln = a.lx * a.ly * (unsigned)((a.n%d + a.lc - 1) / a.lc);" % last)
-            wide = ["a.n0 < %d" % (64 + 2 * plan.reach), "a.n%d < %d" % (last, 2 * plan.reach)]
+            wide = ["a.n0 < %d" % (64 + 2 * plan.reach),
+                    "a.n%d < %d" % (last, 2 * plan.reach + (64 if bits else 0))]
             if self.ndim == 3:
                 wide.append("a.n1 < %d" % (plan.rows + 2 * plan.reach))
             wide = "(%s) ? 1 : 0" % " || ".join(wide)

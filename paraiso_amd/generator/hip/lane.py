@@ -341,11 +341,11 @@ class LaneEmitter:
         return moved[key]
 
     # ------------------------------------------------------------ parts
-    def setup(self) -> List[str]:
+    def setup(self, width: int) -> List[str]:
         """Per-wave coordinates: the lane's column, the rows' offsets and the kept registers."""
         p, out = self.p, []
         w = out.append
-        lo, hi = p.lanes
+        lo, hi = p.lanes[0], p.lanes[0] + width - 1
         w("const int x = X0 + lane - %d;" % lo)
         w("const bool ok = lane >= %d && lane <= %d && x < a.n0;" % (lo, hi))
         for place in sorted(set(v.place for v in p.values if v.op == "load" or
@@ -362,8 +362,9 @@ class LaneEmitter:
                         for d in range(1, v.depth + 1))))
         return out
 
-    def step(self, s: str, at: Optional[int]) -> List[str]:
-        """One step; ``at`` is its number in the run-up before the first store, or None."""
+    def step(self, s: str, at: Optional[int], when: str = "") -> List[str]:
+        """One step; ``at`` is its number in the run-up before the first store, or None;
+        ``when``: a condition on its stores and reductions."""
         p, out = self.p, []
         w = out.append
         on = lambda v: at is None or v.first <= at
@@ -410,8 +411,9 @@ class LaneEmitter:
                 vals = [target(t) for _, _, t in self.stores]
                 reds = [target(t) for _, _, _, _, t in self.reduces]
                 out.extend(pre)
-                if p.ndim == 3:
-                    w("if (Y0 + %d < a.n1) {" % r)
+                cond = [when] * bool(when) + ["Y0 + %d < a.n1" % r] * (p.ndim == 3)
+                if cond:
+                    w("if (%s) {" % " && ".join(cond))
                 if self.stores:
                     w("if (ok) {")
                     row = ("(size_t)(S0 + (%s)) * a.n0" % s if p.ndim == 2 else
@@ -421,7 +423,7 @@ class LaneEmitter:
                     w("}")
                 for (acc, op, tn, init, _), val in zip(self.reduces, reds):
                     w("%s = %s(%s, ok ? (%s)%s : (%s)%s);" % (acc, op, acc, tn, val, tn, init))
-                if p.ndim == 3:
+                if cond:
                     w("}")
         for v in p.values:
             if on(v):
@@ -430,16 +432,17 @@ class LaneEmitter:
                         w("%s = %s;" % (self.name(v, r, d), self.name(v, r, d - 1)))
         return out
 
-    def body(self, unroll: int) -> List[str]:
+    def body(self, unroll: int, width: int, peel: bool = True) -> List[str]:
         """The steps of a wave: the run-up, each step with only the values that something reads
-        later, then the loop."""
-        out = ["    " + ln for ln in self.setup()]
-        for s in range(self.p.first, 0):
+        later, then the loop.  Without ``peel`` the loop runs the run-up too (less code)."""
+        out = ["    " + ln for ln in self.setup(width)]
+        first = 0 if peel else self.p.first
+        for s in range(self.p.first, first):
             out.append("    {  // run-up, step %d" % s)
             out += ["      " + ln for ln in self.step("%d" % s, s)]
             out.append("    }")
         out.append("#pragma unroll %d" % max(1, unroll))
-        out.append("    for (int s = 0; s < H; ++s) {")
-        out += ["      " + ln for ln in self.step("s", None)]
+        out.append("    for (int s = %d; s < H; ++s) {" % first)
+        out += ["      " + ln for ln in self.step("s", None, "" if peel else "s >= 0")]
         out.append("    }")
         return out

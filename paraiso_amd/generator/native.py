@@ -58,7 +58,8 @@ class Setup:
     # below which a launch gains from more (om_lane_chunk), "steps": least steps per wave,
     # "unroll", "prefetch": steps the loads are issued ahead, "min_cells": smallest grid that
     # takes the form, "always": every grid does and no tile form is built, "ratio": see
-    # MachineEmitter._lane_fill, "small": what differs on grids of fewer than "below" cells}
+    # MachineEmitter._lane_fill, "small": what differs on grids of fewer than "below" cells,
+    # "bits": bit planes instead (hip/bits.py)}
     lane: Optional[dict] = None
     # ((kernel, kernel that makes n calls of it at once, n), ...), such as those transform.unroll
     # adds: a run of at least n calls uses them, the largest n first

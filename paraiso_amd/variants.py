@@ -19,11 +19,11 @@ OPEN2 = (A.Condition.Open,) * 2
 
 
 def _life():
-    """Life with ``proceed_x4`` and ``proceed_x8``: four or eight generations per launch
-    (temporal blocking)."""
+    """Life with ``proceed_x4``, ``proceed_x8`` and ``proceed_x16``: four, eight or sixteen
+    generations per launch (temporal blocking)."""
     from .schemes.life import life_om
     from .transform import unroll
-    return unroll(unroll(life_om(), "proceed", 4), "proceed", 8)
+    return unroll(unroll(unroll(life_om(), "proceed", 4), "proceed", 8), "proceed", 16)
 
 
 def _life_plain():
@@ -129,13 +129,24 @@ LANE_WAVE_F32 = {"rows": 8, "waves": 4, "occupancy": 3, "steps": 4, "fill": 3, "
 LANE_WAVE_F64 = {"rows": 4, "waves": 4, "occupancy": 2, "steps": 4, "fill": 3,
                  "small": {"rows": 3, "occupancy": 3, "below": 2_000_000}}
 
+# Life in bit planes (generator/hip/bits.py): 1024^2, 16 generations 7.1 us a launch (the LDS
+# tiles took 10 us for eight), 4096^2 eight 31 us against 162 (4.4 TB/s).  One generation a
+# launch is a matter of latency below a million cells, where the tiles are as fast.
+BITS = {"bits": True, "waves": 4, "occupancy": 4, "steps": 8}
+LIFE_FORMS = (("proceed", {"lane": dict(BITS, min_cells=1_000_000)}),
+              ("proceed_x4", {"lane": BITS}), ("proceed_x8", {"lane": BITS}),
+              ("proceed_x16", {"lane": BITS}))
+
 # Runs of calls take the kernels that make several at once (transform.unroll).
-FUSED_LIFE = (("proceed", "proceed_x4", 4), ("proceed", "proceed_x8", 8))
+FUSED_LIFE = (("proceed", "proceed_x4", 4), ("proceed", "proceed_x8", 8),
+              ("proceed", "proceed_x16", 16), ("proceed_x8", "proceed_x16", 2),
+              ("proceed_x4", "proceed_x16", 4), ("proceed_x4", "proceed_x8", 2))
 FUSED_WAVE = (("proceed", "proceed_x2", 2), ("proceed_adjoint", "proceed_adjoint_x2", 2))
 
 # name -> (OM factory, setup, precise)
 VARIANTS = {
-    "life_i32": (_life, Setup((64, 64), Language.HIP, boundary=CYC2, fused=FUSED_LIFE), True),
+    "life_i32": (_life, Setup((64, 64), Language.HIP, boundary=CYC2, fused=FUSED_LIFE,
+                              kernel_forms=LIFE_FORMS), True),
     "hydro_f32": (_hydro(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2, batched=True,
                                              lane=LANE_HYDRO_F32), False),
     # the headline machine's launch form (tile, work-items, resident tile loop), correctly
