@@ -45,6 +45,13 @@ enum pr_ctype { PR_BOOL = 0, PR_INT = 1, PR_FLOAT = 2, PR_DOUBLE = 3 };
 
 typedef struct pr_machine pr_machine;
 
+/* Partials of a kernel's first launch that its second folds itself, one value per workgroup of
+ * the first (n 0: they have been folded into the scalar slots). */
+typedef struct pr_fold {
+  const char* part;
+  unsigned stride, n;
+} pr_fold;
+
 /* Where a launch stands in a run of calls of one kernel (pr_run, pr_run_graph).  Only what
  * the last call leaves behind can be seen, so
  *   - a kernel with a form that makes several calls in one launch (Setup.fused) asks for it:
@@ -72,6 +79,7 @@ typedef struct pr_launch_ctx {
   unsigned ntiles;         /* product of tiles[] */
   void* stream;            /* hipStream_t */
   struct pr_run_state* run; /* null: one call, finished before the launcher returns */
+  struct pr_fold* fold;    /* null: a launch's reductions are finished before the next starts */
 } pr_launch_ctx;
 
 typedef int (*pr_launch_fn)(const pr_launch_ctx* ctx);

@@ -63,6 +63,14 @@ __device__ __forceinline__ int om_clamp(int x, int n) { return x < 0 ? 0 : (x < 
 template <class T> __device__ __forceinline__ T om_max(T a, T b) { return (a < b) ? b : a; }
 template <class T> __device__ __forceinline__ T om_min(T a, T b) { return (b < a) ? b : a; }
 
+// a * b <= 0 ? 0 : (|a| < |b| ? a : b): the median of a, b and 0, and b where one is not a
+// number (fast FP32 builds: the same but for a product that underflows to 0, where the limiter
+// returns the smaller value as exact arithmetic would).  Three instructions for six.
+__device__ __forceinline__ float om_minmod(float a, float b) {
+  const float m = __builtin_amdgcn_fmed3f(a, b, 0.0f);
+  return __builtin_isunordered(a, b) ? b : m;
+}
+
 struct OmSum {
   template <class T> __device__ __forceinline__ T operator()(T a, T b) const { return a + b; }
 };
@@ -135,6 +143,21 @@ __device__ int om_writelane(int value, int lane, int old) __asm("llvm.amdgcn.wri
 __device__ __forceinline__ void om_turn(int r, unsigned long long mask, unsigned& w0, unsigned& w1) {
   w0 = (unsigned)om_writelane((int)(unsigned)mask, r, (int)w0);
   w1 = (unsigned)om_writelane((int)(unsigned)(mask >> 32), r, (int)w1);
+}
+
+// A value that every lane holds, in scalar registers, rounded to its type (nothing is
+// contracted across it: the same bits as a value read back from memory).
+__device__ __forceinline__ int om_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ bool om_uniform(bool v) { return om_uniform((int)v) != 0; }
+__device__ __forceinline__ float om_uniform(float v) {
+  asm("" : "+v"(v));   // (the compiler sees through readfirstlane of a uniform value)
+  return __builtin_bit_cast(float, om_uniform(__builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ double om_uniform(double v) {
+  asm("" : "+v"(v));
+  struct P { int lo, hi; };
+  const P p = __builtin_bit_cast(P, v);
+  return __builtin_bit_cast(double, P{om_uniform(p.lo), om_uniform(p.hi)});
 }
 
 template <class T, class Op> __device__ __forceinline__ T om_wave_reduce(T v, Op op) {

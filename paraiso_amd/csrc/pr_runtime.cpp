@@ -133,6 +133,7 @@ int launch_kernel_ov(pr_machine* m, int k, const void* const* cur_ov, void* cons
     cur[s] = m->buf[m->cur[s]][s];
     if (m->stored_any[s]) next[s] = m->buf[1 - m->cur[s]][s];
   }
+  pr_fold fold = {};
   for (int l = 0; l < kd.n_launch; ++l) {
     pr_launch_ctx ctx;
     ctx.cur = cur;
@@ -147,6 +148,7 @@ int launch_kernel_ov(pr_machine* m, int k, const void* const* cur_ov, void* cons
     ctx.ntiles = m->ntiles[k][l];
     ctx.stream = m->stream;
     ctx.run = run;
+    ctx.fold = &fold;
     hipEvent_t* ev = m->timing ? m->timing + 2 * ((size_t)m->timing_call * m->timing_stride + l)
                                : nullptr;
     if (ev) (void)hipEventRecord(ev[0], m->stream);
@@ -848,6 +850,7 @@ void grid_ctx(pr_machine* m, int k, int l, std::vector<const void*>& cur, std::v
   ctx.ntiles = m->ntiles[k][l];
   ctx.stream = m->stream;
   ctx.run = nullptr;
+  ctx.fold = nullptr;
 }
 
 // Device block of packed arguments for (k, l) at the grids' current parity; built on first use
@@ -1224,6 +1227,7 @@ extern "C" int pr_run_noalloc(const pr_machine_desc* d, const int* local_size, i
       cur[s] = buffers[2 * s + parity[s]];
       if (stored[s]) next[s] = buffers[2 * s + 1 - parity[s]];
     }
+    pr_fold fold = {};
     for (int l = 0; l < kd.n_launch; ++l) {
       pr_launch_ctx ctx;
       ctx.cur = cur;
@@ -1238,6 +1242,7 @@ extern "C" int pr_run_noalloc(const pr_machine_desc* d, const int* local_size, i
       ctx.ntiles = ntiles[l];
       ctx.stream = st;
       ctx.run = nullptr;
+      ctx.fold = &fold;
       if (kd.launches[l].fn(&ctx) != 0)
         return noalloc_fail(err, err_len, PR_E_HIP, "launch %s[%d]: %s", kd.name, l,
                             hipGetErrorString(hipGetLastError()));

@@ -37,7 +37,7 @@ from ...om.dyn import CType, Realm, fraction_to_float32
 from ...om.literal import c_literal
 from .ir import LKernel
 from .bits import BitEmitter, plan_bits
-from .lane import LaneEmitter, fused_products, plan_lane
+from .lane import MINMOD, LaneEmitter, fused_products, plan_lane
 from .schedule import OUT, ArrayLaunch, KernelSchedule, ring_depth
 
 NT = 256
@@ -336,7 +336,18 @@ class MachineEmitter:
                    "int wide;  /* some axis shorter than tile plus reach: om_wrap takes the "
                    "remainder */",
                    "unsigned nwg;   /* reduction partials written (workgroups that reduce) */"]
-        fields.append("int repeat;   /* calls the finish kernel stands for */")
+        fields.append("int repeat;   /* calls the finish stands for */")
+        # the second of two launches folds the first one's partials itself: every workgroup
+        # reads them (at most a few KB) where a finish kernel between the two would have cost
+        # a launch
+        first = sch.launches[0]
+        folds = len(sch.launches) == 2 and bool(first.reduces) and bool(first.targets)
+        fold = first if folds and L == 1 else None
+        if fold:
+            fields += ["const char* fpart;", "unsigned fstride, fn;"]
+        # a launch without reductions stores its scalars itself (no workgroup reads them)
+        inline = (bool(la.targets) and not la.reduces and la.commit and bool(sch.scalar_stores)
+                  and not self._reads_stored(sch, la.targets))
         if lane:
             fields += ["unsigned ln, lx, ly, mx, my;  /* register streaming: waves, strips along "
                        "x and y, reciprocals */", "int lc;  /* steps a wave streams */",
@@ -355,17 +366,55 @@ class MachineEmitter:
         coords = self._tile_coords("tile")
         body: List[str] = []
         w = body.append
-        # uniform scalars
-        for n in nodes:
-            if n.realm is not Realm.Scalar:
-                continue
-            lvl = sch.level[n.id]
-            if lvl == 0:
-                w("  const %s u%d = %s;" % (n.ctype.c_name, n.id, self.scalar_expr(k, n.id)))
-            elif lvl <= L:
-                w("  const %s u%d = *(const %s*)(a.scal + %d);" % (
-                    n.ctype.c_name, n.id, n.ctype.c_name, self.slot_off(ki, n.id)))
-        uniforms = list(body)
+        def uniform_lines(nt, folding):
+            """Uniform scalars; ``folding``: those of the previous launch's finish from its
+            partials (for an ``nt``-thread workgroup), else from their slots."""
+            out = []
+            fk = fold.kernel_override or sch.kernel if fold else None
+            if fold and folding:
+                for j, r in enumerate(fold.reduces):
+                    at = acc_type(fk.nodes[r].payload, fk.nodes[fk.nodes[r].args[0]].ctype)
+                    init, op = (g(fk.nodes[r].payload, at) for g in (acc_init, acc_op))
+                    out.append("  const %s fr%d = a.fn ? om_partials_reduce<%d>((const %s*)a.fpart + %d * a.fstride, "
+                               "(int)a.fn, (%s)%s, %s, om_fold_%s) : (%s)%s;" % (
+                                   at.c_name, r, nt, at.c_name, j, at.c_name, init, op, at.c_name,
+                                   at.c_name, init))
+            for n in nodes:
+                if n.realm is not Realm.Scalar:
+                    continue
+                lvl = sch.level[n.id]
+                tn = n.ctype.c_name
+                if lvl == 0:
+                    out.append("  const %s u%d = %s;" % (tn, n.id, self.scalar_expr(k, n.id)))
+                elif lvl <= L:
+                    slot = "*(const %s*)(a.scal + %d)" % (tn, self.slot_off(ki, n.id))
+                    if fold and folding:
+                        e = "fr%d" % n.id if n.op == "reduce" else self.scalar_expr(k, n.id)
+                        slot = "a.fn ? om_uniform((%s)(%s)) : %s" % (tn, e, slot)
+                    out.append("  const %s u%d = %s;" % (tn, n.id, slot))
+            return out
+
+        def fold_scratch(nt):
+            fk = fold.kernel_override or sch.kernel if fold else None
+            return ["  __shared__ %s om_fold_%s[%d];" % (at.c_name, at.c_name, nt // 64)
+                    for at in sorted(set(acc_type(fk.nodes[r].payload,
+                                                  fk.nodes[fk.nodes[r].args[0]].ctype)
+                                         for r in fold.reduces), key=lambda c: c.value)] if fold else []
+
+        def own_scalars(first_thread):
+            """The scalar stores of a launch that makes them itself, by one thread."""
+            if not inline:
+                return []
+            out = ["  if (%s) {" % first_thread]
+            if defer:
+                out.append("  for (int it = 0; it < a.repeat; ++it) {")
+                out += uniform_lines(0, False)
+            for s_, v in sch.scalar_stores:
+                out.append("    *(%s*)(a.scal + %d) = u%d;" % (nodes[v].ctype.c_name, 8 * s_, v))
+            return out + ["  }"] * (2 if defer else 1)
+        needs_tail = not inline and (bool(la.reduces) or bool(la.tail_scalars)
+                                     or (la.commit and bool(sch.scalar_stores)))
+        defer = (needs_tail or inline) and self._defers(sch)
         # LDS views
         for v, b in sorted(la.lds.items()):
             w("  %s* __restrict__ s%d = (%s*)(smem + %d);" % (
@@ -375,7 +424,8 @@ class MachineEmitter:
             a_ct = nodes[nodes[r].args[0]].ctype
             at = acc_type(nodes[r].payload, a_ct)
             w("  %s acc%d = %s;" % (at.c_name, r, acc_init(nodes[r].payload, at)))
-        pre = list(body)             # tile-independent: scalars, LDS views, accumulators
+        views = list(body)           # tile-independent: scalars, LDS views, accumulators
+        pre = uniform_lines(self.nt, True) + views
         work: List[str] = []
         if has_work and self.march:
             self._emit_march(k, la, work.append)
@@ -388,10 +438,6 @@ class MachineEmitter:
         # ---- epilogue: per-workgroup partials; the finish kernel does the rest
         # the finish kernel: reductions, scalars computed from them, and the commit of the
         # kernel's scalar stores (a launch with none of these has no finish kernel)
-        needs_tail = bool(la.reduces) or bool(la.tail_scalars) or (la.commit and bool(sch.scalar_stores))
-
-        defer = needs_tail and self._defers(sch)
-
         def epilogue(index):
             e = []
             for j, r in enumerate(la.reduces):
@@ -434,7 +480,8 @@ class MachineEmitter:
             for v in la.tail_scalars:
                 n = nodes[v]
                 expr = "(%s)(fr%d)" % (n.ctype.c_name, v) if n.op == "reduce" else self.scalar_expr(k, v)
-                f("    const %s u%d = %s;" % (n.ctype.c_name, v, expr))
+                # (rounded one by one, as where the next launch folds the partials itself)
+                f("    const %s u%d = om_uniform((%s)(%s));" % (n.ctype.c_name, v, n.ctype.c_name, expr))
                 f("    *(%s*)(a.scal + %d) = u%d;" % (n.ctype.c_name, self.slot_off(ki, v), v))
             if la.commit:
                 for s_, v in sch.scalar_stores:
@@ -447,15 +494,18 @@ class MachineEmitter:
         ks = [struct]
         if lane:
             for form, plan, name in lanes:
-                ks.extend(self._lane_kernel(ki, k, la, form, plan, fn, name, uniforms))
-        core = "\n".join(coords + pre + work + epilogue("tile"))
+                ks.extend(self._lane_kernel(ki, k, la, form, plan, fn, name, uniform_lines,
+                                            fold_scratch, own_scalars))
+        core = "\n".join(coords + pre + work + epilogue("tile")
+                         + own_scalars("tile == 0 && threadIdx.x == 0"))
         if block:
             ks.append("extern \"C\" __global__ void __launch_bounds__(%d) %s(Args_%s a) {" % (self.nt, fn, fn))
-            ks.extend(decls)
+            ks.extend(decls + fold_scratch(self.nt))
             if persist:
                 ks.extend(pre)
                 ks.extend(loop)
                 ks.extend(epilogue("blockIdx.x"))
+                ks.extend(own_scalars("blockIdx.x == 0 && threadIdx.x == 0"))
             else:
                 ks.append("  unsigned tile = blockIdx.x;")
                 ks.append("  if ((a.ntiles & 7u) == 0u) tile = (tile & 7u) * (a.ntiles >> 3) + (tile >> 3);")
@@ -472,7 +522,8 @@ class MachineEmitter:
             ks.append("  const int g = tile_grid[b];")
             ks.append("  const Args_%s a = grids[g];" % fn)
             ks.append("  const unsigned tile = b - tile_base[g];")
-            ks.append(core)
+            ks += coords + uniform_lines(self.nt, False) + views + work + epilogue("tile")
+            ks += own_scalars("tile == 0 && threadIdx.x == 0")
             ks.append("}")
         if needs_tail:
             fcore = "\n".join(fin)
@@ -516,6 +567,9 @@ class MachineEmitter:
             h.append("  a.nwg = a.ntiles;")
         if lane:
             h.extend(self._lane_fill(la, lanes))
+        if fold:
+            h.append("  a.fpart = c->fold ? c->fold->part : nullptr;")
+            h.append("  a.fstride = c->fold ? c->fold->stride : 0u; a.fn = c->fold ? c->fold->n : 0u;")
         h.append("}")
         h.append("static void pack_%s(const pr_launch_ctx* c, void* out) {" % fn)
         # (a batch's waves follow the runtime's table of tiles: a fixed number of steps each)
@@ -550,6 +604,14 @@ class MachineEmitter:
                 h.append("  if (c->run && c->run->left >= %d) { c->run->use = %d; c->run->done = %d; "
                          "return 1; }" % (n_, kb, n_))
         h.append("  Args_%s a; fill_%s(c, a);" % (fn, fn))
+        if defer:
+            # (a shorter rest of the run goes to this kernel's own fused forms or to itself)
+            h.append("  bool finish = true;")
+            h.append("  if (c->run) {")
+            h.append("    if (c->run->left > 1) { ++c->run->pending; a.repeat = 0; finish = false; }")
+            h.append("    else { a.repeat = c->run->pending + 1; c->run->pending = 0; }")
+            h.append("  }")
+            h.append("  (void)finish;")
         if lane:
             wg = self.lane["waves"]
             h.append("  if (a.ln) {")
@@ -561,19 +623,31 @@ class MachineEmitter:
         if has_work and block:
             h.append("  hipLaunchKernelGGL(%s, dim3(%s), dim3(%d), 0, (hipStream_t)c->stream, a);"
                      % (fn, "a.nwg" if persist else "a.ntiles", self.nt))
-        if defer:
-            # (a shorter rest of the run goes to this kernel's own fused forms or to itself)
-            h.append("  if (c->run) {")
-            h.append("    if (c->run->left > 1) { ++c->run->pending; "
-                     "return hipPeekAtLastError() == hipSuccess ? 0 : -1; }")
-            h.append("    a.repeat = c->run->pending + 1; c->run->pending = 0;")
-            h.append("  }")
         if needs_tail:
-            h.append("  hipLaunchKernelGGL(%s_fin, dim3(1), dim3(%d), 0, (hipStream_t)c->stream, a);"
-                     % (fn, self.nt))
+            cond = "if (finish) " if defer else ""
+            if folds and L == 0:
+                # up to 1024 partials (8 KB) every workgroup of the next launch folds them
+                h.append("  if (c->fold) { c->fold->part = a.part; c->fold->stride = a.ntiles; "
+                         "c->fold->n = a.nwg <= 1024u ? a.nwg : 0u; }")
+                cond = "if (!c->fold || !c->fold->n) "
+            h.append("  %shipLaunchKernelGGL(%s_fin, dim3(1), dim3(%d), 0, (hipStream_t)c->stream, a);"
+                     % (cond, fn, self.nt))
         h.append("  return hipPeekAtLastError() == hipSuccess ? 0 : -1;")
         h.append("}")
         return kernel_src, "\n".join(h) + "\n"
+
+    def _reads_stored(self, sch, roots) -> bool:
+        """Some value of ``roots`` depends on a scalar static that the kernel stores."""
+        nodes = sch.kernel.nodes
+        own = set(s for s, _ in sch.scalar_stores)
+        seen, stack = set(), list(roots)
+        while stack:
+            x = stack.pop()
+            if x not in seen:
+                seen.add(x)
+                stack.extend(nodes[x].args)
+        return any(nodes[x].op == "load" and nodes[x].realm is Realm.Scalar
+                   and nodes[x].payload in own for x in seen)
 
     def _defers(self, sch) -> bool:
         """The kernel's finish may be left to the last call of a run (pr_run_state): no launch
@@ -583,23 +657,16 @@ class MachineEmitter:
         if len(sch.launches) != 1 or not sch.scalar_stores:
             return False
         nodes = sch.kernel.nodes
-        own = set(s for s, _ in sch.scalar_stores)
-
-        def reads(roots):
-            seen, stack = set(), list(roots)
+        if self._reads_stored(sch, sch.launches[0].targets):
+            return False
+        for _, v in sch.scalar_stores:
+            seen, stack = set(), [v]
             while stack:
                 x = stack.pop()
                 if x not in seen:
                     seen.add(x)
                     stack.extend(nodes[x].args)
-            return [nodes[x] for x in seen]
-        carried = lambda ns: any(n.op == "load" and n.realm is Realm.Scalar and n.payload in own
-                                 for n in ns)
-        if carried(reads(sch.launches[0].targets)):
-            return False
-        for _, v in sch.scalar_stores:
-            ns = reads([v])
-            if carried(ns) and any(n.op == "reduce" for n in ns):
+            if self._reads_stored(sch, [v]) and any(nodes[x].op == "reduce" for x in seen):
                 return False
         return True
 
@@ -619,7 +686,8 @@ class MachineEmitter:
                     if "small" not in f:
                         break
                     f.update(f["small"])
-                p = plan_lane(k, la.targets, f.get("rows", 1), f.get("prefetch", 1))
+                p = plan_lane(k, la.targets, f.get("rows", 1), f.get("prefetch", 1),
+                              fast=self.fast_fp32)
                 if p is not None and f.get("bits"):
                     nodes = k.nodes
                     p = plan_bits(k, p, [v for _, v in la.stores],
@@ -636,13 +704,14 @@ class MachineEmitter:
         steps = form["steps"]
         return ([plan.width, steps, 1] if self.ndim == 2 else [plan.width, plan.rows, steps])
 
-    def _lane_kernel(self, ki, k, la, f, plan, fn, name, uniforms) -> List[str]:
+    def _lane_kernel(self, ki, k, la, f, plan, fn, name, uniform_lines, fold_scratch,
+                     own_scalars) -> List[str]:
         bits = plan if f.get("bits") else None
         plan = bits.lane if bits else plan
         width = bits.width if bits else plan.width
         nodes = k.nodes
         out: List[str] = []
-        pre = list(uniforms)
+        pre: List[str] = []
         for v in plan.uniform:
             n = nodes[v]
             tn = n.ctype.c_name
@@ -669,35 +738,40 @@ class MachineEmitter:
                             acc_init(nodes[r].payload, at), arg))
         stores = [("a.st%d" % self.sidx(ki, s), nodes[v].ctype.c_name, v) for s, v in la.stores]
 
-        def consts(v):
-            return [k.exact.get(x) for x in nodes[v.node].args]
+        def factor(v, args, i):
+            """Argument i of a product as a C operand."""
+            if v.consts[i] is None:
+                return args[i]
+            return c_literal(_split_const(v.consts[i])[0], CType.Float)
 
-        def split(v):
-            """(x, y) of a fusable product: multiplication or division by a value."""
-            if v.op != "arith" or v.ctype is not CType.Float or not self.fast_fp32:
-                return None
-            c = consts(v)
-            if v.payload[0] is Op.Mul:
-                return "mul" if c[0] is None and c[1] is None else None
-            return "div" if v.payload[0] is Op.Div and c[0] is None and c[1] is None else None
+        def product(v):
+            """A multiplication of a fast FP32 build that an addition may take in: of two
+            values, or by a constant that is not multiplied by compensated."""
+            if (v.op != "arith" or v.ctype is not CType.Float or not self.fast_fp32
+                    or v.payload[0] is not Op.Mul or all(c is not None for c in v.consts)):
+                return False
+            return all(c is None or _split_const(c)[1] == 0
+                       or (self._comp is not None and c not in self._comp) for c in v.consts)
 
         def arith(v, args):
             op, cast_to = v.payload
+            if op == MINMOD:
+                return "om_minmod(%s, %s)" % tuple(args)
             pair = next((x for x in args if isinstance(x, tuple)), None)
             if pair is not None:
                 i = args.index(pair)
-                x, y = pair[1]
-                if pair[0].payload[0] is Op.Div:
-                    y = "__builtin_amdgcn_rcpf(%s)" % y
+                x, y = (factor(pair[0], pair[1], j) for j in range(2))
                 other = args[1 - i]
                 if op is Op.Sub and i == 1:
                     return "__builtin_fmaf(-%s, %s, %s)" % (x, y, other)
                 return "__builtin_fmaf(%s, %s, %s%s)" % (x, y, "-" if op is Op.Sub else "", other)
-            types = [nodes[x].ctype for x in nodes[v.node].args]
-            return device_arith(op, args, cast_to, types, v.ctype, self.fast_fp32, consts(v),
+            if self.fast_fp32 and op is Op.Max and v.consts[0] is not None and v.ctype is CType.Float:
+                # om_max of a number and x is the hardware maximum, NaN included
+                return "__builtin_fmaxf(%s, %s)" % (args[0], args[1])
+            return device_arith(op, args, cast_to, v.types, v.ctype, self.fast_fp32, v.consts,
                                 self._comp)
         em = LaneEmitter(plan, k, lambda s: "a.ld%d" % self.sidx(ki, s), arith, stores, reduces,
-                         fused_products(plan, lambda v: split(v) is not None))
+                         fused_products(plan, product))
         last = self.ndim - 1
         where = ["  const int lane = threadIdx.x & 63;"]
         if self.ndim == 2:
@@ -737,9 +811,10 @@ class MachineEmitter:
                 "  const unsigned wv = b_ * %du + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);"
                 % wg]
         out.append("extern \"C\" __global__ void %s %s(Args_%s a) {" % (bounds, name, fn))
-        out += scr + wave + ["  const unsigned tile = wv;"] + where
-        out += ["  const int steps = a.lc;"] + pre
-        out += ["  if (wv < a.ln) {"] + core + ["  }"] + epilogue("b_", False) + ["}"]
+        out += scr + fold_scratch(64 * wg) + wave + ["  const unsigned tile = wv;"] + where
+        out += ["  const int steps = a.lc;"] + uniform_lines(64 * wg, True) + pre
+        out += ["  if (wv < a.ln) {"] + core + ["  }"] + epilogue("b_", False)
+        out += own_scalars("b_ == 0 && threadIdx.x == 0") + ["}"]
         if self.batched and f.get("always"):
             # a tile of the batch is a wave's; `split`: a workgroup's, each wave taking its
             # share of the steps, where the batch has too few tiles to fill the chip
@@ -755,12 +830,12 @@ class MachineEmitter:
                     "  const int steps = split ? a.lc / %d : a.lc;" % wg]
             out += [ln.replace("S0 = (int)chunk * a.lc;",
                                "S0 = (int)chunk * a.lc + (split ? (int)w_ * steps : 0);")
-                    for ln in where] + pre
+                    for ln in where] + uniform_lines(64 * wg, False) + pre
             out += ["  if (S0 < a.n%d) {" % last] + core + ["  }"]
             if la.reduces:
                 out += (["  if (split) {"] + epilogue("tile", False) + ["  } else {"]
                         + epilogue("tile", True) + ["  }"])
-            out += ["}"]
+            out += own_scalars("tile == 0 && lane == 0 && (!split || w_ == 0)") + ["}"]
         return out
 
     def _bit_square(self, bits, la, em, stores, reduces, stream) -> List[str]:

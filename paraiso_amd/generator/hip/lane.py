@@ -37,8 +37,9 @@ class LaneValue:
     op: str                                   # load index arith
     args: List[Tuple[object, Tuple[int, ...]]]   # (value id, offset) or (uniform name, None)
     ctype: CType
-    payload: object
-    node: int                                 # a node of the lowered kernel it stands for
+    payload: object                           # static, axis, or (operator, cast)
+    consts: List[object]                      # per argument: its exact constant value, or None
+    types: List[CType]                        # per argument
     place: int = 0                            # x placement
     lead: int = 0                             # streaming-axis placement
     first: int = 0                            # first step that computes it (0: first store)
@@ -72,10 +73,18 @@ class LanePlan:
                 / max(1, sum(size(v) for v in self.values)))
 
 
-def plan_lane(k: LKernel, targets: List[int], rows: int = 1, prefetch: int = 1
-              ) -> Optional[LanePlan]:
+MINMOD = "minmod"             # of fast FP32 plans: see om_minmod
+
+
+def plan_lane(k: LKernel, targets: List[int], rows: int = 1, prefetch: int = 1,
+              fast: bool = False) -> Optional[LanePlan]:
     """The register-streaming plan of the values ``targets`` of one launch, or None when the
-    launch has no array value to read (nothing to stream)."""
+    launch has no array value to read (nothing to stream).
+
+    ``fast`` (fast FP32 builds): a division is a product with a reciprocal of its own, which
+    other divisions share; the reciprocal of a Select between two values whose reciprocals are
+    there anyway is the Select of those (a transcendental instruction takes four slots, a
+    select one); and ``a * b <= 0 ? 0 : (|a| < |b| ? a : b)`` is one operation."""
     nd = k.ndim
     if nd not in (2, 3):
         return None
@@ -95,12 +104,58 @@ def plan_lane(k: LKernel, targets: List[int], rows: int = 1, prefetch: int = 1
     where: Dict[int, Tuple[object, Optional[Tuple[int, ...]]]] = {}
     uniform: List[int] = []
 
-    def add(op, args, ct, payload, node):
-        key = (op, tuple(args), ct, payload if op != "arith" else (payload[0], payload[1]))
+    def add(op, args, ct, payload, consts=(), types=()):
+        key = (op, tuple(args), ct, payload)
         if key not in memo:
             memo[key] = len(values)
-            values.append(LaneValue(len(values), op, list(args), ct, payload, node))
+            values.append(LaneValue(len(values), op, list(args), ct, payload, list(consts),
+                                    list(types)))
         return memo[key]
+
+    def operation(op, cast, ps, ct, consts, types):
+        """(value, offset) of an operation on (value, offset) arguments, one not uniform."""
+        origin = next(o for _, o in ps if o is not None)
+        args = tuple((b, None if o is None else tuple(x - y for x, y in zip(o, origin)))
+                     for b, o in ps)
+        return add("arith", args, ct, (op, cast), consts, types), origin
+
+    def reciprocal(p):
+        b, o = p
+        v = values[b]
+        if v.op == "arith" and v.payload[0] is Op.Select and v.args[0][1] is not None:
+            c, x, y = v.args
+            there = [("arith", ((z[0], zero),), CType.Float, (Op.Inv, None)) for z in (x, y)]
+            if all(z[1] is not None and t in memo for z, t in zip((x, y), there)):
+                ix, iy = ((memo[t], z[1]) for t, z in zip(there, (x, y)))
+                w, ow = operation(Op.Select, None, [c, ix, iy], CType.Float, [None] * 3,
+                                  [CType.Bool, CType.Float, CType.Float])
+                return w, tuple(i + j for i, j in zip(o, ow))
+        return add("arith", ((b, zero),), CType.Float, (Op.Inv, None), [None], [CType.Float]), o
+
+    def minmod(v):
+        """(a, b) where value v is a * b <= 0 ? 0 : (|a| < |b| ? a : b), else None."""
+        def is_op(p, op):
+            return (p[1] == zero and values[p[0]].op == "arith"
+                    and values[p[0]].payload[0] is op)
+        if v.op != "arith" or v.payload[0] is not Op.Select or v.ctype is not CType.Float:
+            return None
+        cond, nil, inner = v.args
+        if v.consts[1] != 0 or not is_op(cond, Op.LE) or not is_op(inner, Op.Select):
+            return None
+        le, sel = values[cond[0]], values[inner[0]]
+        if le.consts[1] != 0 or not is_op(le.args[0], Op.Mul) or not is_op(sel.args[0], Op.LT):
+            return None
+        a, b = sel.args[1:]
+        lt = values[sel.args[0][0]]
+        if set(values[le.args[0][0]].args) != {a, b} or a[1] is None or b[1] is None:
+            return None
+        for p, x in zip(lt.args, (a, b)):
+            if p[1] is None or values[p[0]].op != "arith" or values[p[0]].payload[0] is not Op.Abs:
+                return None
+            y, oy = values[p[0]].args[0]
+            if oy is None or (y, tuple(i + j for i, j in zip(oy, p[1]))) != x:
+                return None
+        return [a, b]
 
     for v in sorted(cone):
         n = nodes[v]
@@ -108,22 +163,28 @@ def plan_lane(k: LKernel, targets: List[int], rows: int = 1, prefetch: int = 1
             uniform.append(v)
             where[v] = ("n%d" % v, None)
         elif n.op in ("load", "index"):
-            where[v] = (add(n.op, (), n.ctype, n.payload, v), zero)
+            where[v] = (add(n.op, (), n.ctype, n.payload), zero)
         elif n.op == "shift":
             b, o = where[n.args[0]]
             where[v] = (b, None if o is None else tuple(x - y for x, y in zip(o, n.payload)))
-            if o is None:
-                where[v] = (b, None)
         elif n.op == "arith":
             ps = [where[a] for a in n.args]
-            origin = next((o for _, o in ps if o is not None), None)
-            if origin is None:
+            if all(o is None for _, o in ps):
                 uniform.append(v)
                 where[v] = ("n%d" % v, None)
                 continue
-            args = tuple((b, None if o is None else tuple(x - y for x, y in zip(o, origin)))
-                         for b, o in ps)
-            where[v] = (add("arith", args, n.ctype, n.payload, v), origin)
+            op, cast = n.payload
+            consts = [k.exact.get(a) for a in n.args]
+            types = [nodes[a].ctype for a in n.args]
+            if (fast and op is Op.Div and n.ctype is CType.Float and consts[1] is None
+                    and ps[1][1] is not None):
+                ps = [ps[0], reciprocal(ps[1])]
+                op, consts = Op.Mul, [consts[0], None]
+            where[v] = operation(op, cast, ps, n.ctype, consts, types)
+            m = minmod(values[where[v][0]]) if fast else None
+            if m is not None:
+                w, o = operation(MINMOD, None, m, CType.Float, [None] * 2, [CType.Float] * 2)
+                where[v] = (w, tuple(i + j for i, j in zip(o, where[v][1])))
         else:
             raise NotImplementedError(n.op)
     tgt = {t: where[t] for t in targets if where[t][1] is not None}
