@@ -45,6 +45,10 @@ enum pr_ctype { PR_BOOL = 0, PR_INT = 1, PR_FLOAT = 2, PR_DOUBLE = 3 };
 
 typedef struct pr_machine pr_machine;
 
+/* Space for reduction partials: one per tile, and at least this many per reduction, so that a
+ * launch may take other tiles than its descriptor's on a small grid. */
+#define PR_MIN_PARTIALS 4096
+
 /* Partials of a kernel's first launch that its second folds itself, one value per workgroup of
  * the first (n 0: they have been folded into the scalar slots). */
 typedef struct pr_fold {

@@ -84,6 +84,9 @@ size_t ctype_size(int ct) {
   return 8;
 }
 
+// Partials a launch of nt tiles has space for, per reduction.
+size_t partials(unsigned nt) { return nt < PR_MIN_PARTIALS ? PR_MIN_PARTIALS : nt; }
+
 int fail(pr_machine* m, int code, const std::string& msg) {
   if (m) m->err = msg;
   return code;
@@ -250,7 +253,7 @@ int pr_create(const pr_machine_desc* d, const int* local_size, pr_machine** out)
       m->tiles[k].push_back(t);
       m->ntiles[k].push_back(nt);
       m->part_off[k].push_back(part_bytes);
-      part_bytes += ((size_t)ld.n_reduce * nt * 8 + 255) / 256 * 256;
+      part_bytes += ((size_t)ld.n_reduce * partials(nt) * 8 + 255) / 256 * 256;
     }
   }
   hipError_t e;
@@ -1149,7 +1152,7 @@ extern "C" int pr_run_noalloc(const pr_machine_desc* d, const int* local_size, i
     }
     ntiles[l] = nt;
     part_off[l] = need;
-    need += round256((size_t)ld.n_reduce * nt * 8);
+    need += round256((size_t)ld.n_reduce * partials(nt) * 8);
   }
   size_t array_off[PR_NOALLOC_MAX_STATICS];
   for (int s = 0; s < ns; ++s) {

@@ -54,6 +54,9 @@ def _hip_sources(setup: Setup, om: OM, precise: bool = True) -> Tuple[Plan, str,
     for ki, k in enumerate(lowered):
         f = setup.form_of(om_opt.kernels[ki].name)
         f["tile"] = tuple(f["tile"]) if f["tile"] else tile
+        f["tiny"] = [dict(t, schedule=schedule_kernel(k, tuple(t["tile"]), lds_budget(t["threads"]),
+                                                      t.get("mat_gain", 48)))
+                     for t in f["tiny"]]
         forms.append(f)
         scheds.append(schedule_kernel(k, f["tile"], lds_budget(f["threads"]), f["mat_gain"],
                                       f["march"], f.get("manifest", ()), f.get("delayed", ()),

@@ -27,6 +27,7 @@ Per-point expressions follow the reference's SASA naming (``a<node>_<cursor>``,
 from __future__ import annotations
 
 import re
+from contextlib import contextmanager
 from fractions import Fraction
 from typing import Dict, List, Optional, Set, Tuple
 
@@ -235,8 +236,9 @@ class MachineEmitter:
         self.schedules = schedules
         self.tile = tuple(tile) + (1,) * (3 - len(tile))
         self._base = {"tile": self.tile, "threads": self.nt, "persist": self.persist,
-                      "march": self.march, "lane": None}
+                      "march": self.march, "lane": None, "tiny": ()}
         self.lane = None
+        self.tiny = ()
         names = [sch.kernel.name for sch in schedules]
         self.fused: Dict[int, List[Tuple[int, int]]] = {}       # kernel -> [(n, kernel)]
         for a, b, n in fused:
@@ -276,6 +278,18 @@ class MachineEmitter:
         self.march = int(f["march"])
         self.persist = bool(f["persist"]) and not self.march
         self.lane = f["lane"]
+        self.tiny = f["tiny"] or ()
+
+    @contextmanager
+    def _form(self, tile, threads: int):
+        """Another tile and work-items, one tile per workgroup, for the emission of one form."""
+        kept = self.tile, self.nt, self.march, self.persist
+        self.tile = tuple(tile) + (1,) * (3 - len(tile))
+        self.nt, self.march, self.persist = int(threads), 0, False
+        try:
+            yield
+        finally:
+            self.tile, self.nt, self.march, self.persist = kept
 
     def fn_name(self, ki: int, launch: int) -> str:
         """Kernel symbol: machine, OM kernel and launch, so that profiles name them."""
@@ -348,24 +362,21 @@ class MachineEmitter:
         # a launch without reductions stores its scalars itself (no workgroup reads them)
         inline = (bool(la.targets) and not la.reduces and la.commit and bool(sch.scalar_stores)
                   and not self._reads_stored(sch, la.targets))
+        if self.tiny:
+            fields.append("int bv;   /* which of the launch's tiles */")
         if lane:
             fields += ["unsigned ln, lx, ly, mx, my;  /* register streaming: waves, strips along "
                        "x and y, reciprocals */", "int lc;  /* steps a wave streams */",
                        "int lv;  /* which of the launch's streaming forms */"]
         struct = "struct Args_%s {\n  %s\n};\n" % (fn, "\n  ".join(fields))
 
-        decls: List[str] = []
-        if la.lds_bytes:
-            decls.append("  __shared__ __align__(16) char smem[%d];" % la.lds_bytes)
-        acc_types = set()
-        for r in la.reduces:
-            acc_types.add(acc_type(nodes[r].payload, nodes[nodes[r].args[0]].ctype))
-        for at in sorted(acc_types, key=lambda c: c.value):
-            decls.append("  __shared__ %s om_scr_%s[%d];" % (at.c_name, at.c_name,
-                                                             self.nt // 64))
-        coords = self._tile_coords("tile")
-        body: List[str] = []
-        w = body.append
+        acc_types = set(acc_type(nodes[r].payload, nodes[nodes[r].args[0]].ctype)
+                        for r in la.reduces)
+
+        def scratch(nt):
+            return ["  __shared__ %s om_scr_%s[%d];" % (at.c_name, at.c_name, nt // 64)
+                    for at in sorted(acc_types, key=lambda c: c.value)]
+
         def uniform_lines(nt, folding):
             """Uniform scalars; ``folding``: those of the previous launch's finish from its
             partials (for an ``nt``-thread workgroup), else from their slots."""
@@ -415,29 +426,6 @@ class MachineEmitter:
         needs_tail = not inline and (bool(la.reduces) or bool(la.tail_scalars)
                                      or (la.commit and bool(sch.scalar_stores)))
         defer = (needs_tail or inline) and self._defers(sch)
-        # LDS views
-        for v, b in sorted(la.lds.items()):
-            w("  %s* __restrict__ s%d = (%s*)(smem + %d);" % (
-                nodes[v].ctype.c_name, v, nodes[v].ctype.c_name, b.offset))
-        # accumulators
-        for r in la.reduces:
-            a_ct = nodes[nodes[r].args[0]].ctype
-            at = acc_type(nodes[r].payload, a_ct)
-            w("  %s acc%d = %s;" % (at.c_name, r, acc_init(nodes[r].payload, at)))
-        views = list(body)           # tile-independent: scalars, LDS views, accumulators
-        pre = uniform_lines(self.nt, True) + views
-        work: List[str] = []
-        if has_work and self.march:
-            self._emit_march(k, la, work.append)
-        elif has_work:
-            for ph in la.phases:
-                self._emit_phase(k, la, ph, work.append)
-        persist = has_work and self.persist
-        if persist:
-            loop = self._persistent_loop(k, la)
-        # ---- epilogue: per-workgroup partials; the finish kernel does the rest
-        # the finish kernel: reductions, scalars computed from them, and the commit of the
-        # kernel's scalar stores (a launch with none of these has no finish kernel)
         def epilogue(index):
             e = []
             for j, r in enumerate(la.reduces):
@@ -448,6 +436,55 @@ class MachineEmitter:
                 e.append("    if (threadIdx.x == 0) ((%s*)a.part)[%d * a.ntiles + %s] = br; }" % (
                     at.c_name, j, index))
             return e if has_work else []
+
+        def tile_kernel(name, la_x, batched):
+            """The tile form of the launch as scheduled in ``la_x``, under the emitter's current
+            tile, work-items and loop form; ``batched``: also over the tiles of many grids."""
+            out: List[str] = []
+            decls = scratch(self.nt)
+            if la_x.lds_bytes:
+                decls.insert(0, "  __shared__ __align__(16) char smem[%d];" % la_x.lds_bytes)
+            views = ["  %s* __restrict__ s%d = (%s*)(smem + %d);" % (
+                nodes[v].ctype.c_name, v, nodes[v].ctype.c_name, b.offset)
+                for v, b in sorted(la_x.lds.items())]
+            for r in la.reduces:
+                at = acc_type(nodes[r].payload, nodes[nodes[r].args[0]].ctype)
+                views.append("  %s acc%d = %s;" % (at.c_name, r, acc_init(nodes[r].payload, at)))
+            coords = self._tile_coords("tile")
+            work: List[str] = []
+            if has_work and self.march:
+                self._emit_march(k, la_x, work.append)
+            elif has_work:
+                for ph in la_x.phases:
+                    self._emit_phase(k, la_x, ph, work.append)
+            out.append("extern \"C\" __global__ void __launch_bounds__(%d) %s(Args_%s a) {"
+                       % (self.nt, name, fn))
+            out += decls + fold_scratch(self.nt)
+            if has_work and self.persist:
+                out += uniform_lines(self.nt, True) + views + self._persistent_loop(k, la_x)
+                out += epilogue("blockIdx.x")
+                out += own_scalars("blockIdx.x == 0 && threadIdx.x == 0")
+            else:
+                out.append("  unsigned tile = blockIdx.x;")
+                out.append("  if ((a.ntiles & 7u) == 0u) tile = (tile & 7u) * (a.ntiles >> 3) + (tile >> 3);")
+                out += coords + uniform_lines(self.nt, True) + views + work + epilogue("tile")
+                out += own_scalars("tile == 0 && threadIdx.x == 0")
+            out.append("}")
+            if batched:
+                # the tiles of many grids in one launch (grid table in device memory)
+                out.append("extern \"C\" __global__ void __launch_bounds__(%d) %s_batched(const Args_%s* __restrict__ grids, "
+                           "const int* __restrict__ tile_grid, const unsigned* __restrict__ tile_base, unsigned total) {"
+                           % (self.nt, name, fn))
+                out += decls
+                out.append("  unsigned b = blockIdx.x;")
+                out.append("  if ((total & 7u) == 0u) b = (b & 7u) * (total >> 3) + (b >> 3);")
+                out.append("  const int g = tile_grid[b];")
+                out.append("  const Args_%s a = grids[g];" % fn)
+                out.append("  const unsigned tile = b - tile_base[g];")
+                out += coords + uniform_lines(self.nt, False) + views + work + epilogue("tile")
+                out += own_scalars("tile == 0 && threadIdx.x == 0")
+                out.append("}")
+            return out
         fin = []
         if needs_tail:
             f = fin.append
@@ -489,42 +526,29 @@ class MachineEmitter:
             if defer:
                 f("  }")
             f("  }")
-        fin_decls = ["  __shared__ %s om_scr_%s[%d];" % (at.c_name, at.c_name, self.nt // 64)
-                     for at in sorted(acc_types, key=lambda c: c.value)]
+        fin_decls = scratch(self.nt)
         ks = [struct]
         if lane:
             for form, plan, name in lanes:
                 ks.extend(self._lane_kernel(ki, k, la, form, plan, fn, name, uniform_lines,
                                             fold_scratch, own_scalars))
-        core = "\n".join(coords + pre + work + epilogue("tile")
-                         + own_scalars("tile == 0 && threadIdx.x == 0"))
+        persist = has_work and self.persist
         if block:
-            ks.append("extern \"C\" __global__ void __launch_bounds__(%d) %s(Args_%s a) {" % (self.nt, fn, fn))
-            ks.extend(decls + fold_scratch(self.nt))
-            if persist:
-                ks.extend(pre)
-                ks.extend(loop)
-                ks.extend(epilogue("blockIdx.x"))
-                ks.extend(own_scalars("blockIdx.x == 0 && threadIdx.x == 0"))
-            else:
-                ks.append("  unsigned tile = blockIdx.x;")
-                ks.append("  if ((a.ntiles & 7u) == 0u) tile = (tile & 7u) * (a.ntiles >> 3) + (tile >> 3);")
-                ks.append(core)
-            ks.append("}")
-        # batched form: the tiles of many grids in one launch (grid table in device memory)
-        if self.batched and block:
-            ks.append("extern \"C\" __global__ void __launch_bounds__(%d) %s_batched(const Args_%s* __restrict__ grids, "
-                      "const int* __restrict__ tile_grid, const unsigned* __restrict__ tile_base, unsigned total) {"
-                      % (self.nt, fn, fn))
-            ks.extend(decls)
-            ks.append("  unsigned b = blockIdx.x;")
-            ks.append("  if ((total & 7u) == 0u) b = (b & 7u) * (total >> 3) + (b >> 3);")
-            ks.append("  const int g = tile_grid[b];")
-            ks.append("  const Args_%s a = grids[g];" % fn)
-            ks.append("  const unsigned tile = b - tile_base[g];")
-            ks += coords + uniform_lines(self.nt, False) + views + work + epilogue("tile")
-            ks += own_scalars("tile == 0 && threadIdx.x == 0")
-            ks.append("}")
+            ks += tile_kernel(fn, la, self.batched)
+        reach = self._max_reach(sch, la)
+        # smaller tiles for small grids: (cells below, name, tile, work-items, reach)
+        small = []
+        for i, f in enumerate(self.tiny if block and has_work else ()):
+            la_x = f["schedule"].launches[L] if len(f["schedule"].launches) == len(sch.launches) else None
+            if la_x is None or la_x.targets != la.targets or any(
+                    nodes[v].op == "load" and self.sidx(ki, nodes[v].payload) not in loads
+                    for v in la_x.lc if nodes[v].realm is Realm.Array):
+                continue
+            with self._form(f["tile"], f["threads"]):
+                self._launch_reach = 0
+                name = "%s_tile%d" % (fn, i)
+                ks += tile_kernel(name, la_x, False)
+                small.append((f["below"], name, self.tile, self.nt, self._max_reach(sch, la_x)))
         if needs_tail:
             fcore = "\n".join(fin)
             ks.append("extern \"C\" __global__ void __launch_bounds__(%d) %s_fin(Args_%s a) {" % (self.nt, fn, fn))
@@ -542,7 +566,8 @@ class MachineEmitter:
 
         # ---- host launcher
         h = []
-        h.append("static void fill_%s(const pr_launch_ctx* c, Args_%s& a) {" % (fn, fn))
+        h.append("static void fill_%s(const pr_launch_ctx* c, Args_%s& a, bool batch = false) {" % (fn, fn))
+        h.append("  (void)batch;")
         for s in loads:
             h.append("  a.ld%d = (const %s*)c->cur[%d];" % (s, self.statics[s].dyn.ctype.c_name, s))
         for s in stores:
@@ -558,7 +583,6 @@ class MachineEmitter:
             h.append("  a.t0 = c->tiles[0]; a.t1 = c->tiles[1]; a.t2 = c->tiles[2]; a.ntiles = c->ntiles;")
         h.append("  a.m0 = om_udiv_magic((unsigned)a.t0); a.m1 = om_udiv_magic((unsigned)a.t1);")
         h.append("  a.repeat = 1;")
-        reach = self._max_reach(sch, la)
         h.append("  a.wide = (%s) ? 1 : 0;" % " || ".join(
             "c->n[%d] < %d" % (ax, self.tile[ax] + reach) for ax in range(self.ndim)))
         if persist:
@@ -567,6 +591,24 @@ class MachineEmitter:
             h.append("  a.nwg = a.ntiles;")
         if lane:
             h.extend(self._lane_fill(la, lanes))
+        if small:
+            h.append("  a.bv = 0;")
+            h.append("  if (!batch%s) {" % (" && !a.ln" if lane else ""))
+            h.append("    const long long all = (long long)a.n0 * a.n1 * a.n2;")
+            h.append("    const unsigned space = c->ntiles < PR_MIN_PARTIALS ? PR_MIN_PARTIALS : c->ntiles;")
+            for i, (below, _, T_, nt_, reach_) in enumerate(small):
+                h.append("    if (!a.bv && all < %dLL) {" % below)
+                h.append("      const int t0 = (a.n0 + %d) / %d, t1 = (a.n1 + %d) / %d, t2 = (a.n2 + %d) / %d;"
+                         % (T_[0] - 1, T_[0], T_[1] - 1, T_[1], T_[2] - 1, T_[2]))
+                h.append("      const unsigned nt = (unsigned)t0 * (unsigned)t1 * (unsigned)t2;")
+                h.append("      if (nt <= space) {")
+                h.append("        a.bv = %d; a.t0 = t0; a.t1 = t1; a.t2 = t2; a.ntiles = a.nwg = nt;" % (i + 1))
+                h.append("        a.m0 = om_udiv_magic((unsigned)t0); a.m1 = om_udiv_magic((unsigned)t1);")
+                h.append("        a.wide = (%s) ? 1 : 0;" % " || ".join(
+                    "a.n%d < %d" % (ax, T_[ax] + reach_) for ax in range(self.ndim)))
+                h.append("      }")
+                h.append("    }")
+            h.append("  }")
         if fold:
             h.append("  a.fpart = c->fold ? c->fold->part : nullptr;")
             h.append("  a.fstride = c->fold ? c->fold->stride : 0u; a.fn = c->fold ? c->fold->n : 0u;")
@@ -574,7 +616,7 @@ class MachineEmitter:
         h.append("static void pack_%s(const pr_launch_ctx* c, void* out) {" % fn)
         # (a batch's waves follow the runtime's table of tiles: a fixed number of steps each)
         fixed = "" if block else " a.lc = %d; a.ln = c->ntiles;" % self.lane["steps"]
-        h.append("  Args_%s a; fill_%s(c, a); a.nwg = c->ntiles;%s memcpy(out, &a, sizeof a);"
+        h.append("  Args_%s a; fill_%s(c, a, true); a.nwg = c->ntiles;%s memcpy(out, &a, sizeof a);"
                  % (fn, fn, fixed))
         h.append("}")
         h.append("static int launch_batched_%s(const pr_batch_ctx* bc) {" % fn)
@@ -620,6 +662,9 @@ class MachineEmitter:
                 h.append("  %sif (a.lv == %d) hipLaunchKernelGGL(%s, dim3(a.nwg), dim3(%d), 0, "
                          "(hipStream_t)c->stream, a);" % ("else " if i else "", i, name, 64 * wg))
             h.append("  }" + (" else" if block else ""))
+        for i, (_, name, _, nt_, _) in enumerate(small):
+            h.append("  if (a.bv == %d) hipLaunchKernelGGL(%s, dim3(a.ntiles), dim3(%d), 0, "
+                     "(hipStream_t)c->stream, a);\n  else" % (i + 1, name, nt_))
         if has_work and block:
             h.append("  hipLaunchKernelGGL(%s, dim3(%s), dim3(%d), 0, (hipStream_t)c->stream, a);"
                      % (fn, "a.nwg" if persist else "a.ntiles", self.nt))

@@ -61,6 +61,9 @@ class Setup:
     # MachineEmitter._lane_fill, "small": what differs on grids of fewer than "below" cells,
     # "bits": bit planes instead (hip/bits.py)}
     lane: Optional[dict] = None
+    # smaller tiles for small single grids, smallest first: ({"below": cells, "tile": ...,
+    # "threads": ..., "mat_gain": ...}, ...)
+    tiny: Tuple[dict, ...] = ()
     # ((kernel, kernel that makes n calls of it at once, n), ...), such as those transform.unroll
     # adds: a run of at least n calls uses them, the largest n first
     fused: Tuple[Tuple[str, str, int], ...] = ()
@@ -89,7 +92,7 @@ class Setup:
         """The launch form of one OM kernel: the machine's, with the kernel's overrides."""
         f = {"tile": self.tile, "threads": self.threads, "persist": self.persist,
              "march": self.march, "mat_gain": self.mat_gain, "join": self.join,
-             "lane": self.lane}
+             "lane": self.lane, "tiny": self.tiny}
         for name, over in self.kernel_forms:
             if name == kernel:
                 f.update(over)

@@ -115,6 +115,14 @@ def _optable(real):
 # 31.9 and 33.7 at 512^2, 55.9 and 51.2 at 700^2, 344 and 250 at 2048^2).
 LANE_HYDRO_F32 = {"waves": 4, "occupancy": 2, "steps": 4, "min_cells": 600_000}
 LANE_HYDRO_F64 = {"waves": 4, "occupancy": 2, "steps": 4, "min_cells": 400_000}
+# Below that, tiles by the number of cells: a small grid is a matter of how long a workgroup
+# takes, which small tiles with one loop point per work-item and phase shorten.  FP32, us a
+# step at 96x64, 400x300, 512^2, 700^2: 16x8 tiles 7.7 13.7 20.1 30.2, 32x16 10.6 12.2 14.4
+# 21.7, 64x32 resident 17.8 18.5 18.7 22.3.  FP64 at 96x64, 300x200, 512^2: 16x8 11.5 21.2 64,
+# 16x16 13.4 15.4 43.6, 32x32 resident 26.9 28.0 31.7.
+TINY_HYDRO_F32 = ({"below": 60_000, "tile": (16, 8), "threads": 320},)
+TINY_HYDRO_F64 = ({"below": 30_000, "tile": (16, 8), "threads": 320},
+                  {"below": 120_000, "tile": (16, 16), "threads": 512})
 # Batches: a tile is 32 steps of one wave (24 and 40: within 1%), 0.92 -> 0.64 ms a step for
 # 256 uneven grids.
 LANE_HYDRO_BATCH = {"waves": 4, "occupancy": 2, "steps": 32, "always": True}
@@ -148,7 +156,7 @@ VARIANTS = {
     "life_i32": (_life, Setup((64, 64), Language.HIP, boundary=CYC2, fused=FUSED_LIFE,
                               kernel_forms=LIFE_FORMS), True),
     "hydro_f32": (_hydro(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2, batched=True,
-                                             lane=LANE_HYDRO_F32), False),
+                                             lane=LANE_HYDRO_F32, tiny=TINY_HYDRO_F32), False),
     # the headline machine's launch form (tile, work-items, resident tile loop), correctly
     # rounded: checked bit for bit against the oracle
     "hydro_f32_precise": (_hydro(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2,
@@ -158,7 +166,7 @@ VARIANTS = {
     "hydro_f32_batch": (_hydro(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2,
                                                    batched=True, lane=LANE_HYDRO_BATCH), False),
     "hydro_f64": (_hydro(CType.Double), Setup((64, 64), Language.HIP, boundary=CYC2, batched=True,
-                                              lane=LANE_HYDRO_F64), True),
+                                              lane=LANE_HYDRO_F64, tiny=TINY_HYDRO_F64), True),
     # register streaming at every size, correctly rounded: checked bit for bit
     "hydro_f64_lane": (_hydro(CType.Double), Setup((64, 64), Language.HIP, boundary=CYC2,
                                                    batched=True, lane=LANE_HYDRO_BATCH), True),
