@@ -390,6 +390,7 @@ class MachineEmitter:
                                "(int)a.fn, (%s)%s, %s, om_fold_%s) : (%s)%s;" % (
                                    at.c_name, r, nt, at.c_name, j, at.c_name, init, op, at.c_name,
                                    at.c_name, init))
+                out.append("  if (a.fn) __syncthreads();")
             for n in nodes:
                 if n.realm is not Realm.Scalar:
                     continue
@@ -405,9 +406,12 @@ class MachineEmitter:
                     out.append("  const %s u%d = %s;" % (tn, n.id, slot))
             return out
 
-        def fold_scratch(nt):
+        def fold_scratch(nt, smem=0):
+            """Scratch of the fold: the LDS tiles' own space where there is enough (nothing is in
+            it yet), so that tiles that fill the CU's LDS leave room."""
             fk = fold.kernel_override or sch.kernel if fold else None
-            return ["  __shared__ %s om_fold_%s[%d];" % (at.c_name, at.c_name, nt // 64)
+            return [("  %s* const om_fold_%s = (%s*)smem;" % ((at.c_name,) * 3) if smem >= nt // 8
+                     else "  __shared__ %s om_fold_%s[%d];" % (at.c_name, at.c_name, nt // 64))
                     for at in sorted(set(acc_type(fk.nodes[r].payload,
                                                   fk.nodes[fk.nodes[r].args[0]].ctype)
                                          for r in fold.reduces), key=lambda c: c.value)] if fold else []
@@ -459,7 +463,7 @@ class MachineEmitter:
                     self._emit_phase(k, la_x, ph, work.append)
             out.append("extern \"C\" __global__ void __launch_bounds__(%d) %s(Args_%s a) {"
                        % (self.nt, name, fn))
-            out += decls + fold_scratch(self.nt)
+            out += decls + fold_scratch(self.nt, la_x.lds_bytes)
             if has_work and self.persist:
                 out += uniform_lines(self.nt, True) + views + self._persistent_loop(k, la_x)
                 out += epilogue("blockIdx.x")

@@ -123,9 +123,10 @@ LANE_HYDRO_F64 = {"waves": 4, "occupancy": 2, "steps": 4, "min_cells": 400_000}
 TINY_HYDRO_F32 = ({"below": 60_000, "tile": (16, 8), "threads": 320},)
 TINY_HYDRO_F64 = ({"below": 30_000, "tile": (16, 8), "threads": 320},
                   {"below": 120_000, "tile": (16, 16), "threads": 512})
-# Batches: a tile is 32 steps of one wave (24 and 40: within 1%), 0.92 -> 0.64 ms a step for
+# Batches: a tile is 24 steps of one wave, 0.92 -> 0.58 ms a step (32: 0.59; small batches 17.6 us
+# against 18.5) for
 # 256 uneven grids.
-LANE_HYDRO_BATCH = {"waves": 4, "occupancy": 2, "steps": 32, "always": True}
+LANE_HYDRO_BATCH = {"waves": 4, "occupancy": 2, "steps": 24, "always": True}
 # LinearWave 3-D: a lane holds rows of y, fewer on small grids (64^3: 11.6 us a step with 8, 8.9
 # with 4; 128^3 15.3 and 13.9; 300^3 128 and 128, two steps 123 and 141).  FP32 keeps its
 # streaming tiles where they fill the chip: at 512^3 they move 4.7 TB/s and the waves' unaligned
