@@ -59,13 +59,14 @@ typedef struct pr_fold {
 /* Where a launch stands in a run of calls of one kernel (pr_run, pr_run_graph).  Only what
  * the last call leaves behind can be seen, so
  *   - a kernel with a form that makes several calls in one launch (Setup.fused) asks for it:
- *     its launcher returns 1, with the kernel in `use` and its number of calls in `done`,
+ *     its launcher returns 1, with the kernel in `use`,
  *   - a kernel none of whose launches reads a scalar it stores leaves its reductions and
  *     scalar stores to the last call of the run, which repeats the scalar stores that count
  *     calls (`pending` of them before its own). */
 typedef struct pr_run_state {
   int left;                /* calls still to make, this one included */
-  int use, done;           /* set by a launcher that returns 1 */
+  int use, times, done;    /* set by a launcher that returns 1: `times` launches of kernel `use`
+                              make `done` calls */
   int pending;             /* launches whose finish is still to come */
 } pr_run_state;
 

@@ -179,9 +179,13 @@ int launch_kernel_run(pr_machine* m, int k, int count) {
   for (int c = 0; c < count;) {
     own.left = count - c;
     int rc = launch_kernel_ov(m, k, nullptr, nullptr, &own);
-    if (rc > 0) {   // a kernel that makes own.done calls at once
-      other.left = own.left / own.done;
-      rc = launch_kernel_ov(m, own.use, nullptr, nullptr, &other);
+    if (rc > 0) {   // own.times launches of another kernel make own.done calls
+      rc = PR_OK;
+      const int groups = own.left / own.done;
+      for (int i = 0; i < own.times && rc == PR_OK; ++i) {
+        other.left = groups * own.times - i;
+        rc = launch_kernel_ov(m, own.use, nullptr, nullptr, &other);
+      }
       c += own.done;
     } else {
       ++c;
@@ -655,11 +659,17 @@ int pr_adjoint_forward_seq(pr_machine* m, const int* fwd, int n_fwd, int nsteps,
   const int S = (nsteps + every - 1) / every;
   if ((int)m->snaps.size() < S + every)
     return fail(m, PR_E_INVALID, "pr_snapshot_alloc needs ceil(n/every) + every slots");
-  for (int n = 0; n < nsteps; ++n) {
-    int rc;
-    if (n % every == 0 && (rc = pr_snapshot_save(m, n / every))) return rc;
-    for (int i = 0; i < n_fwd; ++i)
-      if ((rc = launch_kernel_once(m, fwd[i]))) return rc;
+  for (int n = 0; n < nsteps; n += every) {
+    const int steps = nsteps - n < every ? nsteps - n : every;
+    int rc = pr_snapshot_save(m, n / every);
+    if (rc) return rc;
+    if (n_fwd == 1) {   // between two checkpoints only the last step's scalars can be seen
+      if ((rc = launch_kernel_run(m, fwd[0], steps))) return rc;
+      continue;
+    }
+    for (int j = 0; j < steps; ++j)
+      for (int i = 0; i < n_fwd; ++i)
+        if ((rc = launch_kernel_once(m, fwd[i]))) return rc;
   }
   return PR_OK;
 }
@@ -721,6 +731,10 @@ int pr_adjoint_backward_seq(pr_machine* m, const int* fwd, int n_fwd, int tape_a
   }
   int rc;
   if (!needs_state) {
+    if (n_adj == 1) {
+      if ((rc = launch_kernel_run(m, adj[0], nsteps))) return rc;
+      return S > 0 ? pr_snapshot_load(m, 0) : PR_OK;
+    }
     for (int j = 0; j < nsteps; ++j)
       for (int i = 0; i < n_adj; ++i)
         if ((rc = launch_kernel_once(m, adj[i]))) return rc;

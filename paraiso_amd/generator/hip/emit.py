@@ -202,7 +202,7 @@ class MachineEmitter:
                  threads: int = NT, open_axes: Tuple[bool, ...] = (), margins=None,
                  regions=None, march: int = 0, prefetch: bool = True, persist: bool = False,
                  forms: Optional[List[dict]] = None, fused=()):
-        """``fused``: (kernel, kernel making n calls of it, n) names (Setup.fused).  ``forms``: per kernel, the launch form overriding the machine's (keys ``tile``,
+        """``fused``: as Setup.fused.  ``forms``: per kernel, the launch form overriding the machine's (keys ``tile``,
         ``threads``, ``persist``, ``march``), or None."""
         self.name = name
         self.nt = threads
@@ -240,13 +240,14 @@ class MachineEmitter:
         self.lane = None
         self.tiny = ()
         names = [sch.kernel.name for sch in schedules]
-        self.fused: Dict[int, List[Tuple[int, int]]] = {}       # kernel -> [(n, kernel)]
-        for a, b, n in fused:
+        # kernel -> [(calls, kernel that makes them, its launches, smallest grid in cells)]
+        self.fused: Dict[int, List[Tuple[int, int, int, int]]] = {}
+        for a, b, n, times, cells in fused:
             ka, kb = names.index(a), names.index(b)
             if set(s for s, _ in schedules[ka].kernel.stores) != set(
-                    s for s, _ in schedules[kb].kernel.stores) or n < 2:
-                raise ValueError("%s does not stand for %d calls of %s" % (b, n, a))
-            self.fused.setdefault(ka, []).append((n, kb))
+                    s for s, _ in schedules[kb].kernel.stores) or n < 2 or times < 1:
+                raise ValueError("%s does not stand for calls of %s" % (b, a))
+            self.fused.setdefault(ka, []).append((n, kb, times, cells))
         self._lane_memo: Dict[Tuple[int, int], list] = {}
         self.forms = forms or [None] * len(schedules)
         self.ns = len(statics)
@@ -646,9 +647,11 @@ class MachineEmitter:
         h.append("}")
         h.append("static int launch_%s(const pr_launch_ctx* c) {" % fn)
         if L == 0:
-            for n_, kb in sorted(self.fused.get(ki, ()), reverse=True):
-                h.append("  if (c->run && c->run->left >= %d) { c->run->use = %d; c->run->done = %d; "
-                         "return 1; }" % (n_, kb, n_))
+            for n_, kb, times, cells in sorted(self.fused.get(ki, ()), reverse=True):
+                h.append("  if (c->run && c->run->left >= %d && (long long)c->n[0] * c->n[1] * c->n[2] "
+                         ">= %dLL) {" % (n_, cells))
+                h.append("    c->run->use = %d; c->run->times = %d; c->run->done = %d; return 1; }"
+                         % (kb, times, n_))
         h.append("  Args_%s a; fill_%s(c, a);" % (fn, fn))
         if defer:
             # (a shorter rest of the run goes to this kernel's own fused forms or to itself)

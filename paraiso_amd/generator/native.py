@@ -64,9 +64,10 @@ class Setup:
     # smaller tiles for small single grids, smallest first: ({"below": cells, "tile": ...,
     # "threads": ..., "mat_gain": ...}, ...)
     tiny: Tuple[dict, ...] = ()
-    # ((kernel, kernel that makes n calls of it at once, n), ...), such as those transform.unroll
-    # adds: a run of at least n calls uses them, the largest n first
-    fused: Tuple[Tuple[str, str, int], ...] = ()
+    # ((kernel, other kernel, n, launches, cells), ...): `launches` launches of the other make n
+    # calls of the kernel, on grids of at least that many cells, such as those transform.unroll adds: a run of at least n calls on such a
+    # grid uses them, the largest n first
+    fused: Tuple[Tuple[str, str, int, int, int], ...] = ()
     # per OM kernel, a launch form overriding the above: ((kernel name, {"tile": ...,
     # "threads": ..., "persist": ..., "march": ..., "mat_gain": ..., "join": ...}), ...)
     kernel_forms: Tuple[Tuple[str, dict], ...] = ()

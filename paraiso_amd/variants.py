@@ -89,16 +89,17 @@ def _hydro_adj_staged(real):
     return mk
 
 
-def _wave_adj(ndim, real):
+def _wave_adj(ndim, real, most=2):
     """LinearWave with its adjoint, and both fused two steps per launch (``proceed_x2``,
-    ``proceed_adjoint_x2``; more steps per launch need deeper halos than a streaming tile's
-    LDS holds, and lose to two)."""
+    ``proceed_adjoint_x2``), or up to ``most``."""
     def mk():
         from .adjoint import add_adjoint
         from .schemes.linear_wave import linear_wave_om
         from .transform import unroll
         om = add_adjoint(linear_wave_om(ndim, real), "proceed", ["fieldF", "fieldG"])
-        return unroll(unroll(om, "proceed", 2), "proceed_adjoint", 2)
+        for k in range(2, most + 1):
+            om = unroll(unroll(om, "proceed", k), "proceed_adjoint", k)
+        return om
     return mk
 
 
@@ -147,10 +148,17 @@ LIFE_FORMS = (("proceed", {"lane": dict(BITS, min_cells=1_000_000)}),
               ("proceed_x16", {"lane": BITS}))
 
 # Runs of calls take the kernels that make several at once (transform.unroll).
-FUSED_LIFE = (("proceed", "proceed_x4", 4), ("proceed", "proceed_x8", 8),
-              ("proceed", "proceed_x16", 16), ("proceed_x8", "proceed_x16", 2),
-              ("proceed_x4", "proceed_x16", 4), ("proceed_x4", "proceed_x8", 2))
-FUSED_WAVE = (("proceed", "proceed_x2", 2), ("proceed_adjoint", "proceed_adjoint_x2", 2))
+FUSED_LIFE = (("proceed", "proceed_x4", 4, 1, 0), ("proceed", "proceed_x8", 8, 1, 0),
+              ("proceed", "proceed_x16", 16, 1, 0), ("proceed_x8", "proceed_x16", 2, 1, 0),
+              ("proceed_x4", "proceed_x16", 4, 1, 0), ("proceed_x4", "proceed_x8", 2, 1, 0))
+FUSED_WAVE = (("proceed", "proceed_x2", 2, 1, 0), ("proceed_adjoint", "proceed_adjoint_x2", 2, 1, 0))
+# Three steps a launch pay where memory bounds: 512^3 212 us a step (two: 262), 192^3 17 (16).
+LARGE = 20_000_000
+FUSED_WAVE_F32 = FUSED_WAVE + tuple(
+    (k + x, k + "_x3", n, times, LARGE) for k in ("proceed", "proceed_adjoint")
+    for x, n, times in (("", 3, 1), ("_x2", 3, 2)))
+THREE = {"lane": {"rows": 8, "waves": 4, "occupancy": 2, "steps": 4, "fill": 2}}
+WAVE_FORMS = (("proceed_x3", THREE), ("proceed_adjoint_x3", THREE))
 
 # name -> (OM factory, setup, precise)
 VARIANTS = {
@@ -201,8 +209,9 @@ VARIANTS = {
                                   kernel_forms=(("proceed_stage1_adjoint", {"join": True}),
                                                 ("proceed_stage2_adjoint", {"join": True}))),
                             True),
-    "wave3d_f32": (_wave_adj(3, CType.Float), Setup((64, 64, 64), Language.HIP, boundary=CYC3,
-                                                    lane=LANE_WAVE_F32, fused=FUSED_WAVE), False),
+    "wave3d_f32": (_wave_adj(3, CType.Float, 3), Setup((64, 64, 64), Language.HIP, boundary=CYC3,
+                                                    lane=LANE_WAVE_F32, fused=FUSED_WAVE_F32,
+                                                    kernel_forms=WAVE_FORMS), False),
     "wave3d_f64": (_wave_adj(3, CType.Double), Setup((64, 64, 64), Language.HIP, boundary=CYC3,
                                                      lane=LANE_WAVE_F64, fused=FUSED_WAVE), True),
     # streaming along the last axis (rings of planes in LDS), checked bit for bit
