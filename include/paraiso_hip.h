@@ -68,6 +68,14 @@ typedef struct pr_run_state {
   int use, times, done;    /* set by a launcher that returns 1: `times` launches of kernel `use`
                               make `done` calls */
   int pending;             /* launches whose finish is still to come */
+  /* A kernel whose arrays need the last call's reductions (a CFL step carried from call to
+   * call) folds that call's partials at its start instead of waiting for a finish kernel.
+   * `turn` calls of the run have gone so; scalars and partials alternate between the
+   * machine's own space and scal2 and part2, as a launch reads one while it writes the other,
+   * and the run's last finish leaves the scalars in the machine's own. */
+  int turn;
+  char *scal2, *part2;
+  pr_fold prev;            /* partials of the previous call */
 } pr_run_state;
 
 /* What a generated launch callback receives (one kernel launch of one OM kernel). */

@@ -57,6 +57,7 @@ struct pr_machine {
   char* scal = nullptr;
   size_t scal_bytes = 0;
   char* part = nullptr;
+  size_t part_bytes = 0;            // of one of the two sets of partials (pr_run_state)
   std::vector<std::vector<size_t>> part_off;    // [kernel][launch]
   std::vector<std::vector<unsigned>> ntiles;    // [kernel][launch]
   std::vector<std::vector<std::array<int, 3>>> tiles;
@@ -151,6 +152,10 @@ int launch_kernel_ov(pr_machine* m, int k, const void* const* cur_ov, void* cons
     ctx.ntiles = m->ntiles[k][l];
     ctx.stream = m->stream;
     ctx.run = run;
+    if (run) {
+      run->scal2 = m->scal + m->scal_bytes;
+      run->part2 = m->part + m->part_bytes + m->part_off[k][l];
+    }
     ctx.fold = &fold;
     hipEvent_t* ev = m->timing ? m->timing + 2 * ((size_t)m->timing_call * m->timing_stride + l)
                                : nullptr;
@@ -281,9 +286,10 @@ int pr_create(const pr_machine_desc* d, const int* local_size, pr_machine** out)
       }
     }
   }
-  e = hipMalloc(&m->scal, m->scal_bytes);
-  if (e == hipSuccess) e = hipMemsetAsync(m->scal, 0, m->scal_bytes, m->stream);
-  if (e == hipSuccess) e = hipMalloc(&m->part, part_bytes > 0 ? part_bytes : 256);
+  m->part_bytes = part_bytes > 0 ? part_bytes : 256;
+  e = hipMalloc(&m->scal, 2 * m->scal_bytes);
+  if (e == hipSuccess) e = hipMemsetAsync(m->scal, 0, 2 * m->scal_bytes, m->stream);
+  if (e == hipSuccess) e = hipMalloc(&m->part, 2 * m->part_bytes);
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
   if (e != hipSuccess) {
     pr_destroy(m);

@@ -360,6 +360,12 @@ class MachineEmitter:
         fold = first if folds and L == 1 else None
         if fold:
             fields += ["const char* fpart;", "unsigned fstride, fn;"]
+        # a kernel whose next call needs this call's reductions folds them there (pr_run_state)
+        chain = (len(sch.launches) == 1 and bool(la.targets) and bool(la.reduces)
+                 and bool(sch.scalar_stores) and not self._defers(sch))
+        fields.append("char* scal_out;   /* where scalar stores go */")
+        if chain:
+            fields += ["const char* cpart;", "unsigned cstride, cn;   /* the last call's partials */"]
         # a launch without reductions stores its scalars itself (no workgroup reads them)
         inline = (bool(la.targets) and not la.reduces and la.commit and bool(sch.scalar_stores)
                   and not self._reads_stored(sch, la.targets))
@@ -382,6 +388,8 @@ class MachineEmitter:
             """Uniform scalars; ``folding``: those of the previous launch's finish from its
             partials (for an ``nt``-thread workgroup), else from their slots."""
             out = []
+            if chain and folding:
+                return chain_lines(nt)
             fk = fold.kernel_override or sch.kernel if fold else None
             if fold and folding:
                 for j, r in enumerate(fold.reduces):
@@ -407,15 +415,65 @@ class MachineEmitter:
                     out.append("  const %s u%d = %s;" % (tn, n.id, slot))
             return out
 
+        def chain_lines(nt):
+            """Uniform scalars of a call that first finishes the one before it (a.cn partials):
+            p<n> are the finish's scalars, as the finish kernel computes them, u<n> the call's."""
+            out = []
+            stored = {s_: v for s_, v in sch.scalar_stores}
+            scalars = [n for n in nodes if n.realm is Realm.Scalar]
+            expr = lambda n: re.sub(r"\bu(\d+)\b", r"p\1", self.scalar_expr(k, n.id))
+            for n in scalars:
+                if sch.level[n.id] == 0:
+                    e = expr(n)
+                    out.append("  const %s p%d = %s;" % (
+                        n.ctype.c_name, n.id,
+                        "om_uniform((%s)(%s))" % (n.ctype.c_name, e) if n.op == "arith" else e))
+            for j, r in enumerate(la.reduces):
+                at = acc_type(nodes[r].payload, nodes[nodes[r].args[0]].ctype)
+                init, op = (g(nodes[r].payload, at) for g in (acc_init, acc_op))
+                out.append("  const %s fr%d = a.cn ? om_partials_reduce<%d>((const %s*)a.cpart + %d * a.cstride, "
+                           "(int)a.cn, (%s)%s, %s, om_fold_%s) : (%s)%s;" % (
+                               at.c_name, r, nt, at.c_name, j, at.c_name, init, op, at.c_name,
+                               at.c_name, init))
+            out.append("  if (a.cn) __syncthreads();")
+            for v in la.tail_scalars:
+                n = nodes[v]
+                e = "fr%d" % v if n.op == "reduce" else expr(n)
+                out.append("  const %s p%d = om_uniform((%s)(%s));" % ((n.ctype.c_name, v) + (n.ctype.c_name, e)))
+            for n in scalars:
+                if sch.level[n.id] == 0:
+                    if n.op == "load" and n.payload in stored:
+                        e = "a.cn ? p%d : p%d" % (stored[n.payload], n.id)
+                    else:
+                        e = "p%d" % n.id if n.op == "load" else self.scalar_expr(k, n.id)
+                    out.append("  const %s u%d = %s;" % (n.ctype.c_name, n.id, e))
+            return out
+
+        def chain_stores(first_thread):
+            """The scalars the next call and the last finish read, by one thread."""
+            if not chain:
+                return []
+            out = ["  if (a.cn && %s) {" % first_thread]
+            seen = set()
+            for n in nodes:
+                if n.realm is Realm.Scalar and n.op == "load":
+                    seen.add(n.payload)
+                    out.append("    *(%s*)(a.scal_out + %d) = u%d;" % (n.ctype.c_name, 8 * n.payload, n.id))
+            for s_, v in sch.scalar_stores:
+                if s_ not in seen:
+                    out.append("    *(%s*)(a.scal_out + %d) = p%d;" % (nodes[v].ctype.c_name, 8 * s_, v))
+            return out + ["  }"]
+
         def fold_scratch(nt, smem=0):
             """Scratch of the fold: the LDS tiles' own space where there is enough (nothing is in
             it yet), so that tiles that fill the CU's LDS leave room."""
             fk = fold.kernel_override or sch.kernel if fold else None
             return [("  %s* const om_fold_%s = (%s*)smem;" % ((at.c_name,) * 3) if smem >= nt // 8
                      else "  __shared__ %s om_fold_%s[%d];" % (at.c_name, at.c_name, nt // 64))
-                    for at in sorted(set(acc_type(fk.nodes[r].payload,
-                                                  fk.nodes[fk.nodes[r].args[0]].ctype)
-                                         for r in fold.reduces), key=lambda c: c.value)] if fold else []
+                    for at in (sorted(set(acc_type(fk.nodes[r].payload,
+                                                   fk.nodes[fk.nodes[r].args[0]].ctype)
+                                          for r in fold.reduces), key=lambda c: c.value) if fold
+                               else sorted(acc_types, key=lambda c: c.value) if chain else ())]
 
         def own_scalars(first_thread):
             """The scalar stores of a launch that makes them itself, by one thread."""
@@ -469,11 +527,13 @@ class MachineEmitter:
                 out += uniform_lines(self.nt, True) + views + self._persistent_loop(k, la_x)
                 out += epilogue("blockIdx.x")
                 out += own_scalars("blockIdx.x == 0 && threadIdx.x == 0")
+                out += chain_stores("blockIdx.x == 0 && threadIdx.x == 0")
             else:
                 out.append("  unsigned tile = blockIdx.x;")
                 out.append("  if ((a.ntiles & 7u) == 0u) tile = (tile & 7u) * (a.ntiles >> 3) + (tile >> 3);")
                 out += coords + uniform_lines(self.nt, True) + views + work + epilogue("tile")
                 out += own_scalars("tile == 0 && threadIdx.x == 0")
+                out += chain_stores("tile == 0 && threadIdx.x == 0")
             out.append("}")
             if batched:
                 # the tiles of many grids in one launch (grid table in device memory)
@@ -500,7 +560,10 @@ class MachineEmitter:
                         continue
                     lvl = sch.level[n.id]
                     if lvl == 0:
-                        f(ind + "const %s u%d = %s;" % (n.ctype.c_name, n.id, self.scalar_expr(k, n.id)))
+                        e = self.scalar_expr(k, n.id)
+                        if chain and n.op == "arith":     # rounded as chain_lines does
+                            e = "om_uniform((%s)(%s))" % (n.ctype.c_name, e)
+                        f(ind + "const %s u%d = %s;" % (n.ctype.c_name, n.id, e))
                     elif lvl <= L:
                         f(ind + "const %s u%d = *(const %s*)(a.scal + %d);" % (
                             n.ctype.c_name, n.id, n.ctype.c_name, self.slot_off(ki, n.id)))
@@ -527,7 +590,7 @@ class MachineEmitter:
                 f("    *(%s*)(a.scal + %d) = u%d;" % (n.ctype.c_name, self.slot_off(ki, v), v))
             if la.commit:
                 for s_, v in sch.scalar_stores:
-                    f("    *(%s*)(a.scal + %d) = u%d;" % (nodes[v].ctype.c_name, 8 * s_, v))
+                    f("    *(%s*)(a.scal_out + %d) = u%d;" % (nodes[v].ctype.c_name, 8 * s_, v))
             if defer:
                 f("  }")
             f("  }")
@@ -536,7 +599,7 @@ class MachineEmitter:
         if lane:
             for form, plan, name in lanes:
                 ks.extend(self._lane_kernel(ki, k, la, form, plan, fn, name, uniform_lines,
-                                            fold_scratch, own_scalars))
+                                            fold_scratch, own_scalars, chain_stores))
         persist = has_work and self.persist
         if block:
             ks += tile_kernel(fn, la, self.batched)
@@ -578,7 +641,9 @@ class MachineEmitter:
         for s in stores:
             src = "cur" if self.is_scratch(s) else "next"
             h.append("  a.st%d = (%s*)c->%s[%d];" % (s, self.statics[s].dyn.ctype.c_name, src, s))
-        h.append("  a.scal = c->scal; a.part = c->part; a.counter = c->counter;")
+        h.append("  a.scal = a.scal_out = c->scal; a.part = c->part; a.counter = c->counter;")
+        if chain:
+            h.append("  a.cpart = nullptr; a.cstride = a.cn = 0;")
         h.append("  a.n0 = c->n[0]; a.n1 = c->n[1]; a.n2 = c->n[2];")
         if self._own_tiles(lane):
             for ax in range(3):
@@ -661,6 +726,15 @@ class MachineEmitter:
             h.append("    else { a.repeat = c->run->pending + 1; c->run->pending = 0; }")
             h.append("  }")
             h.append("  (void)finish;")
+        if chain:
+            h += ["  pr_run_state* const r = c->run;",
+                  "  char* const scal[2] = {c->scal, r ? r->scal2 : c->scal};",
+                  "  const int turn = r ? r->turn : 0;",
+                  "  if (turn) {",
+                  "    a.cpart = r->prev.part; a.cstride = r->prev.stride; a.cn = r->prev.n;",
+                  "    a.scal = scal[(turn - 1) & 1]; a.scal_out = scal[turn & 1];",
+                  "    if (turn & 1) a.part = r->part2;",
+                  "  }"]
         if lane:
             wg = self.lane["waves"]
             h.append("  if (a.ln) {")
@@ -675,6 +749,14 @@ class MachineEmitter:
         if has_work and block:
             h.append("  hipLaunchKernelGGL(%s, dim3(%s), dim3(%d), 0, (hipStream_t)c->stream, a);"
                      % (fn, "a.nwg" if persist else "a.ntiles", self.nt))
+        if chain:
+            # up to 2048 partials (16 KB) every workgroup of the next call folds them
+            h += ["  if (r && r->left > 1 && a.nwg <= 2048u) {",
+                  "    r->prev.part = a.part; r->prev.stride = a.ntiles; r->prev.n = a.nwg; ++r->turn;",
+                  "    return hipPeekAtLastError() == hipSuccess ? 0 : -1;",
+                  "  }",
+                  "  a.scal = scal[turn & 1]; a.scal_out = c->scal;",
+                  "  if (r) r->turn = 0;"]
         if needs_tail:
             cond = "if (finish) " if defer else ""
             if folds and L == 0:
@@ -757,7 +839,7 @@ class MachineEmitter:
         return ([plan.width, steps, 1] if self.ndim == 2 else [plan.width, plan.rows, steps])
 
     def _lane_kernel(self, ki, k, la, f, plan, fn, name, uniform_lines, fold_scratch,
-                     own_scalars) -> List[str]:
+                     own_scalars, chain_stores) -> List[str]:
         bits = plan if f.get("bits") else None
         plan = bits.lane if bits else plan
         width = bits.width if bits else plan.width
@@ -866,7 +948,8 @@ class MachineEmitter:
         out += scr + fold_scratch(64 * wg) + wave + ["  const unsigned tile = wv;"] + where
         out += ["  const int steps = a.lc;"] + uniform_lines(64 * wg, True) + pre
         out += ["  if (wv < a.ln) {"] + core + ["  }"] + epilogue("b_", False)
-        out += own_scalars("b_ == 0 && threadIdx.x == 0") + ["}"]
+        out += own_scalars("b_ == 0 && threadIdx.x == 0")
+        out += chain_stores("b_ == 0 && threadIdx.x == 0") + ["}"]
         if self.batched and f.get("always"):
             # a tile of the batch is a wave's; `split`: a workgroup's, each wave taking its
             # share of the steps, where the batch has too few tiles to fill the chip
