@@ -106,6 +106,7 @@ typedef struct pr_batch_ctx {
   unsigned total_tiles;
   int n_grids;
   void* stream;
+  int far_rows;            /* some grid's rows hold 2^29 cells or more */
 } pr_batch_ctx;
 
 typedef void (*pr_pack_fn)(const pr_launch_ctx* ctx, void* out);
@@ -259,7 +260,7 @@ int pr_adjoint_backward_seq(pr_machine* m, const int* fwd, int n_fwd, int tape_a
  * a kernel and grid that need more are rejected with PR_E_INVALID before any work is
  * issued.  Calls on one GPU share that array: calls that overlap on one GPU (other
  * streams, other host threads) race and must be serialised by the caller. */
-#define PR_NOALLOC_SCRATCH_BYTES (32u << 20)
+#define PR_NOALLOC_SCRATCH_BYTES (65u << 20)
 int pr_run_noalloc(const pr_machine_desc* desc, const int* local_size, int k, int count,
                    void* const* buffers, int* parity, void* scalars, void* stream,
                    char* err, size_t err_len);

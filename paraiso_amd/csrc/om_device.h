@@ -7,6 +7,8 @@
 //   * om_max/om_min  exactly std::max/std::min (the reference's CPU Max/Min,
 //                    Generator/PlanTrans.hs:690-691): ties and NaNs resolve as there,
 //   * om_resident_workgroups  grid size of a persistent (tile-looping) launch,
+//   * om_lane*, om_at/om_put, om_turn  register streaming: a neighbour lane's value, a
+//                    row's element at a scalar address, 64 cells as a row of bits,
 //   * om_block_*     wave64 shuffle tree + LDS combine for Reduce: each
 //                    workgroup writes one partial, and a one-workgroup finish
 //                    kernel folds the partials in a fixed order, replacing the
@@ -16,9 +18,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-// Workgroups a persistent launch starts: as many as the device holds at once (per_cu per
-// CU, from the launch's LDS and work-items), a multiple of 8 so that workgroup b, which the
-// dispatcher places on XCD b % 8, keeps to that XCD's band of tiles; at most ntiles.
+// CUs of the current device.
 static inline int om_cus() {
   static int cus = 0;
   if (cus <= 0) {
@@ -31,6 +31,9 @@ static inline int om_cus() {
   return cus;
 }
 
+// Workgroups a persistent launch starts: as many as the device holds at once (per_cu per
+// CU, from the launch's LDS and work-items), a multiple of 8 so that workgroup b, which the
+// dispatcher places on XCD b % 8, keeps to that XCD's band of tiles; at most ntiles.
 static inline unsigned om_resident_workgroups(unsigned ntiles, int per_cu) {
   unsigned n = ((unsigned)om_cus() * (unsigned)(per_cu > 0 ? per_cu : 1)) & ~7u;
   if (n == 0) n = 8;
@@ -128,14 +131,16 @@ template <int D> __device__ __forceinline__ double om_lane(double v) {
 }
 
 // Element x of the row at a scalar address: the address stays in scalar registers and the
-// lane adds a 32-bit byte offset (a row has fewer than 2^31 cells of at most 8 bytes; rows
-// of 2^29 cells or more, whose byte offset does not fit, do not take this form).
+// lane adds a 32-bit byte offset.  Rows of 2^29 cells or more, whose byte offset may not fit,
+// take the tile form, or om_far_at where a kernel has no tile form.
 template <class T> __device__ __forceinline__ T om_at(const T* row, int x) {
   return *(const T*)((const char*)row + (unsigned)x * (unsigned)sizeof(T));
 }
 template <class T> __device__ __forceinline__ void om_put(T* row, int x, T v) {
   *(T*)((char*)row + (unsigned)x * (unsigned)sizeof(T)) = v;
 }
+template <class T> __device__ __forceinline__ T om_far_at(const T* row, int x) { return row[x]; }
+template <class T> __device__ __forceinline__ void om_far_put(T* row, int x, T v) { row[x] = v; }
 
 // Lane r's two words become the 64-bit mask: row r of a square of bits (r is a constant after
 // unrolling; the masks are scalar).

@@ -917,6 +917,8 @@ int batch_once(pr_batch* b, int k, double* launch_ms, std::vector<hipEvent_t>* e
     bc.total_tiles = b->total[k][l];
     bc.n_grids = (int)b->grids.size();
     bc.stream = b->stream;
+    bc.far_rows = 0;
+    for (const pr_machine* m : b->grids) bc.far_rows |= m->n[0] >= (1 << 29);
     if (ev) (void)hipEventRecord((*ev)[2 * l], b->stream);
     if (kd.launches[l].batched(&bc) != 0)
       return bfail(b, PR_E_HIP, std::string("batched launch: ") + hipGetErrorString(hipGetLastError()));
@@ -947,8 +949,7 @@ int pr_batch_create(const pr_machine_desc* d, int n_grids, const int* sizes, pr_
   }
   for (int g = 0; g < n_grids; ++g) {
     pr_machine* m = nullptr;
-    // batched launches address a row with 32-bit byte offsets
-    int rc = sizes[3 * g] < (1 << 29) ? pr_create(d, sizes + 3 * g, &m) : PR_E_INVALID;
+    int rc = pr_create(d, sizes + 3 * g, &m);
     if (rc == PR_OK) rc = pr_set_stream(m, b->stream);
     if (rc) {
       b->err = "grid " + std::to_string(g) + ": " + (m ? m->err : std::string("pr_create"));

@@ -700,10 +700,11 @@ class MachineEmitter:
             else:
                 # below two waves per SIMD a tile is split over a workgroup
                 h.append("  const int split = bc->total_tiles < 8u * (unsigned)om_cus();")
-                h.append("  hipLaunchKernelGGL(%s_batched, dim3(split ? bc->total_tiles : "
+                h.append("  hipLaunchKernelGGL((bc->far_rows ? %s_far_batched : %s_batched), "
+                         "dim3(split ? bc->total_tiles : "
                          "(bc->total_tiles + %du) / %du), dim3(%d), 0, (hipStream_t)bc->stream, "
                          "(const Args_%s*)bc->args, bc->tile_grid, bc->tile_base, bc->total_tiles, split);"
-                         % (fn, wg - 1, wg, 64 * wg, fn))
+                         % (fn, fn, wg - 1, wg, 64 * wg, fn))
         if needs_tail and self.batched:
             h.append("  hipLaunchKernelGGL(%s_fin_batched, dim3(bc->n_grids), dim3(%d), 0, (hipStream_t)bc->stream, "
                      "(const Args_%s*)bc->args);" % (fn, self.nt, fn))
@@ -740,8 +741,9 @@ class MachineEmitter:
             h.append("  if (a.ln) {")
             h.append("  a.nwg = (a.ln + %du) / %du;" % (wg - 1, wg))
             for i, (_, _, name) in enumerate(lanes):
+                form = name if block else "(a.n0 < (1 << 29) ? %s : %s_far)" % (name, name)
                 h.append("  %sif (a.lv == %d) hipLaunchKernelGGL(%s, dim3(a.nwg), dim3(%d), 0, "
-                         "(hipStream_t)c->stream, a);" % ("else " if i else "", i, name, 64 * wg))
+                         "(hipStream_t)c->stream, a);" % ("else " if i else "", i, form, 64 * wg))
             h.append("  }" + (" else" if block else ""))
         for i, (_, name, _, nt_, _) in enumerate(small):
             h.append("  if (a.bv == %d) hipLaunchKernelGGL(%s, dim3(a.ntiles), dim3(%d), 0, "
@@ -971,6 +973,12 @@ class MachineEmitter:
                 out += (["  if (split) {"] + epilogue("tile", False) + ["  } else {"]
                         + epilogue("tile", True) + ["  }"])
             out += own_scalars("tile == 0 && lane == 0 && (!split || w_ == 0)") + ["}"]
+        if f.get("always"):
+            # no tile form takes the rows whose byte offsets pass 32 bits: the same kernels with
+            # 64-bit lane offsets do
+            out += [re.sub(r"\bom_(at|put)\(", r"om_far_\1(", ln)
+                    .replace(" %s(Args_" % name, " %s_far(Args_" % name)
+                    .replace(" %s_batched(" % fn, " %s_far_batched(" % fn) for ln in out]
         return out
 
     def _bit_square(self, bits, la, em, stores, reduces, stream) -> List[str]:

@@ -56,6 +56,30 @@ def test_hydro_on_both_sides_of_the_rule(require_gpu):
         same(a, b)
 
 
+@pytest.mark.parametrize("batch", [False, True])
+def test_hydro_rows_past_32_bit_offsets(require_gpu, batch):
+    """A row of 2^29 cells or more takes the kernels with 64-bit lane offsets: one row of a
+    repeated pattern (its period divides the row), against the small grid of one period."""
+    period, times = 8191, 65545
+    nx = period * times
+    print("hydro lane far rows %d" % nx, flush=True)
+    b = variants.batch("hydro_f64_lane", [(nx, 1)]) if batch else None
+    m = b.grids[0] if batch else variants.machine("hydro_f64_lane", (nx, 1))
+    one = variants.machine("hydro_f64", (period, 1))
+    for k, v in inputs.hydro_scalars(period, 1).items():
+        m.set(k, v)
+        one.set(k, v)
+    for f, a in zip(F, hydro_state(period, 1, 9)):
+        one.set(f, a)
+        m.set(f, np.tile(a.reshape(1, -1), (1, times)))
+    (b or m).run("proceed")
+    one.run("proceed")
+    for f in F:
+        got = m.get(f).reshape(times, period)
+        assert (got == one.get(f).reshape(1, -1)).all(), f
+        print("same", f, flush=True)
+
+
 @pytest.mark.parametrize("count,lo,hi", [(5, 5, 90), (9, 64, 700)])
 def test_hydro_batch(require_gpu, count, lo, hi):
     """Few tiles are split over a workgroup's waves, many are a wave's each."""
