@@ -66,7 +66,9 @@ typedef struct pr_fold {
 typedef struct pr_run_state {
   int left;                /* calls still to make, this one included */
   int use, times, done;    /* set by a launcher that returns 1: `times` launches of kernel `use`
-                              make `done` calls */
+                              make `done` calls; by one that returns 2, after a launch that left
+                              its partials in `prev`: kernel `use` makes every call still to make,
+                              the first of them from these partials */
   int pending;             /* launches whose finish is still to come */
   /* A kernel whose arrays need the last call's reductions (a CFL step carried from call to
    * call) folds that call's partials at its start instead of waiting for a finish kernel.
@@ -74,7 +76,9 @@ typedef struct pr_run_state {
    * machine's own space and scal2 and part2, as a launch reads one while it writes the other,
    * and the run's last finish leaves the scalars in the machine's own. */
   int turn;
-  char *scal2, *part2;
+  char *scal2, *scal3, *part2;
+  int keep;                /* calls made for another kernel: what this one carries stays as it
+                              was (scal3 stands in for the machine's own space) */
   pr_fold prev;            /* partials of the previous call */
 } pr_run_state;
 

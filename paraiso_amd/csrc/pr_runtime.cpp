@@ -154,6 +154,7 @@ int launch_kernel_ov(pr_machine* m, int k, const void* const* cur_ov, void* cons
     ctx.run = run;
     if (run) {
       run->scal2 = m->scal + m->scal_bytes;
+      run->scal3 = m->scal + 2 * m->scal_bytes;
       run->part2 = m->part + m->part_bytes + m->part_off[k][l];
     }
     ctx.fold = &fold;
@@ -184,7 +185,16 @@ int launch_kernel_run(pr_machine* m, int k, int count) {
   for (int c = 0; c < count;) {
     own.left = count - c;
     int rc = launch_kernel_ov(m, k, nullptr, nullptr, &own);
-    if (rc > 0) {   // own.times launches of another kernel make own.done calls
+    if (rc == 2) {   // another kernel makes the rest of the calls, from own.prev's partials
+      other = {};
+      other.turn = other.keep = 1;
+      other.prev = own.prev;
+      rc = PR_OK;
+      for (; c < count && rc == PR_OK; ++c) {
+        other.left = count - c;
+        rc = launch_kernel_ov(m, own.use, nullptr, nullptr, &other);
+      }
+    } else if (rc > 0) {   // own.times launches of another kernel make own.done calls
       rc = PR_OK;
       const int groups = own.left / own.done;
       for (int i = 0; i < own.times && rc == PR_OK; ++i) {
@@ -287,8 +297,8 @@ int pr_create(const pr_machine_desc* d, const int* local_size, pr_machine** out)
     }
   }
   m->part_bytes = part_bytes > 0 ? part_bytes : 256;
-  e = hipMalloc(&m->scal, 2 * m->scal_bytes);
-  if (e == hipSuccess) e = hipMemsetAsync(m->scal, 0, 2 * m->scal_bytes, m->stream);
+  e = hipMalloc(&m->scal, 3 * m->scal_bytes);
+  if (e == hipSuccess) e = hipMemsetAsync(m->scal, 0, 3 * m->scal_bytes, m->stream);
   if (e == hipSuccess) e = hipMalloc(&m->part, 2 * m->part_bytes);
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
   if (e != hipSuccess) {

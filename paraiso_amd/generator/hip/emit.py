@@ -20,6 +20,14 @@ from the hand-written templates in ``csrc/om_device.h``:
    ``om_broadcast``, ``PlanTrans.hs:566-569``) and, in the kernel's last launch,
    commits the scalar stores.  Stream order replaces a device-wide fence per
    workgroup, which on a multi-XCD part would write back L2 thousands of times.
+   Where nothing else waits for it the finish is left out: the next launch folds
+   the partials itself (the second of a kernel's two launches, the next call of a
+   run), a launch without reductions stores the scalars, a run finishes once.
+
+A kernel may have more forms than that one: small tiles for small grids
+(``Setup.tiny``), register streaming (``lane.py``: a wave's lanes hold a strip's
+columns and walk along the last axis, no LDS and no barrier) and bit planes
+(``bits.py``: Life's cells as bits).  The launcher picks one from the grid's size.
 
 Per-point expressions follow the reference's SASA naming (``a<node>_<cursor>``,
 ``PlanTrans.hs:625-644``) as ``n<value>_<cursor>``.
@@ -365,7 +373,9 @@ class MachineEmitter:
                  and bool(sch.scalar_stores) and not self._defers(sch))
         fields.append("char* scal_out;   /* where scalar stores go */")
         if chain:
-            fields += ["const char* cpart;", "unsigned cstride, cn;   /* the last call's partials */"]
+            fields += ["const char* cpart;", "unsigned cstride, cn;   /* the last call's partials */",
+                       "int cfirst;   /* they are another kernel's, which stored no scalar */",
+                       "int keep;   /* the finish leaves the carried scalars as they are */"]
         # a launch without reductions stores its scalars itself (no workgroup reads them)
         inline = (bool(la.targets) and not la.reduces and la.commit and bool(sch.scalar_stores)
                   and not self._reads_stored(sch, la.targets))
@@ -443,7 +453,8 @@ class MachineEmitter:
             for n in scalars:
                 if sch.level[n.id] == 0:
                     if n.op == "load" and n.payload in stored:
-                        e = "a.cn ? p%d : p%d" % (stored[n.payload], n.id)
+                        e = "a.cn%s ? p%d : p%d" % ("" if self.carried(n.payload) else " && !a.cfirst",
+                                                    stored[n.payload], n.id)
                     else:
                         e = "p%d" % n.id if n.op == "load" else self.scalar_expr(k, n.id)
                     out.append("  const %s u%d = %s;" % (n.ctype.c_name, n.id, e))
@@ -590,7 +601,9 @@ class MachineEmitter:
                 f("    *(%s*)(a.scal + %d) = u%d;" % (n.ctype.c_name, self.slot_off(ki, v), v))
             if la.commit:
                 for s_, v in sch.scalar_stores:
-                    f("    *(%s*)(a.scal_out + %d) = u%d;" % (nodes[v].ctype.c_name, 8 * s_, v))
+                    f("    %s*(%s*)(a.scal_out + %d) = u%d;" % (
+                        "if (!a.keep) " if chain and self.carried(s_) else "",
+                        nodes[v].ctype.c_name, 8 * s_, v))
             if defer:
                 f("  }")
             f("  }")
@@ -643,7 +656,7 @@ class MachineEmitter:
             h.append("  a.st%d = (%s*)c->%s[%d];" % (s, self.statics[s].dyn.ctype.c_name, src, s))
         h.append("  a.scal = a.scal_out = c->scal; a.part = c->part; a.counter = c->counter;")
         if chain:
-            h.append("  a.cpart = nullptr; a.cstride = a.cn = 0;")
+            h.append("  a.cpart = nullptr; a.cstride = a.cn = 0; a.cfirst = a.keep = 0;")
         h.append("  a.n0 = c->n[0]; a.n1 = c->n[1]; a.n2 = c->n[2];")
         if self._own_tiles(lane):
             for ax in range(3):
@@ -729,11 +742,13 @@ class MachineEmitter:
             h.append("  (void)finish;")
         if chain:
             h += ["  pr_run_state* const r = c->run;",
-                  "  char* const scal[2] = {c->scal, r ? r->scal2 : c->scal};",
                   "  const int turn = r ? r->turn : 0;",
+                  "  a.keep = r ? r->keep : 0;",
+                  "  char* const scal[2] = {a.keep ? r->scal3 : c->scal, r ? r->scal2 : c->scal};",
                   "  if (turn) {",
                   "    a.cpart = r->prev.part; a.cstride = r->prev.stride; a.cn = r->prev.n;",
-                  "    a.scal = scal[(turn - 1) & 1]; a.scal_out = scal[turn & 1];",
+                  "    a.scal = turn == 1 ? c->scal : scal[(turn - 1) & 1]; a.scal_out = scal[turn & 1];",
+                  "    a.cfirst = a.keep && turn == 1;",
                   "    if (turn & 1) a.part = r->part2;",
                   "  }"]
         if lane:
@@ -753,11 +768,11 @@ class MachineEmitter:
                      % (fn, "a.nwg" if persist else "a.ntiles", self.nt))
         if chain:
             # up to 2048 partials (16 KB) every workgroup of the next call folds them
-            h += ["  if (r && r->left > 1 && a.nwg <= 2048u) {",
+            h += ["  if (r && r->left > 1 && (a.keep || a.nwg <= 2048u)) {",
                   "    r->prev.part = a.part; r->prev.stride = a.ntiles; r->prev.n = a.nwg; ++r->turn;",
                   "    return hipPeekAtLastError() == hipSuccess ? 0 : -1;",
                   "  }",
-                  "  a.scal = scal[turn & 1]; a.scal_out = c->scal;",
+                  "  a.scal = turn ? scal[turn & 1] : c->scal; a.scal_out = c->scal;",
                   "  if (r) r->turn = 0;"]
         if needs_tail:
             cond = "if (finish) " if defer else ""
@@ -768,9 +783,36 @@ class MachineEmitter:
                 cond = "if (!c->fold || !c->fold->n) "
             h.append("  %shipLaunchKernelGGL(%s_fin, dim3(1), dim3(%d), 0, (hipStream_t)c->stream, a);"
                      % (cond, fn, self.nt))
+            if folds and L == 0 and self.carrier(ki, sch) is not None:
+                # the rest of a run of calls needs one pass a call: the carrying kernel's, which
+                # folds these partials first (hydro_f32, us a step: 18.3 -> 17.2 at 1021x767,
+                # 7.0 -> 4.7 at 96x64)
+                h.append("  if (c->run && c->run->left > 1 && c->fold && c->fold->n) {")
+                h.append("    if (hipPeekAtLastError() != hipSuccess) return -1;")
+                h.append("    c->run->use = %d; c->run->prev = *c->fold; return 2; }"
+                         % self.carrier(ki, sch))
         h.append("  return hipPeekAtLastError() == hipSuccess ? 0 : -1;")
         h.append("}")
         return kernel_src, "\n".join(h) + "\n"
+
+    def carried(self, s) -> bool:
+        """Static s holds a reduction carried from call to call (transform.pipeline_reduce)."""
+        return self.statics[s].name.startswith("__carry_")
+
+    def carrier(self, ki, sch) -> Optional[int]:
+        """The kernel that makes a run of calls of kernel ki, whose first launch only reduces,
+        in one pass a call (transform.pipeline_reduce): it starts from that launch's partials.
+        With one reduction, its place among the partials is the same in both."""
+        names = [x.kernel.name for x in self.schedules]
+        name = names[ki]
+        mine = sum(s.name.startswith("__carry_%s_" % name) for s in self.statics)
+        first = sch.launches[0]
+        if (name + "_pipelined" not in names or mine != 1 or len(first.reduces) != 1
+                or first.stores):
+            return None
+        kp = names.index(name + "_pipelined")
+        one = self.schedules[kp].launches
+        return kp if len(one) == 1 and len(one[0].reduces) == 1 and one[0].targets else None
 
     def _reads_stored(self, sch, roots) -> bool:
         """Some value of ``roots`` depends on a scalar static that the kernel stores."""

@@ -124,9 +124,8 @@ LANE_HYDRO_F64 = {"waves": 4, "occupancy": 2, "steps": 4, "min_cells": 400_000}
 TINY_HYDRO_F32 = ({"below": 60_000, "tile": (16, 8), "threads": 320},)
 TINY_HYDRO_F64 = ({"below": 30_000, "tile": (16, 8), "threads": 320},
                   {"below": 120_000, "tile": (16, 16), "threads": 512})
-# Batches: a tile is 24 steps of one wave, 0.92 -> 0.58 ms a step (32: 0.59; small batches 17.6 us
-# against 18.5) for
-# 256 uneven grids.
+# Batches: a tile is 24 steps of one wave: 256 uneven grids 0.92 ms a step in LDS tiles, 0.58 so
+# (32 steps: 0.59; small batches 18.5 us a step against 17.6).
 LANE_HYDRO_BATCH = {"waves": 4, "occupancy": 2, "steps": 24, "always": True}
 # LinearWave 3-D: a lane holds rows of y, fewer on small grids (64^3: 11.6 us a step with 8, 8.9
 # with 4; 128^3 15.3 and 13.9; 300^3 128 and 128, two steps 123 and 141).  FP32 keeps its

@@ -94,3 +94,38 @@ def test_time_counts_every_call(require_gpu):
         b.run("proceed")
     assert a.get("time") == b.get("time")
     assert np.array_equal(a.get("density"), b.get("density"))
+
+
+@pytest.mark.parametrize("variant,size", [("hydro_f64", (40, 23)), ("hydro_f64", (201, 170)),
+                                          ("hydro_f64", (400, 333)), ("hydro_f64", (701, 633)),
+                                          ("hydro_f64_lane", (117, 65)),
+                                          ("hydro_f32_precise", (130, 67))])
+@pytest.mark.parametrize("count,graph", [(2, False), (3, False), (4, True), (5, True)])
+def test_hydro_calls_in_one_pass(require_gpu, variant, size, count, graph):
+    """A run of ``proceed`` carries its reduction: what single calls leave, and the statics that
+    carry it for ``proceed_pipelined`` stay as they were."""
+    print("hydro run %s %s of %d, graph %s" % (variant, size, count, graph), flush=True)
+    a, b = variants.machine(variant, size), variants.machine(variant, size)
+    names = ("density", "velocity0", "velocity1", "pressure")
+    rng = np.random.default_rng(8)
+    state = [x + 0.05 * rng.standard_normal(x.shape) for x in inputs.kh_init(*size, 6)]
+    dt = np.float32 if "f32" in variant else np.float64
+    for m in (a, b):
+        for k, v in inputs.hydro_scalars(*size).items():
+            m.set(k, v)
+        for f, x in zip(names, state):
+            m.set(f, x.astype(dt))
+        m.run("proceed_prime")
+    for _ in range(2):
+        a.run("proceed", count, graph=graph)
+        for _ in range(count):
+            b.run("proceed")
+        for f in names:
+            assert np.array_equal(a.get(f), b.get(f)), f
+        for s in ("time", "__carry_proceed_0"):
+            assert a.get(s) == b.get(s), s
+    for m in (a, b):
+        m.run("proceed_pipelined", 3)
+    for f in names:
+        assert np.array_equal(a.get(f), b.get(f)), f
+    assert a.get("time") == b.get("time")
