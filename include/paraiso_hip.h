@@ -66,9 +66,9 @@ typedef struct pr_fold {
 typedef struct pr_run_state {
   int left;                /* calls still to make, this one included */
   int use, times, done;    /* set by a launcher that returns 1: `times` launches of kernel `use`
-                              make `done` calls; by one that returns 2, after a launch that left
-                              its partials in `prev`: kernel `use` makes every call still to make,
-                              the first of them from these partials */
+                              make `done` calls; by one that returns 2, after it has left the
+                              scalars that kernel `use` starts from in scal3: `use` makes every
+                              call still to make */
   int pending;             /* launches whose finish is still to come */
   /* A kernel whose arrays need the last call's reductions (a CFL step carried from call to
    * call) folds that call's partials at its start instead of waiting for a finish kernel.

@@ -185,10 +185,9 @@ int launch_kernel_run(pr_machine* m, int k, int count) {
   for (int c = 0; c < count;) {
     own.left = count - c;
     int rc = launch_kernel_ov(m, k, nullptr, nullptr, &own);
-    if (rc == 2) {   // another kernel makes the rest of the calls, from own.prev's partials
+    if (rc == 2) {   // another kernel makes the rest of the calls
       other = {};
-      other.turn = other.keep = 1;
-      other.prev = own.prev;
+      other.keep = 1;
       rc = PR_OK;
       for (; c < count && rc == PR_OK; ++c) {
         other.left = count - c;

@@ -373,9 +373,7 @@ class MachineEmitter:
                  and bool(sch.scalar_stores) and not self._defers(sch))
         fields.append("char* scal_out;   /* where scalar stores go */")
         if chain:
-            fields += ["const char* cpart;", "unsigned cstride, cn;   /* the last call's partials */",
-                       "int cfirst;   /* they are another kernel's, which stored no scalar */",
-                       "int keep;   /* the finish leaves the carried scalars as they are */"]
+            fields += ["const char* cpart;", "unsigned cstride, cn;   /* the last call's partials */"]
         # a launch without reductions stores its scalars itself (no workgroup reads them)
         inline = (bool(la.targets) and not la.reduces and la.commit and bool(sch.scalar_stores)
                   and not self._reads_stored(sch, la.targets))
@@ -385,6 +383,8 @@ class MachineEmitter:
             fields += ["unsigned ln, lx, ly, mx, my;  /* register streaming: waves, strips along "
                        "x and y, reciprocals */", "int lc;  /* steps a wave streams */",
                        "int lv;  /* which of the launch's streaming forms */"]
+        if chain:
+            fields.append("int keep;   /* the finish leaves the carried scalars as they are */")
         struct = "struct Args_%s {\n  %s\n};\n" % (fn, "\n  ".join(fields))
 
         acc_types = set(acc_type(nodes[r].payload, nodes[nodes[r].args[0]].ctype)
@@ -453,8 +453,7 @@ class MachineEmitter:
             for n in scalars:
                 if sch.level[n.id] == 0:
                     if n.op == "load" and n.payload in stored:
-                        e = "a.cn%s ? p%d : p%d" % ("" if self.carried(n.payload) else " && !a.cfirst",
-                                                    stored[n.payload], n.id)
+                        e = "a.cn ? p%d : p%d" % (stored[n.payload], n.id)
                     else:
                         e = "p%d" % n.id if n.op == "load" else self.scalar_expr(k, n.id)
                     out.append("  const %s u%d = %s;" % (n.ctype.c_name, n.id, e))
@@ -643,6 +642,20 @@ class MachineEmitter:
                 ks.append("  const Args_%s a = grids[blockIdx.x];" % fn)
                 ks.append(fcore)
                 ks.append("}")
+        carrier = self.carrier(ki, sch) if folds and L == 0 else None
+        if carrier:
+            # the carrying kernel's scalars: the machine's and, folded, this launch's reduction
+            r = la.reduces[0]
+            ct, at = nodes[r].ctype.c_name, acc_type(nodes[r].payload, nodes[nodes[r].args[0]].ctype)
+            ks += ["extern \"C\" __global__ void __launch_bounds__(%d) %s_carry(Args_%s a) {"
+                   % (self.nt, fn, fn)] + fin_decls + [
+                "  const %s fr = om_partials_reduce<%d>((const %s*)a.part, (int)a.nwg, (%s)%s, %s, om_scr_%s);"
+                % (at.c_name, self.nt, at.c_name, at.c_name, acc_init(nodes[r].payload, at),
+                   acc_op(nodes[r].payload, at), at.c_name),
+                "  for (int i = threadIdx.x; i < %d; i += %d)" % (self.ns, self.nt),
+                "    if (i != %d) ((double*)a.scal_out)[i] = ((const double*)a.scal)[i];" % carrier[1],
+                "  if (threadIdx.x == 0) *(%s*)(a.scal_out + %d) = om_uniform((%s)(fr));"
+                % (ct, 8 * carrier[1], ct), "}"]
         kernel_src = "\n".join(ks) + "\n"
 
         # ---- host launcher
@@ -656,7 +669,7 @@ class MachineEmitter:
             h.append("  a.st%d = (%s*)c->%s[%d];" % (s, self.statics[s].dyn.ctype.c_name, src, s))
         h.append("  a.scal = a.scal_out = c->scal; a.part = c->part; a.counter = c->counter;")
         if chain:
-            h.append("  a.cpart = nullptr; a.cstride = a.cn = 0; a.cfirst = a.keep = 0;")
+            h.append("  a.cpart = nullptr; a.cstride = a.cn = 0; a.keep = 0;")
         h.append("  a.n0 = c->n[0]; a.n1 = c->n[1]; a.n2 = c->n[2];")
         if self._own_tiles(lane):
             for ax in range(3):
@@ -743,12 +756,11 @@ class MachineEmitter:
         if chain:
             h += ["  pr_run_state* const r = c->run;",
                   "  const int turn = r ? r->turn : 0;",
-                  "  a.keep = r ? r->keep : 0;",
-                  "  char* const scal[2] = {a.keep ? r->scal3 : c->scal, r ? r->scal2 : c->scal};",
+                  "  char* const scal[2] = {r && r->keep ? r->scal3 : c->scal, r ? r->scal2 : c->scal};",
+                  "  a.scal = scal[0];",
                   "  if (turn) {",
                   "    a.cpart = r->prev.part; a.cstride = r->prev.stride; a.cn = r->prev.n;",
-                  "    a.scal = turn == 1 ? c->scal : scal[(turn - 1) & 1]; a.scal_out = scal[turn & 1];",
-                  "    a.cfirst = a.keep && turn == 1;",
+                  "    a.scal = scal[(turn - 1) & 1]; a.scal_out = scal[turn & 1];",
                   "    if (turn & 1) a.part = r->part2;",
                   "  }"]
         if lane:
@@ -768,12 +780,23 @@ class MachineEmitter:
                      % (fn, "a.nwg" if persist else "a.ntiles", self.nt))
         if chain:
             # up to 2048 partials (16 KB) every workgroup of the next call folds them
-            h += ["  if (r && r->left > 1 && (a.keep || a.nwg <= 2048u)) {",
+            h += ["  if (r && r->left > 1 && a.nwg <= 2048u) {",
                   "    r->prev.part = a.part; r->prev.stride = a.ntiles; r->prev.n = a.nwg; ++r->turn;",
                   "    return hipPeekAtLastError() == hipSuccess ? 0 : -1;",
                   "  }",
-                  "  a.scal = turn ? scal[turn & 1] : c->scal; a.scal_out = c->scal;",
+                  "  a.scal = scal[turn & 1]; a.scal_out = r && r->left > 1 ? scal[0] : c->scal;",
+                  "  a.keep = r && r->keep && r->left == 1;",
                   "  if (r) r->turn = 0;"]
+        if carrier:
+            # the rest of a run of calls needs one pass a call: the carrying kernel's, after this
+            # one has told it the first reduction (hydro_f32, us a step: 18.4 -> 17.0 at 1021x767,
+            # 7.9 -> 5.1 at 96x64)
+            h += ["  if (c->run && c->run->left > 1) {",
+                  "    a.scal_out = c->run->scal3;",
+                  "    hipLaunchKernelGGL(%s_carry, dim3(1), dim3(%d), 0, (hipStream_t)c->stream, a);"
+                  % (fn, self.nt),
+                  "    c->run->use = %d;" % carrier[0],
+                  "    return hipPeekAtLastError() == hipSuccess ? 2 : -1;", "  }"]
         if needs_tail:
             cond = "if (finish) " if defer else ""
             if folds and L == 0:
@@ -783,14 +806,6 @@ class MachineEmitter:
                 cond = "if (!c->fold || !c->fold->n) "
             h.append("  %shipLaunchKernelGGL(%s_fin, dim3(1), dim3(%d), 0, (hipStream_t)c->stream, a);"
                      % (cond, fn, self.nt))
-            if folds and L == 0 and self.carrier(ki, sch) is not None:
-                # the rest of a run of calls needs one pass a call: the carrying kernel's, which
-                # folds these partials first (hydro_f32, us a step: 18.3 -> 17.2 at 1021x767,
-                # 7.0 -> 4.7 at 96x64)
-                h.append("  if (c->run && c->run->left > 1 && c->fold && c->fold->n) {")
-                h.append("    if (hipPeekAtLastError() != hipSuccess) return -1;")
-                h.append("    c->run->use = %d; c->run->prev = *c->fold; return 2; }"
-                         % self.carrier(ki, sch))
         h.append("  return hipPeekAtLastError() == hipSuccess ? 0 : -1;")
         h.append("}")
         return kernel_src, "\n".join(h) + "\n"
@@ -799,20 +814,21 @@ class MachineEmitter:
         """Static s holds a reduction carried from call to call (transform.pipeline_reduce)."""
         return self.statics[s].name.startswith("__carry_")
 
-    def carrier(self, ki, sch) -> Optional[int]:
+    def carrier(self, ki, sch) -> Optional[Tuple[int, int]]:
         """The kernel that makes a run of calls of kernel ki, whose first launch only reduces,
-        in one pass a call (transform.pipeline_reduce): it starts from that launch's partials.
-        With one reduction, its place among the partials is the same in both."""
+        in one pass a call, and the static that carries the reduction for it
+        (transform.pipeline_reduce; with one reduction there is no question which)."""
         names = [x.kernel.name for x in self.schedules]
         name = names[ki]
-        mine = sum(s.name.startswith("__carry_%s_" % name) for s in self.statics)
+        mine = [s for s, st in enumerate(self.statics) if st.name.startswith("__carry_%s_" % name)]
         first = sch.launches[0]
-        if (name + "_pipelined" not in names or mine != 1 or len(first.reduces) != 1
+        if (name + "_pipelined" not in names or len(mine) != 1 or len(first.reduces) != 1
                 or first.stores):
             return None
         kp = names.index(name + "_pipelined")
         one = self.schedules[kp].launches
-        return kp if len(one) == 1 and len(one[0].reduces) == 1 and one[0].targets else None
+        return ((kp, mine[0]) if len(one) == 1 and len(one[0].reduces) == 1 and one[0].targets
+                else None)
 
     def _reads_stored(self, sch, roots) -> bool:
         """Some value of ``roots`` depends on a scalar static that the kernel stores."""
