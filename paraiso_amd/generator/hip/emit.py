@@ -362,9 +362,11 @@ class MachineEmitter:
         fields.append("int repeat;   /* calls the finish stands for */")
         # the second of two launches folds the first one's partials itself: every workgroup
         # reads them (at most a few KB) where a finish kernel between the two would have cost
-        # a launch
+        # a launch.  A second launch with a finish of its own reads the folded scalars from
+        # their slots there, so the first launch's finish writes them
         first = sch.launches[0]
-        folds = len(sch.launches) == 2 and bool(first.reduces) and bool(first.targets)
+        folds = (len(sch.launches) == 2 and bool(first.reduces) and bool(first.targets)
+                 and bool(sch.launches[1].targets) and not self._finishes(sch, sch.launches[1]))
         fold = first if folds and L == 1 else None
         if fold:
             fields += ["const char* fpart;", "unsigned fstride, fn;"]
@@ -374,9 +376,7 @@ class MachineEmitter:
         fields.append("char* scal_out;   /* where scalar stores go */")
         if chain:
             fields += ["const char* cpart;", "unsigned cstride, cn;   /* the last call's partials */"]
-        # a launch without reductions stores its scalars itself (no workgroup reads them)
-        inline = (bool(la.targets) and not la.reduces and la.commit and bool(sch.scalar_stores)
-                  and not self._reads_stored(sch, la.targets))
+        inline = self._stores_inline(sch, la)
         if self.tiny:
             fields.append("int bv;   /* which of the launch's tiles */")
         if lane:
@@ -496,8 +496,7 @@ class MachineEmitter:
             for s_, v in sch.scalar_stores:
                 out.append("    *(%s*)(a.scal + %d) = u%d;" % (nodes[v].ctype.c_name, 8 * s_, v))
             return out + ["  }"] * (2 if defer else 1)
-        needs_tail = not inline and (bool(la.reduces) or bool(la.tail_scalars)
-                                     or (la.commit and bool(sch.scalar_stores)))
+        needs_tail = self._finishes(sch, la)
         defer = (needs_tail or inline) and self._defers(sch)
         def epilogue(index):
             e = []
@@ -829,6 +828,18 @@ class MachineEmitter:
         one = self.schedules[kp].launches
         return ((kp, mine[0]) if len(one) == 1 and len(one[0].reduces) == 1 and one[0].targets
                 else None)
+
+    def _stores_inline(self, sch, la) -> bool:
+        """The launch has no reductions and stores the kernel's scalars itself: no workgroup
+        reads them."""
+        return (bool(la.targets) and not la.reduces and la.commit and bool(sch.scalar_stores)
+                and not self._reads_stored(sch, la.targets))
+
+    def _finishes(self, sch, la) -> bool:
+        """The launch has a finish kernel: reductions, scalars computed from them, or scalar
+        stores that it does not make itself."""
+        return not self._stores_inline(sch, la) and (
+            bool(la.reduces) or bool(la.tail_scalars) or (la.commit and bool(sch.scalar_stores)))
 
     def _reads_stored(self, sch, roots) -> bool:
         """Some value of ``roots`` depends on a scalar static that the kernel stores."""

@@ -110,6 +110,11 @@ def _optable(real):
     return mk
 
 
+def _monitor():
+    from .schemes.monitor import monitor_om
+    return monitor_om()
+
+
 # Register streaming (generator/hip/lane.py).  Hydro: a wave streams along y; below min_cells
 # the strips are too short for their run-up and the tile form is faster (FP32: 22.6 us a step
 # at 700^2 in tiles, 24.0 streaming; 33.4 and 28.3 at 1021x767; 112 and 91 at 2048^2.  FP64:
@@ -242,6 +247,9 @@ VARIANTS = {
                          False),
     "optable_f64": (_optable(CType.Double), Setup((64, 48), Language.HIP, boundary=CYC2), True),
     "optable_i32": (_optable(CType.Int), Setup((64, 48), Language.HIP, boundary=CYC2), True),
+    # scalar statics of every kind of dependence on reductions and calls (schemes/monitor.py),
+    # in LDS tiles
+    "monitor_f64": (_monitor, Setup((64, 64), Language.HIP, boundary=CYC2, tile=(32, 8)), True),
     # Open (non-periodic) boundaries: ghost margins, as the reference's shipped examples
     "life_open_i32": (_life_plain, Setup((128, 128), Language.HIP, boundary=OPEN2), True),
     "life_legacy_open_i32": (_life_legacy, Setup((128, 128), Language.HIP, boundary=OPEN2), True),
