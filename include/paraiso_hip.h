@@ -60,9 +60,10 @@ typedef struct pr_fold {
  * the last call leaves behind can be seen, so
  *   - a kernel with a form that makes several calls in one launch (Setup.fused) asks for it:
  *     its launcher returns 1, with the kernel in `use`,
- *   - a kernel none of whose launches reads a scalar it stores leaves its reductions and
- *     scalar stores to the last call of the run, which repeats the scalar stores that count
- *     calls (`pending` of them before its own). */
+ *   - a kernel none of whose launches reads a scalar it stores, and none of whose scalar
+ *     stores reads what an earlier call's reduction left, leaves its reductions and scalar
+ *     stores to the last call of the run, which repeats the scalar stores that count calls
+ *     (`pending` of them before its own). */
 typedef struct pr_run_state {
   int left;                /* calls still to make, this one included */
   int use, times, done;    /* set by a launcher that returns 1: `times` launches of kernel `use`

@@ -841,39 +841,46 @@ class MachineEmitter:
         return not self._stores_inline(sch, la) and (
             bool(la.reduces) or bool(la.tail_scalars) or (la.commit and bool(sch.scalar_stores)))
 
-    def _reads_stored(self, sch, roots) -> bool:
-        """Some value of ``roots`` depends on a scalar static that the kernel stores."""
-        nodes = sch.kernel.nodes
-        own = set(s for s, _ in sch.scalar_stores)
+    def _cone(self, nodes, roots) -> Set[int]:
+        """The values that ``roots`` depend on, themselves among them."""
         seen, stack = set(), list(roots)
         while stack:
             x = stack.pop()
             if x not in seen:
                 seen.add(x)
                 stack.extend(nodes[x].args)
+        return seen
+
+    def _reads_stored(self, sch, roots) -> bool:
+        """Some value of ``roots`` depends on a scalar static that the kernel stores."""
+        nodes = sch.kernel.nodes
+        own = set(s for s, _ in sch.scalar_stores)
         return any(nodes[x].op == "load" and nodes[x].realm is Realm.Scalar
-                   and nodes[x].payload in own for x in seen)
+                   and nodes[x].payload in own for x in self._cone(nodes, roots))
 
     def _defers(self, sch) -> bool:
         """The kernel's finish may be left to the last call of a run (pr_run_state): no launch
-        reads a scalar the kernel stores, and no stored scalar counts something of every call
-        but what it can count from scalars alone (a reduction's result is then only the last
-        call's)."""
+        reads a scalar the kernel stores, and the scalar stores, repeated with the last call's
+        reductions, leave what the calls would have left one by one.  They do where no store
+        reads a static that holds something of an earlier call's reductions: one that a
+        reduction is stored in, or one that is stored from such a static."""
         if len(sch.launches) != 1 or not sch.scalar_stores:
             return False
         nodes = sch.kernel.nodes
         if self._reads_stored(sch, sch.launches[0].targets):
             return False
-        for _, v in sch.scalar_stores:
-            seen, stack = set(), [v]
-            while stack:
-                x = stack.pop()
-                if x not in seen:
-                    seen.add(x)
-                    stack.extend(nodes[x].args)
-            if self._reads_stored(sch, [v]) and any(nodes[x].op == "reduce" for x in seen):
-                return False
-        return True
+        reads, held = {}, set()
+        for s, v in sch.scalar_stores:
+            cone = self._cone(nodes, [v])
+            reads[s] = set(nodes[x].payload for x in cone
+                           if nodes[x].op == "load" and nodes[x].realm is Realm.Scalar)
+            if any(nodes[x].op == "reduce" for x in cone):
+                held.add(s)
+        while True:
+            more = set(s for s in reads if s not in held and reads[s] & held)
+            if not more:
+                return not any(r & held for r in reads.values())
+            held |= more
 
     # ------------------------------------------------------------ register streaming
     def _lane_plans(self, ki, k, la):

@@ -35,3 +35,15 @@ def test_a_finish_reads_only_slots_that_are_written(kernel):
 def test_the_hydro_step_needs_no_finish_between_its_launches():
     launch = body(source("hydro_f64"), "static int launch_Hydro_proceed_l0(")
     assert "if (!c->fold || !c->fold->n) hipLaunchKernelGGL(Hydro_proceed_l0_fin" in launch
+
+
+@pytest.mark.parametrize("kernel", ["watch", "record"])
+def test_a_store_of_an_earlier_reduction_is_not_left_to_the_end(kernel):
+    """``last`` and ``older`` hold reductions of earlier calls, ``high`` of them all: the last
+    call of a run cannot store them from its own reduction alone."""
+    fin = body(source("monitor_f64"), "Monitor_%s_l0_fin(" % kernel)
+    assert "a.repeat" not in fin
+
+
+def test_life_stores_its_scalars_at_the_end_of_a_run():
+    assert "it < a.repeat" in body(source("life_i32"), "Life_proceed_l0_fin(")

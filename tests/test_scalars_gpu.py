@@ -94,3 +94,18 @@ def test_two_launches_that_allocate_nothing(require_gpu, size):
     assert np.array_equal(bufs[parity[0]].cpu().numpy(), model.f)
     got = scal.cpu().numpy()
     assert [got[m.static_index(k)] for k in ("top", "low")] == [model.s["top"], model.s["low"]]
+
+
+@pytest.mark.parametrize("size", SIZES)
+@pytest.mark.parametrize("kernel", ["watch", "record"])
+def test_runs_of_calls(require_gpu, size, kernel):
+    """A run leaves what single calls leave, of this call and of those before it."""
+    print("monitor %s %s" % (kernel, size), flush=True)
+    m, model = variants.machine("monitor_f64", size), Model(field(*size, 5))
+    m.set("f", model.f)
+    m.set("weight", model.s["weight"])
+    for count, graph in ((1, False), (2, False), (5, False), (3, True), (3, True), (1, False)):
+        m.run(kernel, count, graph=graph)
+        for _ in range(count):
+            model.run(kernel)
+        check(m, model)
