@@ -684,7 +684,10 @@ class MachineEmitter:
             h.append("  a.nwg = om_resident_workgroups(a.ntiles, %d);" % self._per_cu(la))
         else:
             h.append("  a.nwg = a.ntiles;")
-        if lane:
+        if lane and block and self.batched:
+            # a batch runs the tile form whatever the grid: `wide` stays the tiles'
+            h += ["  a.ln = 0; a.lv = 0;", "  if (!batch) {"] + self._lane_fill(la, lanes) + ["  }"]
+        elif lane:
             h.extend(self._lane_fill(la, lanes))
         if small:
             h.append("  a.bv = 0;")
