@@ -250,6 +250,9 @@ VARIANTS = {
     # scalar statics of every kind of dependence on reductions and calls (schemes/monitor.py),
     # in LDS tiles
     "monitor_f64": (_monitor, Setup((64, 64), Language.HIP, boundary=CYC2, tile=(32, 8)), True),
+    # the same in batches that stream tiles of ten steps, shared by workgroups of four waves
+    "monitor_f64_batch": (_monitor, Setup((64, 64), Language.HIP, boundary=CYC2, batched=True,
+                                          lane=dict(LANE_HYDRO_BATCH, steps=10)), True),
     # Open (non-periodic) boundaries: ghost margins, as the reference's shipped examples
     "life_open_i32": (_life_plain, Setup((128, 128), Language.HIP, boundary=OPEN2), True),
     "life_legacy_open_i32": (_life_legacy, Setup((128, 128), Language.HIP, boundary=OPEN2), True),

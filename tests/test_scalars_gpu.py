@@ -109,3 +109,24 @@ def test_runs_of_calls(require_gpu, size, kernel):
         for _ in range(count):
             model.run(kernel)
         check(m, model)
+
+
+@pytest.mark.parametrize("count", [1, 40])
+def test_batches_whose_tiles_do_not_divide(require_gpu, count):
+    """Tiles of ten steps over workgroups of four waves, split over the waves (a few tiles) or
+    a wave's each (more than eight a CU)."""
+    sizes = [(300, 251), (61, 9), (62, 10), (63, 11), (5, 7)] * count
+    sizes += [(1900, 1210)] * (count // 20)
+    print("monitor batch of %d" % len(sizes), flush=True)
+    b = variants.batch("monitor_f64_batch", sizes)
+    models = [Model(field(nx, ny, g)) for g, (nx, ny) in enumerate(sizes)]
+    for m, model in zip(b.grids, models):
+        m.set("f", model.f)
+        m.set("weight", model.s["weight"])
+    for kernel in ("watch", "normalize", "damp", "record", "watch", "watch"):
+        b.run(kernel)
+        for model in models:
+            model.run(kernel)
+    b.sync()
+    for m, model in zip(b.grids, models):
+        check(m, model)
