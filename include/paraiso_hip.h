@@ -81,6 +81,7 @@ typedef struct pr_run_state {
   int keep;                /* calls made for another kernel: what this one carries stays as it
                               was (scal3 stands in for the machine's own space) */
   pr_fold prev;            /* partials of the previous call */
+  int plain;               /* made for another kernel: its own fused forms are not asked for */
 } pr_run_state;
 
 /* What a generated launch callback receives (one kernel launch of one OM kernel). */

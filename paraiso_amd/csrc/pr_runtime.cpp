@@ -182,12 +182,13 @@ int launch_kernel_once(pr_machine* m, int k) { return launch_kernel_ov(m, k, nul
 // `count` calls of kernel k, of which only the last one's results can be seen.
 int launch_kernel_run(pr_machine* m, int k, int count) {
   pr_run_state own = {}, other = {};
+  other.plain = 1;
   for (int c = 0; c < count;) {
     own.left = count - c;
     int rc = launch_kernel_ov(m, k, nullptr, nullptr, &own);
     if (rc == 2) {   // another kernel makes the rest of the calls
       other = {};
-      other.keep = 1;
+      other.keep = other.plain = 1;
       rc = PR_OK;
       for (; c < count && rc == PR_OK; ++c) {
         other.left = count - c;

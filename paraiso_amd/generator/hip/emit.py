@@ -742,7 +742,7 @@ class MachineEmitter:
         h.append("static int launch_%s(const pr_launch_ctx* c) {" % fn)
         if L == 0:
             for n_, kb, times, cells in sorted(self.fused.get(ki, ()), reverse=True):
-                h.append("  if (c->run && c->run->left >= %d && (long long)c->n[0] * c->n[1] * c->n[2] "
+                h.append("  if (c->run && !c->run->plain && c->run->left >= %d && (long long)c->n[0] * c->n[1] * c->n[2] "
                          ">= %dLL) {" % (n_, cells))
                 h.append("    c->run->use = %d; c->run->times = %d; c->run->done = %d; return 1; }"
                          % (kb, times, n_))

@@ -115,6 +115,12 @@ def _monitor():
     return monitor_om()
 
 
+def _monitor_fused():
+    """With ``watch_x2`` and ``watch_x4``."""
+    from .transform import unroll
+    return unroll(unroll(_monitor(), "watch", 2), "watch", 4)
+
+
 # Register streaming (generator/hip/lane.py).  Hydro: a wave streams along y; below min_cells
 # the strips are too short for their run-up and the tile form is faster (FP32: 22.6 us a step
 # at 700^2 in tiles, 24.0 streaming; 33.4 and 28.3 at 1021x767; 112 and 91 at 2048^2.  FP64:
@@ -250,9 +256,13 @@ VARIANTS = {
     # scalar statics of every kind of dependence on reductions and calls (schemes/monitor.py),
     # in LDS tiles
     "monitor_f64": (_monitor, Setup((64, 64), Language.HIP, boundary=CYC2, tile=(32, 8)), True),
-    # the same in batches that stream tiles of ten steps, shared by workgroups of four waves
-    "monitor_f64_batch": (_monitor, Setup((64, 64), Language.HIP, boundary=CYC2, batched=True,
-                                          lane=dict(LANE_HYDRO_BATCH, steps=10)), True),
+    # the same in batches that stream tiles of ten steps, shared by workgroups of four waves, and
+    # with kernels that make two and four calls, the four by way of the two
+    "monitor_f64_batch": (_monitor_fused,
+                          Setup((64, 64), Language.HIP, boundary=CYC2, batched=True,
+                                lane=dict(LANE_HYDRO_BATCH, steps=10),
+                                fused=(("watch", "watch_x2", 2, 1, 0),
+                                       ("watch_x2", "watch_x4", 2, 1, 0))), True),
     # Open (non-periodic) boundaries: ghost margins, as the reference's shipped examples
     "life_open_i32": (_life_plain, Setup((128, 128), Language.HIP, boundary=OPEN2), True),
     "life_legacy_open_i32": (_life_legacy, Setup((128, 128), Language.HIP, boundary=OPEN2), True),

@@ -130,3 +130,17 @@ def test_batches_whose_tiles_do_not_divide(require_gpu, count):
     b.sync()
     for m, model in zip(b.grids, models):
         check(m, model)
+
+
+@pytest.mark.parametrize("count", [1, 2, 3, 4, 5, 8, 11])
+def test_fused_kernels_that_have_fused_kernels(require_gpu, count):
+    """``watch`` has a kernel for two calls, and that one another for two of its own."""
+    print("monitor fused run of %d" % count, flush=True)
+    m, model = variants.machine("monitor_f64_batch", (150, 77)), Model(field(150, 77, 6))
+    m.set("f", model.f)
+    m.set("weight", model.s["weight"])
+    for graph in (False, True, True):
+        m.run("watch", count, graph=graph)
+        for _ in range(count):
+            model.run("watch")
+        check(m, model)
