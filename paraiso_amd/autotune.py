@@ -19,6 +19,9 @@ kernels that fuse several steps per launch (halo depth) as candidates of their o
 step; ``alloc-prepare`` / ``alloc-measure`` / ``alloc-select`` flip the Manifest/Delayed
 choice of single values nearest the scheduler's threshold and keep a flip that pays (the
 per-node genome of Tuning/Genetic.hs:138-146, searched locally from the tuned machine).
+
+What is tuned is the tile form: candidates are built without the forms that take its place on
+some grids (register streaming, small tiles), so that each is timed at every size.
 """
 from __future__ import annotations
 
@@ -129,7 +132,7 @@ def _build_candidate(variant: str, c):
     if persist is not None:
         form["persist"] = persist
     try:
-        return c, build_machine(setup.with_(**form), mk(), name, precise=precise)
+        return c, build_machine(setup.tiles_only().with_(**form), mk(), name, precise=precise)
     except (ValueError, subprocess.CalledProcessError) as e:
         print("candidate %s skipped: %s" % (name, str(e).splitlines()[0]), file=sys.stderr)
         return c, None
@@ -269,12 +272,15 @@ def alloc_candidates(variant: str, kernel: str, count: int = 8) -> List[Tuple[st
 
 
 def _flip_name(variant: str, kernel: str, flip) -> str:
-    return "%s__alloc_%s_%s%d" % (variant, kernel, flip[0][0], flip[1])
+    return "%s__alloc_%s" % (variant, kernel) + ("_%s%d" % (flip[0][0], flip[1]) if flip else "")
 
 
 def _flipped_setup(variant: str, kernel: str, flip):
+    """The variant's tile form as tuned (``flip`` None) or with one choice flipped."""
     from . import variants
-    setup = variants.setup_of(variant)
+    setup = variants.setup_of(variant).tiles_only()
+    if flip is None:
+        return setup
     forms = dict(setup.kernel_forms)
     f = dict(forms.get(kernel, {}))
     man, dly = set(f.get("manifest", ())), set(f.get("delayed", ()))
@@ -303,9 +309,10 @@ def _build_flip(variant: str, kernel: str, flip):
 
 
 def prepare_alloc(variant: str, kernel: str, count: int = 8, jobs: int = 4):
-    """Compile one machine per flip of the Manifest/Delayed choice (alloc_candidates)."""
+    """Compile the tile form as tuned (None) and one machine per flip of its Manifest/Delayed
+    choice (alloc_candidates)."""
     from concurrent.futures import ProcessPoolExecutor
-    flips = alloc_candidates(variant, kernel, count)
+    flips = [None] + alloc_candidates(variant, kernel, count)
     with ProcessPoolExecutor(max_workers=max(1, jobs)) as ex:
         futs = [ex.submit(_build_flip, variant, kernel, fl) for fl in flips]
         return [r for r in (f.result() for f in futs) if r[1] is not None]
@@ -313,12 +320,11 @@ def prepare_alloc(variant: str, kernel: str, count: int = 8, jobs: int = 4):
 
 def measure_alloc(variant: str, kernel: str, size, count: int = 8, steps: int = 50,
                   warmup: int = 5, step_kernel: str = None) -> List[Dict]:
-    """Device time per step of the variant as tuned and of each compiled flip."""
-    from . import variants
+    """Device time per step of the variant's tile form as tuned and of each compiled flip."""
     from .generator import GEN_DIR
     from .machine import Machine
-    libs = [(None, variants.library(variant))]
-    for fl in alloc_candidates(variant, kernel, count):
+    libs = []
+    for fl in [None] + alloc_candidates(variant, kernel, count):
         name = _flip_name(variant, kernel, fl)
         so = os.path.join(GEN_DIR, name, "lib%s.so" % name)
         if os.path.exists(so):

@@ -89,6 +89,13 @@ class Setup:
     def with_(self, **kw) -> "Setup":
         return replace(self, **kw)
 
+    def tiles_only(self) -> "Setup":
+        """The same machine without register streaming and small tiles: every grid takes the
+        tile form (what a tuner of tiles times)."""
+        forms = ((k, {x: y for x, y in f.items() if x not in ("lane", "tiny")})
+                 for k, f in self.kernel_forms)
+        return self.with_(lane=None, tiny=(), kernel_forms=tuple((k, f) for k, f in forms if f))
+
     def form_of(self, kernel: str) -> dict:
         """The launch form of one OM kernel: the machine's, with the kernel's overrides."""
         f = {"tile": self.tile, "threads": self.threads, "persist": self.persist,
