@@ -282,9 +282,10 @@ def setup_of(name: str):
                             persist=bool(rec.get("persist", setup.persist)),
                             join=bool(rec.get("join", setup.join)))
     if rec is not None and "kernel_forms" in rec:
-        forms = []
+        # (over the variant's own forms: a recorded tile keeps a kernel's streaming form)
+        forms = dict(setup.kernel_forms)
         for k, f in sorted(rec["kernel_forms"].items()):
-            form = {}
+            form = dict(forms.get(k, {}))
             if "tile" in f:
                 form.update({"tile": tuple(f["tile"]), "threads": int(f["threads"]),
                              "mat_gain": int(f.get("mat_gain", 48)),
@@ -295,8 +296,8 @@ def setup_of(name: str):
             for key in ("manifest", "delayed"):
                 if f.get(key):
                     form[key] = tuple(int(v) for v in f[key])
-            forms.append((k, form))
-        setup = setup.with_(kernel_forms=tuple(forms))
+            forms[k] = form
+        setup = setup.with_(kernel_forms=tuple(sorted(forms.items())))
     return setup
 
 

@@ -41,3 +41,14 @@ def test_flips_and_their_baseline_are_tiles_at_every_size(built):
     forms = [s.form_of(kernel) for s, _ in built.values()]
     assert len(set(str(f) for f in forms)) == 3          # only the flipped choice differs
     assert len(set(f["tile"] for f in forms)) == 1
+
+
+def test_recorded_forms_keep_the_variants_own(monkeypatch):
+    """A recorded tile or flip of one kernel leaves every kernel its streaming form."""
+    rec = {"proceed_x8": {"tile": [32, 32], "threads": 512}, "proceed": {"manifest": [4]}}
+    monkeypatch.setattr(autotune, "tuned", lambda: {"life_i32": {"kernel_forms": rec}})
+    setup, own = variants.setup_of("life_i32"), variants.VARIANTS["life_i32"][1]
+    for k in ("proceed", "proceed_x4", "proceed_x8", "proceed_x16"):
+        assert setup.form_of(k)["lane"] == own.form_of(k)["lane"] is not None
+    assert setup.form_of("proceed_x8")["tile"] == (32, 32)
+    assert setup.form_of("proceed")["manifest"] == (4,)
