@@ -563,13 +563,15 @@ class MachineEmitter:
         if needs_tail:
             f = fin.append
 
+            kept = [n for n in nodes if defer and n.realm is Realm.Scalar and n.op == "load"]
+
             def scalars(ind):
                 for n in nodes:
                     if n.realm is not Realm.Scalar:
                         continue
                     lvl = sch.level[n.id]
                     if lvl == 0:
-                        e = self.scalar_expr(k, n.id)
+                        e = "s%d" % n.payload if n in kept else self.scalar_expr(k, n.id)
                         if chain and n.op == "arith":     # rounded as chain_lines does
                             e = "om_uniform((%s)(%s))" % (n.ctype.c_name, e)
                         f(ind + "const %s u%d = %s;" % (n.ctype.c_name, n.id, e))
@@ -578,6 +580,10 @@ class MachineEmitter:
                             n.ctype.c_name, n.id, n.ctype.c_name, self.slot_off(ki, n.id)))
             if not defer:
                 scalars("  ")
+            # read beside the partials, not behind their sum
+            for n in kept:
+                f("  %s s%d = *(const %s*)(a.scal + %d);" % (n.ctype.c_name, n.payload,
+                                                          n.ctype.c_name, 8 * n.payload))
             for j, r in enumerate(la.reduces):
                 a_ct = nodes[nodes[r].args[0]].ctype
                 at = acc_type(nodes[r].payload, a_ct)
@@ -603,6 +609,10 @@ class MachineEmitter:
                         "if (!a.keep) " if chain and self.carried(s_) else "",
                         nodes[v].ctype.c_name, 8 * s_, v))
             if defer:
+                stored = dict(sch.scalar_stores)
+                for n in kept:
+                    if n.payload in stored:
+                        f("    s%d = u%d;" % (n.payload, stored[n.payload]))
                 f("  }")
             f("  }")
         fin_decls = scratch(self.nt)
