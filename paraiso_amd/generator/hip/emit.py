@@ -353,13 +353,14 @@ class MachineEmitter:
             fields.append("const %s* __restrict__ ld%d;" % (self.statics[s].dyn.ctype.c_name, s))
         for s in stores:
             fields.append("%s* __restrict__ st%d;" % (self.statics[s].dyn.ctype.c_name, s))
-        fields += ["char* __restrict__ scal;", "char* __restrict__ part;", "unsigned* counter;",
-                   "int n0, n1, n2;", "int t0, t1, t2;", "unsigned ntiles;",
-                   "unsigned m0, m1;  /* om_udiv reciprocals of t0 and t1 */",
+        # (every launch passes these by value: with up to 112 bytes the host issues one in 2.7-3.3
+        # us and the stream takes 2.7, with 120 and more 6.7 and 3.4, so nothing is held twice)
+        fields += ["char* __restrict__ scal;", "char* __restrict__ part;",
+                   "int n0, n1, n2;", "int t0, t1, t2;  /* tiles, or strips of streaming waves */",
+                   "unsigned ntiles;", "unsigned m0, m1;  /* om_udiv reciprocals of t0 and t1 */",
                    "int wide;  /* some axis shorter than tile plus reach: om_wrap takes the "
                    "remainder */",
                    "unsigned nwg;   /* reduction partials written (workgroups that reduce) */"]
-        fields.append("int repeat;   /* calls the finish stands for */")
         # the second of two launches folds the first one's partials itself: every workgroup
         # reads them (at most a few KB) where a finish kernel between the two would have cost
         # a launch.  A second launch with a finish of its own reads the folded scalars from
@@ -373,18 +374,21 @@ class MachineEmitter:
         # a kernel whose next call needs this call's reductions folds them there (pr_run_state)
         chain = (len(sch.launches) == 1 and bool(la.targets) and bool(la.reduces)
                  and bool(sch.scalar_stores) and not self._defers(sch))
-        fields.append("char* scal_out;   /* where scalar stores go */")
-        if chain:
-            fields += ["const char* cpart;", "unsigned cstride, cn;   /* the last call's partials */"]
+        # the rest of a run of calls may be another kernel's, which starts from this one's scalars
+        carrier = self.carrier(ki, sch) if folds and L == 0 else None
         inline = self._stores_inline(sch, la)
-        if self.tiny:
-            fields.append("int bv;   /* which of the launch's tiles */")
-        if lane:
-            fields += ["unsigned ln, lx, ly, mx, my;  /* register streaming: waves, strips along "
-                       "x and y, reciprocals */", "int lc;  /* steps a wave streams */",
-                       "int lv;  /* which of the launch's streaming forms */"]
+        needs_tail = self._finishes(sch, la)
+        defer = (needs_tail or inline) and self._defers(sch)
+        if defer:
+            fields.append("int repeat;   /* calls the finish stands for */")
+        if chain or carrier:
+            fields.append("char* scal_out;   /* where scalar stores go */")
         if chain:
-            fields.append("int keep;   /* the finish leaves the carried scalars as they are */")
+            fields += ["const char* cpart;", "unsigned cstride, cn;   /* the last call's partials */",
+                       "int keep;   /* the finish leaves the carried scalars as they are */"]
+        if lane:
+            fields += ["unsigned ln;  /* register streaming: waves, */",
+                       "int lc;  /* and steps of each */"]
         struct = "struct Args_%s {\n  %s\n};\n" % (fn, "\n  ".join(fields))
 
         acc_types = set(acc_type(nodes[r].payload, nodes[nodes[r].args[0]].ctype)
@@ -496,8 +500,7 @@ class MachineEmitter:
             for s_, v in sch.scalar_stores:
                 out.append("    *(%s*)(a.scal + %d) = u%d;" % (nodes[v].ctype.c_name, 8 * s_, v))
             return out + ["  }"] * (2 if defer else 1)
-        needs_tail = self._finishes(sch, la)
-        defer = (needs_tail or inline) and self._defers(sch)
+
         def epilogue(index):
             e = []
             for j, r in enumerate(la.reduces):
@@ -605,9 +608,9 @@ class MachineEmitter:
                 f("    *(%s*)(a.scal + %d) = u%d;" % (n.ctype.c_name, self.slot_off(ki, v), v))
             if la.commit:
                 for s_, v in sch.scalar_stores:
-                    f("    %s*(%s*)(a.scal_out + %d) = u%d;" % (
+                    f("    %s*(%s*)(a.%s + %d) = u%d;" % (
                         "if (!a.keep) " if chain and self.carried(s_) else "",
-                        nodes[v].ctype.c_name, 8 * s_, v))
+                        nodes[v].ctype.c_name, "scal_out" if chain else "scal", 8 * s_, v))
             if defer:
                 stored = dict(sch.scalar_stores)
                 for n in kept:
@@ -651,7 +654,6 @@ class MachineEmitter:
                 ks.append("  const Args_%s a = grids[blockIdx.x];" % fn)
                 ks.append(fcore)
                 ks.append("}")
-        carrier = self.carrier(ki, sch) if folds and L == 0 else None
         if carrier:
             # the carrying kernel's scalars: the machine's and, folded, this launch's reduction
             r = la.reduces[0]
@@ -669,14 +671,17 @@ class MachineEmitter:
 
         # ---- host launcher
         h = []
-        h.append("static void fill_%s(const pr_launch_ctx* c, Args_%s& a, bool batch = false) {" % (fn, fn))
-        h.append("  (void)batch;")
+        # (returns the form: 0 the tiles, -i - 1 the i-th streaming form, i + 1 the i-th small tiles)
+        h.append("static int fill_%s(const pr_launch_ctx* c, Args_%s& a, bool batch = false) {" % (fn, fn))
+        h.append("  int form = 0; (void)batch;")
         for s in loads:
             h.append("  a.ld%d = (const %s*)c->cur[%d];" % (s, self.statics[s].dyn.ctype.c_name, s))
         for s in stores:
             src = "cur" if self.is_scratch(s) else "next"
             h.append("  a.st%d = (%s*)c->%s[%d];" % (s, self.statics[s].dyn.ctype.c_name, src, s))
-        h.append("  a.scal = a.scal_out = c->scal; a.part = c->part; a.counter = c->counter;")
+        h.append("  a.scal = c->scal; a.part = c->part;")
+        if chain or carrier:
+            h.append("  a.scal_out = c->scal;")
         if chain:
             h.append("  a.cpart = nullptr; a.cstride = a.cn = 0; a.keep = 0;")
         h.append("  a.n0 = c->n[0]; a.n1 = c->n[1]; a.n2 = c->n[2];")
@@ -687,7 +692,8 @@ class MachineEmitter:
         else:
             h.append("  a.t0 = c->tiles[0]; a.t1 = c->tiles[1]; a.t2 = c->tiles[2]; a.ntiles = c->ntiles;")
         h.append("  a.m0 = om_udiv_magic((unsigned)a.t0); a.m1 = om_udiv_magic((unsigned)a.t1);")
-        h.append("  a.repeat = 1;")
+        if defer:
+            h.append("  a.repeat = 1;")
         h.append("  a.wide = (%s) ? 1 : 0;" % " || ".join(
             "c->n[%d] < %d" % (ax, self.tile[ax] + reach) for ax in range(self.ndim)))
         if persist:
@@ -696,21 +702,20 @@ class MachineEmitter:
             h.append("  a.nwg = a.ntiles;")
         if lane and block and self.batched:
             # a batch runs the tile form whatever the grid: `wide` stays the tiles'
-            h += ["  a.ln = 0; a.lv = 0;", "  if (!batch) {"] + self._lane_fill(la, lanes) + ["  }"]
+            h += ["  if (!batch) {"] + self._lane_fill(la, lanes) + ["  }"]
         elif lane:
             h.extend(self._lane_fill(la, lanes))
         if small:
-            h.append("  a.bv = 0;")
-            h.append("  if (!batch%s) {" % (" && !a.ln" if lane else ""))
+            h.append("  if (!batch%s) {" % (" && !form" if lane else ""))
             h.append("    const long long all = (long long)a.n0 * a.n1 * a.n2;")
             h.append("    const unsigned space = c->ntiles < PR_MIN_PARTIALS ? PR_MIN_PARTIALS : c->ntiles;")
             for i, (below, _, T_, nt_, reach_) in enumerate(small):
-                h.append("    if (!a.bv && all < %dLL) {" % below)
+                h.append("    if (!form && all < %dLL) {" % below)
                 h.append("      const int t0 = (a.n0 + %d) / %d, t1 = (a.n1 + %d) / %d, t2 = (a.n2 + %d) / %d;"
                          % (T_[0] - 1, T_[0], T_[1] - 1, T_[1], T_[2] - 1, T_[2]))
                 h.append("      const unsigned nt = (unsigned)t0 * (unsigned)t1 * (unsigned)t2;")
                 h.append("      if (nt <= space) {")
-                h.append("        a.bv = %d; a.t0 = t0; a.t1 = t1; a.t2 = t2; a.ntiles = a.nwg = nt;" % (i + 1))
+                h.append("        form = %d; a.t0 = t0; a.t1 = t1; a.t2 = t2; a.ntiles = a.nwg = nt;" % (i + 1))
                 h.append("        a.m0 = om_udiv_magic((unsigned)t0); a.m1 = om_udiv_magic((unsigned)t1);")
                 h.append("        a.wide = (%s) ? 1 : 0;" % " || ".join(
                     "a.n%d < %d" % (ax, T_[ax] + reach_) for ax in range(self.ndim)))
@@ -720,6 +725,7 @@ class MachineEmitter:
         if fold:
             h.append("  a.fpart = c->fold ? c->fold->part : nullptr;")
             h.append("  a.fstride = c->fold ? c->fold->stride : 0u; a.fn = c->fold ? c->fold->n : 0u;")
+        h.append("  return form;")
         h.append("}")
         h.append("static void pack_%s(const pr_launch_ctx* c, void* out) {" % fn)
         # (a batch's waves follow the runtime's table of tiles: a fixed number of steps each)
@@ -756,7 +762,7 @@ class MachineEmitter:
                          ">= %dLL) {" % (n_, cells))
                 h.append("    c->run->use = %d; c->run->times = %d; c->run->done = %d; return 1; }"
                          % (kb, times, n_))
-        h.append("  Args_%s a; fill_%s(c, a);" % (fn, fn))
+        h.append("  Args_%s a; const int form = fill_%s(c, a); (void)form;" % (fn, fn))
         if defer:
             # (a shorter rest of the run goes to this kernel's own fused forms or to itself)
             h.append("  bool finish = true;")
@@ -777,15 +783,15 @@ class MachineEmitter:
                   "  }"]
         if lane:
             wg = self.lane["waves"]
-            h.append("  if (a.ln) {")
+            h.append("  if (form < 0) {")
             h.append("  a.nwg = (a.ln + %du) / %du;" % (wg - 1, wg))
             for i, (_, _, name) in enumerate(lanes):
-                form = name if block else "(a.n0 < (1 << 29) ? %s : %s_far)" % (name, name)
-                h.append("  %sif (a.lv == %d) hipLaunchKernelGGL(%s, dim3(a.nwg), dim3(%d), 0, "
-                         "(hipStream_t)c->stream, a);" % ("else " if i else "", i, form, 64 * wg))
+                kern = name if block else "(a.n0 < (1 << 29) ? %s : %s_far)" % (name, name)
+                h.append("  %sif (form == %d) hipLaunchKernelGGL(%s, dim3(a.nwg), dim3(%d), 0, "
+                         "(hipStream_t)c->stream, a);" % ("else " if i else "", -i - 1, kern, 64 * wg))
             h.append("  }" + (" else" if block else ""))
         for i, (_, name, _, nt_, _) in enumerate(small):
-            h.append("  if (a.bv == %d) hipLaunchKernelGGL(%s, dim3(a.ntiles), dim3(%d), 0, "
+            h.append("  if (form == %d) hipLaunchKernelGGL(%s, dim3(a.ntiles), dim3(%d), 0, "
                      "(hipStream_t)c->stream, a);\n  else" % (i + 1, name, nt_))
         if has_work and block:
             h.append("  hipLaunchKernelGGL(%s, dim3(%s), dim3(%d), 0, (hipStream_t)c->stream, a);"
@@ -1000,12 +1006,14 @@ class MachineEmitter:
         last = self.ndim - 1
         where = ["  const int lane = threadIdx.x & 63;"]
         if self.ndim == 2:
-            where += ["  const unsigned chunk = om_udiv(tile, a.lx, a.mx);",
-                      "  const int X0 = (int)(tile - chunk * a.lx) * %d, S0 = (int)chunk * a.lc;"
+            where += ["  const unsigned chunk = om_udiv(tile, (unsigned)a.t0, a.m0);",
+                      "  const int X0 = (int)(tile - chunk * (unsigned)a.t0) * %d, S0 = (int)chunk * a.lc;"
                       % width]
         else:
-            where += ["  const unsigned q_ = om_udiv(tile, a.lx, a.mx), chunk = om_udiv(q_, a.ly, a.my);",
-                      "  const int X0 = (int)(tile - q_ * a.lx) * %d, Y0 = (int)(q_ - chunk * a.ly) * %d, "
+            where += ["  const unsigned q_ = om_udiv(tile, (unsigned)a.t0, a.m0), "
+                      "chunk = om_udiv(q_, (unsigned)a.t1, a.m1);",
+                      "  const int X0 = (int)(tile - q_ * (unsigned)a.t0) * %d, "
+                      "Y0 = (int)(q_ - chunk * (unsigned)a.t1) * %d, "
                       "S0 = (int)chunk * a.lc;" % (plan.width, plan.rows)]
         core = ["#pragma clang fp contract(off)"] if self.fast_fp32 else []
         core += ["    const int H = a.n%d - S0 < steps ? a.n%d - S0 : steps;" % (last, last)]
@@ -1100,9 +1108,10 @@ class MachineEmitter:
     def _lane_fill(self, la, lanes) -> List[str]:
         """Host side: the form for this grid, its strips and its steps per wave."""
         last = self.ndim - 1
-        h = ["  const long long cells = (long long)a.n0 * a.n1 * a.n2; (void)cells;", "  a.lv = 0;"]
+        h = ["  const long long cells = (long long)a.n0 * a.n1 * a.n2; (void)cells;",
+             "  int pick = 0;"]
         if len(lanes) > 1:
-            h.append("  if (cells < %dLL) a.lv = 1;" % lanes[1][0]["below"])
+            h.append("  if (cells < %dLL) pick = 1;" % lanes[1][0]["below"])
         for i, (f, plan, _) in enumerate(lanes):
             bits = plan if f.get("bits") else None
             plan = bits.lane if bits else plan
@@ -1110,49 +1119,45 @@ class MachineEmitter:
             wg = f["waves"]
             # (grids below the smallest skip the search for the steps per wave: their launches
             # are short and the host issues them)
-            few = "cells < %dLL" % f["min_cells"] if f.get("min_cells") else ""
-            h.append("  if (%s) a.ln = 0;" % few if few else "")
-            h.append("  %sif (a.lv == %d) {" % ("else " if few else "", i))
-            h += ["  a.lx = (unsigned)((a.n0 + %d) / %d); a.ly = %s;" % (
-                     width - 1, width,
-                     "(unsigned)((a.n1 + %d) / %d)" % (plan.rows - 1, plan.rows)
-                     if self.ndim == 3 else "1u"),
-                  "  a.mx = om_udiv_magic(a.lx); a.my = om_udiv_magic(a.ly);"]
+            h.append("  if (pick == %d%s) {" % (
+                i, " && cells >= %dLL" % f["min_cells"] if f.get("min_cells") else ""))
+            h.append("  const unsigned lx = (unsigned)((a.n0 + %d) / %d), ly = %s;" % (
+                width - 1, width, "(unsigned)((a.n1 + %d) / %d)" % (plan.rows - 1, plan.rows)
+                if self.ndim == 3 else "1u"))
             cap = "c->ntiles * %du" % wg if la.reduces else "0x7fffffffu"
-            if bits:
-                h.append("  a.lc = %d;" % bits.height)
-            else:
-                h.append("  a.lc = om_lane_chunk(a.n%d, a.lx * a.ly, %.2f, %g, %s, %d, "
-                         "(unsigned)om_cus() * 4u);"
-                         % (last, plan.runup, f.get("fill", 1.2), cap, f["steps"]))
-            h.append("  a.ln = a.lx * a.ly * (unsigned)((a.n%d + a.lc - 1) / a.lc);" % last)
+            h.append("  const int lc = %s;" % (
+                bits.height if bits else
+                "om_lane_chunk(a.n%d, lx * ly, %.2f, %g, %s, %d, (unsigned)om_cus() * 4u)"
+                % (last, plan.runup, f.get("fill", 1.2), cap, f["steps"])))
+            h.append("  const unsigned ln = lx * ly * (unsigned)((a.n%d + lc - 1) / lc);" % last)
             wide = ["a.n0 < %d" % (64 + 2 * plan.reach),
                     "a.n%d < %d" % (last, 2 * plan.reach + (64 if bits else 0))]
             if self.ndim == 3:
                 wide.append("a.n1 < %d" % (plan.rows + 2 * plan.reach))
-            wide = "(%s) ? 1 : 0" % " || ".join(wide)
-            if f.get("always"):
-                h += ["  a.wide = %s;" % wide, "  }"]
-                continue
             # grids the form is not for take the tile form: a row's bytes must fit the 32-bit
             # lane offsets, a workgroup's partials the space for them
-            not_for = ["a.n0 >= (1 << 29)"]
-            if la.reduces:
-                not_for.append("(a.ln + %du) / %du > c->ntiles" % (wg - 1, wg))
-            if self.march and f.get("ratio"):
-                # a streaming tile form keeps memory busier where its workgroups (one per CU)
-                # fill the chip: `ratio` is its time per cell next to this form's, measured full
-                vol = 1
-                for t in self.tile:
-                    vol *= t
-                h.append("  const unsigned rounds = (a.ntiles + (unsigned)om_cus() - 1u) / (unsigned)om_cus();")
-                not_for.append("(double)rounds * om_cus() * %d.0 * %g < (double)cells"
-                               % (vol, f["ratio"]))
-            h.append("  if (%s) a.ln = 0;" % " || ".join(not_for))
-            h.append("  if (a.ln) a.wide = %s;" % wide)
+            not_for = []
+            if not f.get("always"):
+                not_for.append("a.n0 >= (1 << 29)")
+                if la.reduces:
+                    not_for.append("(ln + %du) / %du > c->ntiles" % (wg - 1, wg))
+                if self.march and f.get("ratio"):
+                    # a streaming tile form keeps memory busier where its workgroups (one per CU)
+                    # fill the chip: `ratio` is its time per cell next to this form's, measured full
+                    vol = 1
+                    for t in self.tile:
+                        vol *= t
+                    h.append("  const unsigned rounds = (a.ntiles + (unsigned)om_cus() - 1u) / "
+                             "(unsigned)om_cus();")
+                    not_for.append("(double)rounds * om_cus() * %d.0 * %g < (double)cells"
+                                   % (vol, f["ratio"]))
+            h.append("  if (!(%s)) {" % " || ".join(not_for) if not_for else "  {")
+            h += ["    form = %d; a.t0 = (int)lx; a.t1 = (int)ly; a.lc = lc; a.ln = ln;" % (-i - 1),
+                  "    a.m0 = om_udiv_magic(lx); a.m1 = om_udiv_magic(ly);",
+                  "    a.wide = (%s) ? 1 : 0;" % " || ".join(wide)]
             if self._own_tiles(plan):
-                h.append("  if (a.ln) a.ntiles = c->ntiles;   // the stride of the partials")
-            h.append("  }")
+                h.append("    a.ntiles = c->ntiles;   // the stride of the partials")
+            h += ["  }", "  }"]
         return h
 
     def _max_reach(self, sch, la) -> int:
