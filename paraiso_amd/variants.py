@@ -150,11 +150,13 @@ LANE_WAVE_F64 = {"rows": 4, "waves": 4, "occupancy": 2, "steps": 4, "fill": 3,
                  "small": {"rows": 3, "occupancy": 3, "below": 2_000_000}}
 
 # Life in bit planes (generator/hip/bits.py): 1024^2, 16 generations 7.1 us a launch (the LDS
-# tiles took 10 us for eight), 4096^2 eight 31 us against 162 (4.4 TB/s).  One generation a
-# launch is a matter of latency below a million cells, where the tiles are as fast.
+# tiles took 10 us for eight), 4096^2 eight 31 us against 162 (4.4 TB/s).  Few generations a
+# launch are a matter of latency on small grids, where the tiles are faster: us a call of one
+# generation in tiles and bits 6.8 and 9.4 at 1024^2, 10.3 and 9.5 at 1200^2, 12.8 and 9.3 at
+# 1448^2; of four 7.6 and 9.6 at 512^2, 10.7 and 9.6 at 724^2; of eight 10.5 and 8.7 at 64^2.
 BITS = {"bits": True, "waves": 4, "occupancy": 4, "steps": 8}
-LIFE_FORMS = (("proceed", {"lane": dict(BITS, min_cells=1_000_000)}),
-              ("proceed_x4", {"lane": BITS}), ("proceed_x8", {"lane": BITS}),
+LIFE_FORMS = (("proceed", {"lane": dict(BITS, min_cells=1_200_000)}),
+              ("proceed_x4", {"lane": dict(BITS, min_cells=400_000)}), ("proceed_x8", {"lane": BITS}),
               ("proceed_x16", {"lane": BITS}))
 
 # Runs of calls take the kernels that make several at once (transform.unroll).
