@@ -1125,10 +1125,14 @@ class MachineEmitter:
                 width - 1, width, "(unsigned)((a.n1 + %d) / %d)" % (plan.rows - 1, plan.rows)
                 if self.ndim == 3 else "1u"))
             cap = "c->ntiles * %du" % wg if la.reduces else "0x7fffffffu"
+            if f.get("always") and la.reduces:
+                # (a single grid's waves take fewer steps than a batch's tile holds)
+                h.append("  const unsigned space = c->ntiles < PR_MIN_PARTIALS ? PR_MIN_PARTIALS : c->ntiles;")
+                cap = "space * %du" % wg
             h.append("  const int lc = %s;" % (
                 bits.height if bits else
                 "om_lane_chunk(a.n%d, lx * ly, %.2f, %g, %s, %d, (unsigned)om_cus() * 4u)"
-                % (last, plan.runup, f.get("fill", 1.2), cap, f["steps"])))
+                % (last, plan.runup, f.get("fill", 1.2), cap, f.get("least", f["steps"]))))
             h.append("  const unsigned ln = lx * ly * (unsigned)((a.n%d + lc - 1) / lc);" % last)
             wide = ["a.n0 < %d" % (64 + 2 * plan.reach),
                     "a.n%d < %d" % (last, 2 * plan.reach + (64 if bits else 0))]
@@ -1155,8 +1159,12 @@ class MachineEmitter:
             h += ["    form = %d; a.t0 = (int)lx; a.t1 = (int)ly; a.lc = lc; a.ln = ln;" % (-i - 1),
                   "    a.m0 = om_udiv_magic(lx); a.m1 = om_udiv_magic(ly);",
                   "    a.wide = (%s) ? 1 : 0;" % " || ".join(wide)]
+            # the stride of the partials
             if self._own_tiles(plan):
-                h.append("    a.ntiles = c->ntiles;   // the stride of the partials")
+                h.append("    a.ntiles = c->ntiles;")
+            elif f.get("always") and la.reduces:
+                h.append("    if (!batch && (ln + %du) / %du > a.ntiles) a.ntiles = (ln + %du) / %du;"
+                         % (wg - 1, wg, wg - 1, wg))
             h += ["  }", "  }"]
         return h
 

@@ -55,18 +55,18 @@ class Setup:
     merge_selects: bool = True
     # register streaming (hip/lane.py): {"rows": y rows per lane (3-D), "waves": waves per
     # workgroup, "occupancy": waves per SIMD the registers are held to, "fill": waves per SIMD
-    # below which a launch gains from more (om_lane_chunk), "steps": least steps per wave,
-    # "unroll", "prefetch": steps the loads are issued ahead, "min_cells": smallest grid that
-    # takes the form, "always": every grid does and no tile form is built, "ratio": see
-    # MachineEmitter._lane_fill, "small": what differs on grids of fewer than "below" cells,
-    # "bits": bit planes instead (hip/bits.py)}
+    # below which a launch gains from more (om_lane_chunk), "steps": least steps per wave (a
+    # batch's tile holds as many), "least": a single grid's, where "always" is set, "min_cells":
+    # smallest grid that takes the form, "always": every grid does and no tile form is built,
+    # "ratio": see MachineEmitter._lane_fill, "small": what differs on grids of fewer than
+    # "below" cells, "bits": bit planes instead (hip/bits.py)}
     lane: Optional[dict] = None
     # smaller tiles for small single grids, smallest first: ({"below": cells, "tile": ...,
     # "threads": ..., "mat_gain": ...}, ...)
     tiny: Tuple[dict, ...] = ()
-    # ((kernel, other kernel, n, launches, cells), ...): `launches` launches of the other make n
-    # calls of the kernel, on grids of at least that many cells, such as those transform.unroll adds: a run of at least n calls on such a
-    # grid uses them, the largest n first
+    # ((kernel, other kernel, n, launches, cells), ...): on grids of at least that many cells,
+    # `launches` launches of the other kernel (such as those transform.unroll adds) make n calls
+    # of the kernel; a run of at least n calls uses them, the largest n first
     fused: Tuple[Tuple[str, str, int, int, int], ...] = ()
     # per OM kernel, a launch form overriding the above: ((kernel name, {"tile": ...,
     # "threads": ..., "persist": ..., "march": ..., "mat_gain": ..., "join": ...}), ...)

@@ -137,7 +137,9 @@ TINY_HYDRO_F64 = ({"below": 30_000, "tile": (16, 8), "threads": 320},
                   {"below": 120_000, "tile": (16, 16), "threads": 512})
 # Batches: a tile is 24 steps of one wave: 256 uneven grids 0.92 ms a step in LDS tiles, 0.58 so
 # (32 steps: 0.59; small batches 18.5 us a step against 17.6).
-LANE_HYDRO_BATCH = {"waves": 4, "occupancy": 2, "steps": 24, "always": True}
+# A grid of its own takes fewer steps a wave: us a step of 24, 4 and 2 at 64x48, 400x300 and 700^2
+# 36 37 39, 12.2 13.7 21.3, 11.0 13.2 21.5 (LDS tiles 11.7 12.6 22.1).
+LANE_HYDRO_BATCH = {"waves": 4, "occupancy": 2, "steps": 24, "least": 2, "always": True}
 # LinearWave 3-D: a lane holds rows of y, fewer on small grids (64^3: 11.6 us a step with 8, 8.9
 # with 4; 128^3 15.3 and 13.9; 300^3 128 and 128, two steps 123 and 141).  FP32 keeps its
 # streaming tiles where they fill the chip: at 512^3 they move 4.7 TB/s and the waves' unaligned
