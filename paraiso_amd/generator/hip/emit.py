@@ -1145,6 +1145,10 @@ class MachineEmitter:
                 not_for.append("a.n0 >= (1 << 29)")
                 if la.reduces:
                     not_for.append("(ln + %du) / %du > c->ntiles" % (wg - 1, wg))
+                if f.get("rows_below"):
+                    # long rows, and large grids of rows that fill a wave, are the tiles'
+                    not_for.append("a.n0 >= %d || (a.n0 >= 64 && cells >= %dLL)"
+                                   % (f["rows_below"], f["cells_below"]))
                 if self.march and f.get("ratio"):
                     # a streaming tile form keeps memory busier where its workgroups (one per CU)
                     # fill the chip: `ratio` is its time per cell next to this form's, measured full

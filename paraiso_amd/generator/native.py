@@ -58,8 +58,8 @@ class Setup:
     # below which a launch gains from more (om_lane_chunk), "steps": least steps per wave (a
     # batch's tile holds as many), "least": a single grid's, where "always" is set, "min_cells":
     # smallest grid that takes the form, "always": every grid does and no tile form is built,
-    # "ratio": see MachineEmitter._lane_fill, "small": what differs on grids of fewer than
-    # "below" cells, "bits": bit planes instead (hip/bits.py)}
+    # "ratio", "rows_below" with "cells_below": see MachineEmitter._lane_fill, "small": what
+    # differs on grids of fewer than "below" cells, "bits": bit planes instead (hip/bits.py)}
     lane: Optional[dict] = None
     # smaller tiles for small single grids, smallest first: ({"below": cells, "tile": ...,
     # "threads": ..., "mat_gain": ...}, ...)

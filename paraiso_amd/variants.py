@@ -156,6 +156,12 @@ LANE_WAVE_F32 = {"rows": 8, "waves": 4, "occupancy": 3, "steps": 4, "fill": 3, "
                  "small": {"rows": 4, "occupancy": 4, "fill": 4, "below": 2_500_000}}
 LANE_WAVE_F64 = {"rows": 4, "waves": 4, "occupancy": 2, "steps": 4, "fill": 3,
                  "small": {"rows": 3, "occupancy": 3, "below": 2_000_000}}
+# One adjoint step reads and writes two fields and computes little: tiles, whose rows are aligned,
+# are as fast or faster on long rows and large grids.  us a call in strips and in tiles: 512^3
+# 1060 and 960, 200^3 50.7 and 44.0, 500x8x500 17.2 and 12.9, 201x150x97 16.2 and 19.9, 150^3 23.4
+# and 28.6, 8x500x500 39 and 79.
+WAVE_F64_FORMS = (("proceed_adjoint", {"lane": dict(LANE_WAVE_F64, rows_below=256,
+                                                    cells_below=4_000_000)}),)
 
 # Life in bit planes (generator/hip/bits.py): 1024^2, 16 generations 7.1 us a launch (the LDS
 # tiles took 10 us for eight), 4096^2 eight 31 us against 162 (4.4 TB/s).  Few generations a
@@ -235,7 +241,8 @@ VARIANTS = {
                                                     lane=LANE_WAVE_F32, fused=FUSED_WAVE_F32,
                                                     kernel_forms=WAVE_FORMS), False),
     "wave3d_f64": (_wave_adj(3, CType.Double), Setup((64, 64, 64), Language.HIP, boundary=CYC3,
-                                                     lane=LANE_WAVE_F64, fused=FUSED_WAVE), True),
+                                                     lane=LANE_WAVE_F64, fused=FUSED_WAVE,
+                                                     kernel_forms=WAVE_F64_FORMS), True),
     # streaming along the last axis (rings of planes in LDS), checked bit for bit
     "life_i32_march": (_life, Setup((64, 64), Language.HIP, boundary=CYC2, tile=(64, 32),
                                     march=4, fused=FUSED_LIFE), True),
