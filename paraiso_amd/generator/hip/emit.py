@@ -648,10 +648,11 @@ class MachineEmitter:
             ks.append(fcore)
             ks.append("}")
             if self.batched:
-                ks.append("extern \"C\" __global__ void __launch_bounds__(%d) %s_fin_batched(const Args_%s* __restrict__ grids) {"
+                ks.append("extern \"C\" __global__ void __launch_bounds__(%d) %s_fin_batched(const Args_%s* __restrict__ grids, unsigned parts) {"
                           % (self.nt, fn, fn))
                 ks.extend(fin_decls)
-                ks.append("  const Args_%s a = grids[blockIdx.x];" % fn)
+                ks.append("  Args_%s a = grids[blockIdx.x];" % fn)
+                ks.append("  a.nwg *= parts; a.ntiles *= parts;   // partials a tile")
                 ks.append(fcore)
                 ks.append("}")
         if carrier:
@@ -742,16 +743,22 @@ class MachineEmitter:
                 h.append("  hipLaunchKernelGGL(%s_batched, dim3(bc->total_tiles), dim3(%d), 0, (hipStream_t)bc->stream, "
                          "(const Args_%s*)bc->args, bc->tile_grid, bc->tile_base, bc->total_tiles);" % (fn, self.nt, fn))
             else:
-                # below two waves per SIMD a tile is split over a workgroup
-                h.append("  const int split = bc->total_tiles < 8u * (unsigned)om_cus();")
-                h.append("  hipLaunchKernelGGL((bc->far_rows ? %s_far_batched : %s_batched), "
-                         "dim3(split ? bc->total_tiles : "
-                         "(bc->total_tiles + %du) / %du), dim3(%d), 0, (hipStream_t)bc->stream, "
-                         "(const Args_%s*)bc->args, bc->tile_grid, bc->tile_base, bc->total_tiles, split);"
-                         % (fn, fn, wg - 1, wg, 64 * wg, fn))
+                # below two waves per SIMD a tile is split over a workgroup, below half a tile per
+                # CU over two (16 grids of 64^2, 96 tiles of 24 steps: 15.2 and 11.7 us a step)
+                h += ["  const unsigned total = bc->total_tiles, cus = (unsigned)om_cus();",
+                      "  const int parts = total <= cus / 2u ? 2 : total < 8u * cus ? 1 : 0;",
+                      "  const Args_%s* const args = (const Args_%s*)bc->args;" % (fn, fn),
+                      "  if (parts)",
+                      "    hipLaunchKernelGGL((bc->far_rows ? %s_far_split : %s_split), dim3(total * parts), "
+                      "dim3(%d), 0, (hipStream_t)bc->stream, args, bc->tile_grid, bc->tile_base, total, parts);"
+                      % (fn, fn, 64 * wg),
+                      "  else",
+                      "    hipLaunchKernelGGL((bc->far_rows ? %s_far_batched : %s_batched), "
+                      "dim3((total + %du) / %du), dim3(%d), 0, (hipStream_t)bc->stream, args, "
+                      "bc->tile_grid, bc->tile_base, total);" % (fn, fn, wg - 1, wg, 64 * wg)]
         if needs_tail and self.batched:
             h.append("  hipLaunchKernelGGL(%s_fin_batched, dim3(bc->n_grids), dim3(%d), 0, (hipStream_t)bc->stream, "
-                     "(const Args_%s*)bc->args);" % (fn, self.nt, fn))
+                     "(const Args_%s*)bc->args, %s);" % (fn, self.nt, fn, "1" if block else "parts > 1 ? 2 : 1"))
         if self.batched:
             h.append("  return hipPeekAtLastError() == hipSuccess ? 0 : -1;")
         h.append("}")
@@ -1049,40 +1056,43 @@ class MachineEmitter:
         out += ["  if (wv < a.ln) {"] + core + ["  }"] + epilogue("b_", False)
         out += own_scalars("b_ == 0 && threadIdx.x == 0")
         out += chain_stores("b_ == 0 && threadIdx.x == 0") + ["}"]
-        if self.batched and f.get("always"):
-            # a tile of the batch is a wave's; `split`: a workgroup's, each wave taking its
-            # share of the steps, where the batch has too few tiles to fill the chip
-            # (steps that the waves do not divide: the last waves take what is left, or nothing.
-            # As one expression for both, 256 uneven grids took 23.7 ms for 40 steps, 23.3 so)
-            part, even = -(-f["steps"] // wg), f["steps"] % wg == 0
-            share = ("a.lc / %d" % wg if even else
-                     "(a.lc - (int)w_ * %d < %d ? a.lc - (int)w_ * %d : %d)" % ((part,) * 4))
-            out.append("extern \"C\" __global__ void %s %s_batched(const Args_%s* __restrict__ grids, "
+        for split in (False, True) if self.batched and f.get("always") else ():
+            # a tile of the batch is a wave's; `split`: of `parts` workgroups, each wave taking its
+            # share of the steps (the last ones what is left, or nothing)
+            out.append("extern \"C\" __global__ void %s %s_%s(const Args_%s* __restrict__ grids, "
                        "const int* __restrict__ tile_grid, const unsigned* __restrict__ tile_base, "
-                       "unsigned total, int split) {" % (bounds, fn, fn))
+                       "unsigned total%s) {" % (bounds, fn, "split" if split else "batched", fn,
+                                                ", int parts" if split else ""))
             out += scr + wave[:-1]
-            out += ["  const unsigned w_ = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);",
-                    "  const unsigned wv = split ? b_ : b_ * %du + w_;" % wg,
-                    "  if (wv >= total) return;", "  const int g = tile_grid[wv];",
-                    "  const Args_%s a = grids[g];" % fn,
-                    "  const unsigned tile = wv - tile_base[g];",
-                    "  const int steps = split ? %s : a.lc;" % share]
-            out += [ln.replace("S0 = (int)chunk * a.lc;",
-                               "S0 = (int)chunk * a.lc + (split ? (int)w_ * %s : 0);"
-                               % ("steps" if even else "%d" % part))
-                    for ln in where] + uniform_lines(64 * wg, False) + pre
-            out += ["  if (%sS0 < a.n%d) {" % ("" if even else "steps > 0 && ", last)]
-            out += core + ["  }"]
-            if la.reduces:
-                out += (["  if (split) {"] + epilogue("tile", False) + ["  } else {"]
-                        + epilogue("tile", True) + ["  }"])
-            out += own_scalars("tile == 0 && lane == 0 && (!split || w_ == 0)") + ["}"]
+            out.append("  unsigned w_ = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);")
+            if split:
+                out += ["  const unsigned wv = parts > 1 ? b_ >> 1 : b_, sub = b_ - wv * parts;",
+                        "  w_ += sub * %du;" % wg]
+            else:
+                out += ["  const unsigned wv = b_ * %du + w_;" % wg, "  if (wv >= total) return;"]
+            out += ["  const int g = tile_grid[wv];", "  Args_%s a = grids[g];" % fn,
+                    "  const unsigned tile = wv - tile_base[g];"]
+            at = where
+            if split:
+                out += ["  a.ntiles *= parts;", "  const int all = %d * parts;" % wg,
+                        "  const int share = (a.lc + all - 1) / all, first = (int)w_ * share;",
+                        "  const int steps = a.lc - first < share ? a.lc - first : share;"]
+                at = [ln.replace("S0 = (int)chunk * a.lc;", "S0 = (int)chunk * a.lc + first;")
+                      for ln in where]
+            else:
+                out.append("  const int steps = a.lc;")
+            out += at + uniform_lines(64 * wg, False) + pre
+            out += ["  if (%sS0 < a.n%d) {" % ("steps > 0 && " if split else "", last)] + core + ["  }"]
+            out += epilogue("tile * parts + sub", False) if split else epilogue("tile", True)
+            out += own_scalars("tile == 0 && lane == 0 && w_ == 0" if split else
+                               "tile == 0 && lane == 0") + ["}"]
         if f.get("always"):
             # no tile form takes the rows whose byte offsets pass 32 bits: the same kernels with
             # 64-bit lane offsets do
             out += [re.sub(r"\bom_(at|put)\(", r"om_far_\1(", ln)
                     .replace(" %s(Args_" % name, " %s_far(Args_" % name)
-                    .replace(" %s_batched(" % fn, " %s_far_batched(" % fn) for ln in out]
+                    .replace(" %s_batched(" % fn, " %s_far_batched(" % fn)
+                    .replace(" %s_split(" % fn, " %s_far_split(" % fn) for ln in out]
         return out
 
     def _bit_square(self, bits, la, em, stores, reduces, stream) -> List[str]:

@@ -144,3 +144,22 @@ def test_fused_kernels_that_have_fused_kernels(require_gpu, count):
         for _ in range(count):
             model.run("watch")
         check(m, model)
+
+
+def test_batches_of_few_tiles(require_gpu):
+    """A tile of ten steps over the eight waves of two workgroups: two each, some none."""
+    sizes = [(61, 9), (130, 47), (62, 25), (7, 3)]
+    print("monitor batch of %s" % (sizes,), flush=True)
+    b = variants.batch("monitor_f64_batch", sizes)
+    models = [Model(field(nx, ny, g)) for g, (nx, ny) in enumerate(sizes)]
+    for m, model in zip(b.grids, models):
+        m.set("f", model.f)
+        m.set("weight", model.s["weight"])
+    for kernel in ("watch", "normalize", "damp", "record", "watch", "watch"):
+        b.run(kernel, 2, graph=kernel == "watch")
+        for model in models:
+            model.run(kernel)
+            model.run(kernel)
+    b.sync()
+    for m, model in zip(b.grids, models):
+        check(m, model)
