@@ -924,8 +924,7 @@ class MachineEmitter:
                     if "small" not in f:
                         break
                     f.update(f["small"])
-                p = plan_lane(k, la.targets, f.get("rows", 1), f.get("prefetch", 1),
-                              fast=self.fast_fp32)
+                p = plan_lane(k, la.targets, f.get("rows", 1), fast=self.fast_fp32)
                 if p is not None and f.get("bits"):
                     nodes = k.nodes
                     p = plan_bits(k, p, [v for _, v in la.stores],
@@ -1008,7 +1007,7 @@ class MachineEmitter:
                 return "__builtin_fmaxf(%s, %s)" % (args[0], args[1])
             return device_arith(op, args, cast_to, v.types, v.ctype, self.fast_fp32, v.consts,
                                 self._comp)
-        em = LaneEmitter(plan, k, lambda s: "a.ld%d" % self.sidx(ki, s), arith, stores, reduces,
+        em = LaneEmitter(plan, lambda s: "a.ld%d" % self.sidx(ki, s), arith, stores, reduces,
                          fused_products(plan, product))
         last = self.ndim - 1
         where = ["  const int lane = threadIdx.x & 63;"]
@@ -1024,7 +1023,7 @@ class MachineEmitter:
                       "S0 = (int)chunk * a.lc;" % (plan.width, plan.rows)]
         core = ["#pragma clang fp contract(off)"] if self.fast_fp32 else []
         core += ["    const int H = a.n%d - S0 < steps ? a.n%d - S0 : steps;" % (last, last)]
-        core += em.body(f.get("unroll", 1), width, peel=not bits)
+        core += em.body(width, peel=not bits)
         if bits:
             core = self._bit_square(bits, la, em, stores, reduces, core)
         wg = f["waves"]

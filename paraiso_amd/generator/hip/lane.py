@@ -365,10 +365,10 @@ class LaneEmitter:
     operation; ``stores`` and ``reduces`` list (C pointer, C type, target) and (accumulator,
     operator, C type, initial value, target)."""
 
-    def __init__(self, plan: LanePlan, k: LKernel, load_ptr, arith, stores, reduces, fused=None):
+    def __init__(self, plan: LanePlan, load_ptr, arith, stores, reduces, fused=None):
         """``fused``: as ``fused_products`` gives it; ``arith`` then gets, in the place of that
         argument, the pair of names it multiplies."""
-        self.p, self.k = plan, k
+        self.p = plan
         self.fused = fused or {}
         self.inside = set(self._arg(u, i) for u, i in self.fused.items())
         self.by_id = {v.id: v for v in plan.values}
@@ -493,7 +493,7 @@ class LaneEmitter:
                         w("%s = %s;" % (self.name(v, r, d), self.name(v, r, d - 1)))
         return out
 
-    def body(self, unroll: int, width: int, peel: bool = True) -> List[str]:
+    def body(self, width: int, peel: bool = True) -> List[str]:
         """The steps of a wave: the run-up, each step with only the values that something reads
         later, then the loop.  Without ``peel`` the loop runs the run-up too (less code)."""
         out = ["    " + ln for ln in self.setup(width)]
@@ -502,7 +502,7 @@ class LaneEmitter:
             out.append("    {  // run-up, step %d" % s)
             out += ["      " + ln for ln in self.step("%d" % s, s)]
             out.append("    }")
-        out.append("#pragma unroll %d" % max(1, unroll))
+        out.append("#pragma unroll 1")
         out.append("    for (int s = %d; s < H; ++s) {" % first)
         out += ["      " + ln for ln in self.step("s", None, "" if peel else "s >= 0")]
         out.append("    }")
