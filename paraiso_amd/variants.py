@@ -243,6 +243,10 @@ VARIANTS = {
     "wave3d_f64": (_wave_adj(3, CType.Double), Setup((64, 64, 64), Language.HIP, boundary=CYC3,
                                                      lane=LANE_WAVE_F64, fused=FUSED_WAVE,
                                                      kernel_forms=WAVE_F64_FORMS), True),
+    # the FP32 machine's streaming forms, correctly rounded: checked bit for bit
+    "wave3d_f32_precise": (_wave_adj(3, CType.Float, 3), Setup((64, 64, 64), Language.HIP,
+                                                            boundary=CYC3, lane=LANE_WAVE_F32,
+                                                            kernel_forms=WAVE_FORMS), True),
     # streaming along the last axis (rings of planes in LDS), checked bit for bit
     "life_i32_march": (_life, Setup((64, 64), Language.HIP, boundary=CYC2, tile=(64, 32),
                                     march=4, fused=FUSED_LIFE), True),
