@@ -110,6 +110,11 @@ def _optable(real):
     return mk
 
 
+def _rewrites():
+    from .schemes.rewrites import rewrites_om
+    return rewrites_om()
+
+
 def _monitor():
     from .schemes.monitor import monitor_om
     return monitor_om()
@@ -276,6 +281,12 @@ VARIANTS = {
                          False),
     "optable_f64": (_optable(CType.Double), Setup((64, 48), Language.HIP, boundary=CYC2), True),
     "optable_i32": (_optable(CType.Int), Setup((64, 48), Language.HIP, boundary=CYC2), True),
+    # what fast FP32 streaming evaluates in another form (schemes/rewrites.py), streaming and in
+    # tiles
+    "rewrites_f32": (_rewrites, Setup((64, 64), Language.HIP, boundary=CYC2,
+                                      lane=LANE_HYDRO_BATCH), False),
+    "rewrites_f32_tiles": (_rewrites, Setup((64, 64), Language.HIP, boundary=CYC2, tile=(32, 8)),
+                           False),
     # scalar statics of every kind of dependence on reductions and calls (schemes/monitor.py),
     # in LDS tiles
     "monitor_f64": (_monitor, Setup((64, 64), Language.HIP, boundary=CYC2, tile=(32, 8)), True),
