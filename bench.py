@@ -344,43 +344,40 @@ def bench_adjoint(n=512, steps=200, every=20, dt=1e-4, variant="hydro_adj2_f32_f
 
 
 def bench_life(n=1024, gens=1000, seed=1):
-    """Conway Life 1024^2 int32 periodic, Bernoulli(0.5) cells, 1000 generations: one graph of
-    ``proceed_x4`` or ``proceed_x8`` launches (four or eight generations per launch, bit-identical
-    to as many ``proceed``); both are timed and the faster is reported."""
-    runs = [_bench_life(n, gens, seed, k) for k in (4, 8)]
-    best = dict(min(runs, key=lambda r: r["ms_per_step"]))
-    best["alternatives"] = {"proceed_x%d" % r["generations_per_launch"]: r["value"] for r in runs}
-    return best
-
-
-def _bench_life(n, gens, seed, per_launch):
+    """Conway Life 1024^2 int32 periodic, Bernoulli(0.5) cells, 1000 generations of ``proceed`` in
+    one graph, which makes them sixteen a launch (``proceed_x16``), the rest by eight, four and
+    one; then each of those kernels timed a launch at a time."""
     import torch
     from paraiso_amd import inputs, variants
     m = variants.machine("life_i32", (n, n))
     m.run("init")
     m.set("cell", inputs.life_init((n, n), seed))
-    kern = "proceed_x%d" % per_launch
-    m.run(kern, gens // per_launch, graph=True)      # builds and warms the graph
+    m.run("proceed", gens, graph=True)               # builds and warms the graph
     m.run("init")
     m.set("cell", inputs.life_init((n, n), seed))
     m.sync()
     torch.cuda.synchronize()
     t0 = time.perf_counter()
-    m.run(kern, gens // per_launch, graph=True)
+    m.run("proceed", gens, graph=True)
     m.sync()
     t1 = time.perf_counter()
     pop, gen = int(m.get("population")), int(m.get("generation"))
-    ms = m.run_timed(kern, 25)
+    single = {k: sum(m.run_timed(k, 25)) / 25 for k in ("proceed", "proceed_x4", "proceed_x8",
+                                                        "proceed_x16")}
+    m.close()
     cells = n * n
-    launch_s = sum(ms) / 25 * 1e-3
+    launches, left = 0, gens
+    for k in (16, 8, 4, 1):
+        launches, left = launches + left // k, left % k
     return {"workload": "life-%dx%d-int32-%d-generations" % (n, n, gens), "generations": gens,
             "value": cells * gens / (t1 - t0) / 1e9, "unit": "Gcell-updates/s",
-            "ms_per_step": (t1 - t0) / gens * 1e3,
-            "launch_ms_per_launch": [x / 25 for x in ms], "generations_per_launch": per_launch,
+            "ms_per_step": (t1 - t0) / gens * 1e3, "launches": launches,
+            "generations_per_launch": 16, "run_ms_per_launch": (t1 - t0) / launches * 1e3,
+            "single_launch_ms": single,
             "algorithmic_bytes_per_cell": 8,
             # a launch of k generations reads and writes each cell once: 8 B per cell moved
             "hbm_bytes_per_launch": cells * 8,
-            "achieved_GBps": cells * 8 / launch_s / 1e9,
+            "achieved_GBps": cells * 8 * launches / (t1 - t0) / 1e9,
             "population": pop, "generation": gen}
 
 

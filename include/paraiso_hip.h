@@ -182,7 +182,11 @@ int pr_run_graph(pr_machine* m, int k, int count);
  * reference: measurement support). */
 int pr_run_timed(pr_machine* m, int k, int count, double* launch_ms);
 
-/* ---- statics (replaces `T& name()` / `T& name(i0,i1,...)`, PlanTrans.hs:117-157) */
+/* ---- statics (replaces `T& name()` / `T& name(i0,i1,...)`, PlanTrans.hs:117-157)
+ * pr_static_devptr gives the buffer an array static is in now.  It holds the static until the
+ * next call that stores it (pr_run, pr_run_graph, a batch's run, the adjoint drivers): ask
+ * again after each.  Which of its two buffers a run of n calls leaves it in does
+ * not follow from n, as several calls may be one launch. */
 int pr_static_devptr(pr_machine* m, int s, void** dev_ptr);
 int pr_static_write(pr_machine* m, int s, const void* src, size_t bytes, int src_on_device);
 int pr_static_read(pr_machine* m, int s, void* dst, size_t bytes, int dst_on_device);
@@ -262,7 +266,7 @@ int pr_adjoint_backward_seq(pr_machine* m, const int* fwd, int n_fwd, int tape_a
  *   stream   hipStream_t the work is issued on (NULL: the default stream);
  *   err      optional buffer for a message on failure.
  * The scalar slots, reduction partials and scratch arrays the kernels need live in one
- * fixed device array of PR_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends;
+ * fixed device array of PR_NOALLOC_SCRATCH_BYTES (65 MiB) per GPU, held until the process ends;
  * a kernel and grid that need more are rejected with PR_E_INVALID before any work is
  * issued.  Calls on one GPU share that array: calls that overlap on one GPU (other
  * streams, other host threads) race and must be serialised by the caller. */

@@ -15,8 +15,9 @@ same lazy synchronisation:
 * a kernel call first writes back every mirror marked newer, then marks the
   statics the kernel writes as newer on the device;
 * ``set_name(...)`` writes the device directly, ``name_devptr()`` hands out the
-  device buffer (after writing back the mirror), and ``save``/``load`` write
-  and read whole-machine state files.
+  device buffer (after writing back the mirror; it holds the static until the
+  next kernel call that stores it), and ``save``/``load`` write and read
+  whole-machine state files.
 
 The class loads the machine library with ``dlopen`` and drives it through
 ``include/paraiso_hip.h``; it is host code only.

@@ -1,9 +1,9 @@
 """Python host binding of a generated HIP machine (through ``include/paraiso_hip.h``).
 
 ``Machine`` mirrors the generated C++ class: ``run("proceed", n)`` calls an
-OM kernel ``n`` times, ``get``/``set`` read and write statics, ``devptr``
-returns the device buffer of a static (for zero-copy torch views), and
-``tensor`` wraps a static as a torch tensor on ``cuda:0`` without copying.
+OM kernel ``n`` times, ``get``/``set`` read and write statics, and ``devptr``
+returns the device buffer of a static (for zero-copy torch views), which holds
+it until the next run of a kernel that stores it.
 
 There is no CPU fallback: constructing a ``Machine`` without the built
 libraries or without a GPU raises.

@@ -198,8 +198,9 @@ VARIANTS = {
     "hydro_f32": (_hydro(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2, batched=True,
                                              lane=LANE_HYDRO_F32, tiny=TINY_HYDRO_F32,
                                              kernel_forms=PRIME_HYDRO_F32), False),
-    # the headline machine's launch form (tile, work-items, resident tile loop), correctly
-    # rounded: checked bit for bit against the oracle
+    # the FP32 step in 64x32 LDS tiles with the resident tile loop, correctly rounded: checked
+    # bit for bit against the oracle (the headline machine streams; hydro_f64_lane is its
+    # streaming form's bit-for-bit check)
     "hydro_f32_precise": (_hydro(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2,
                                                      tile=(64, 32), threads=1024, persist=True),
                           True),
@@ -218,7 +219,8 @@ VARIANTS = {
     "hydro_adj_f32_fast": (_hydro_adj(CType.Float), Setup((64, 64), Language.HIP, boundary=CYC2,
                                                           tile=(32, 8), merge_selects=False),
                            False),
-    # the fixed-dt step in FP32 (fast arithmetic) at the headline's launch form
+    # the fixed-dt step in FP32 (fast arithmetic): streaming like the headline on large grids, in
+    # 64x32 tiles with the resident tile loop on small ones
     "hydro_fixed_f32": (_hydro(CType.Float, dt_mode="fixed"),
                         Setup((64, 64), Language.HIP, boundary=CYC2, tile=(64, 32), threads=1024,
                               persist=True, lane=LANE_HYDRO_F32), False),
