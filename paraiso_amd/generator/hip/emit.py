@@ -1073,15 +1073,19 @@ class MachineEmitter:
                     "  const unsigned tile = wv - tile_base[g];"]
             at = where
             if split:
-                out += ["  a.ntiles *= parts;", "  const int all = %d * parts;" % wg,
-                        "  const int share = (a.lc + all - 1) / all, first = (int)w_ * share;",
-                        "  const int steps = a.lc - first < share ? a.lc - first : share;"]
+                even = f["steps"] % (2 * wg) == 0
+                out += ["  a.ntiles *= parts;",
+                        "  const int share = parts > 1 ? %d : %d, first = (int)w_ * share;"
+                        % (-(-f["steps"] // (2 * wg)), -(-f["steps"] // wg)),
+                        "  const int steps = %s;" % ("share" if even else
+                                                     "a.lc - first < share ? a.lc - first : share")]
                 at = [ln.replace("S0 = (int)chunk * a.lc;", "S0 = (int)chunk * a.lc + first;")
                       for ln in where]
             else:
                 out.append("  const int steps = a.lc;")
             out += at + uniform_lines(64 * wg, False) + pre
-            out += ["  if (%sS0 < a.n%d) {" % ("steps > 0 && " if split else "", last)] + core + ["  }"]
+            out += ["  if (%sS0 < a.n%d) {" % ("steps > 0 && " if split and not even else "", last)]
+            out += core + ["  }"]
             out += epilogue("tile * parts + sub", False) if split else epilogue("tile", True)
             out += own_scalars("tile == 0 && lane == 0 && w_ == 0" if split else
                                "tile == 0 && lane == 0") + ["}"]
